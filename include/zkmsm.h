@@ -359,14 +359,15 @@ void zkmsm_gen_scalars(uint64_t seed, uint64_t n, int32_t dist, uint8_t* out);
  * a, b, out: n x 32 B Montgomery field elements. */
 ZkMetalStatus zkmsm_test_fp(ZkMetalMSMEngine engine, int32_t op, const uint8_t* a,
                             const uint8_t* b, uint8_t* out, uint32_t n);
-/* op 0: p + q, 1: 2p, 2: p + affine(q.X, q.Y); XYZZ points of 128 B. */
+/* op 0: p + q, 1: 2p, 2: p + affine(q.X, q.Y); XYZZ points of 128 B.
+ * op 9: p + q, 10: 2p by lane teams; 11, 12: the same on Grumpkin. */
 ZkMetalStatus zkmsm_test_xyzz(ZkMetalMSMEngine engine, int32_t op, const uint8_t* p,
                               const uint8_t* q, uint8_t* out, uint32_t n);
 /* BN254 G2 primitives on 256-byte XYZZ points (X, Y, ZZ, ZZZ c0 parts, then
  * the c1 parts; Fp Montgomery form).  op 0: p + q, 1: 2p, 2: p + affine
  * (q.X, q.Y) (all zero = identity), 3: the bucket-loop addition p + (q.X, q.Y)
  * (p the identity = a run start); field ops on X, result in X, the rest zero:
- * 4: p.X * q.X, 5: p.X^2, 6: 1 / p.X. */
+ * 4: p.X * q.X, 5: p.X^2, 6: 1 / p.X; 7: p + q, 8: 2p by lane teams. */
 ZkMetalStatus zkmsm_test_g2(ZkMetalMSMEngine engine, int32_t op, const uint8_t* p,
                             const uint8_t* q, uint8_t* out, uint32_t n);
 /* GLV split of n scalars: out n x 48 B = k1 (16 B), k2 (16 B), neg1, neg2 (u32). */

@@ -18,7 +18,7 @@ LIB = os.path.join(HERE, "libzkmetal_amd.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("ZKMSM_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["kernels.hip", "engine.hip", "server.cpp", "capi.cpp"]
+SOURCES = ["kernels.hip", "reduce.hip", "engine.hip", "server.cpp", "capi.cpp"]
 COMMON = [
     "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
     "-I", os.path.join(HERE, "..", "include"),

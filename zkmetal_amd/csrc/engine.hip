@@ -105,10 +105,10 @@ static void plan_reset(Plan& pl) {
     pl.segs.clear();
     pl.seg_lane0.clear();
     pl.seg_grp0.clear();
-    pl.seg_rcw0.clear();
+    pl.seg_rcb0.clear();
     pl.tile_seg.clear();
     pl.chunk_seg.clear();
-    pl.scalars = pl.entries = pl.buckets = pl.lanes = pl.groups = pl.rc_waves = 0;
+    pl.scalars = pl.entries = pl.buckets = pl.lanes = pl.groups = pl.rc_blocks = 0;
     pl.tiles = pl.chunks = pl.T = pl.dtiles = 0;
     pl.nparts = 1;
     pl.curve = CurveId::Bn254;
@@ -145,6 +145,14 @@ bool shifted_pays(uint64_t n, uint32_t c, uint32_t c_s) {
 // measured on MI355X, one shifted MSM takes 0.42 / 0.74 / 1.81 / 6.23 ms
 // against 0.61 / 0.65 / 1.71 / 6.05 ms plain at 2^16 / 2^18 / 2^20 / 2^22.
 constexpr uint64_t kShiftSingleMax = 1u << 17;
+
+// Row and column sums by lanes from this many additions on (two per bucket),
+// by lane teams below: 2^16 of them make a wave of one-lane chains for every
+// SIMD, but a lane's chain is 7 us per addition against a team's 2.6.  Whole
+// calls on MI355X: 2^16 points (295,000 additions) 492 us by lanes, 509 by
+// teams; 64 MSMs (4.2 million) 15.4 ms against 15.6; 4097 points (13,000)
+// 342 against 327 us, 256 points (4,100) 267 against 245.
+constexpr uint64_t kReduceLanesMin = 3u << 16;
 
 // ceil(log2 x), at most 32
 static uint32_t size_class(uint64_t x) {
@@ -277,15 +285,18 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
         pt.chunk_hi = pl.segs[pt.seg_hi - 1].chunk0 + pl.segs[pt.seg_hi - 1].nchunks;
     }
     pl.T = pl.parts[0].T;
-    // bucket reduction: per buckets per lane before the shuffle tree; 8 keeps
-    // the tree shallow for small calls, larger batches (throughput-bound) use
-    // up to 32 so that fewer additions go to tree levels
+    // bucket reduction: buckets per lane or team before the tree.  Two
+    // additions per bucket on one wave per SIMD (1024 waves) is the least
+    // chain that fills the chip; a shorter one only adds tree levels (down to
+    // 8, which the tables lower to 4 for small calls)
+    pl.reduce_lanes = 2 * pl.buckets >= kReduceLanesMin;
     pl.G = 8;
-    while (pl.G < 32 && (pl.buckets >> 17) >= 2 * pl.G) pl.G *= 2;
+    const uint64_t round = 1024ull * 64 / (pl.reduce_lanes ? 1 : team_lanes(cv));
+    while (pl.G < 64 && 2 * pl.buckets / round > pl.G) pl.G *= 2;
     if (sched && sched->per[size_class(pl.entries)]) pl.G = sched->per[size_class(pl.entries)];
     pl.seg_lane0.resize(nseg + 1);
     pl.seg_grp0.resize(nseg + 1);
-    pl.seg_rcw0.resize(nseg + 1);
+    pl.seg_rcb0.resize(nseg + 1);
     uint32_t part = 0;
     for (uint32_t s = 0; s < nseg; s++) {
         SegDesc& sg = pl.segs[s];
@@ -293,31 +304,30 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
         PlanPart& pt = pl.parts[part];
         if (s == pt.seg_lo) {
             pt.lane_lo = pl.lanes;
-            pt.rcw_lo = pl.rc_waves;
         }
         sg.lane0 = pl.lanes;
         sg.grp0 = pl.groups;
         pl.seg_lane0[s] = pl.lanes;
         pl.seg_grp0[s] = pl.groups;
-        pl.seg_rcw0[s] = pl.rc_waves;
+        pl.seg_rcb0[s] = pl.rc_blocks;
         pl.lanes += (sg.len + pt.T - 1) / pt.T;
         // bucket reduction: 2^h rows of 2^g buckets and 2^g columns of 2^h,
-        // max(1, len/8) lanes per row / column, rows and columns wave-aligned
+        // rows and columns block-aligned (k_br_rowcol)
         const uint32_t cb = 31 - __builtin_clz(sg.nbk), g = cb / 2, h = cb - g;
-        const uint64_t per = pl.G;
-        const uint64_t pr = (1u << g) >= per ? (1u << g) / per : 1, pc = (1u << h) >= per ? (1u << h) / per : 1;
-        pl.rc_waves += (((uint64_t)1 << h) * pr + 63) / 64 + (((uint64_t)1 << g) * pc + 63) / 64;
+        const uint32_t cap = 256 / team_lanes(cv), bt = pl.reduce_lanes ? 256 : cap;
+        for (uint64_t teams : {((uint64_t)1 << h) * reduce_teams(1u << g, pl.G, cap),
+                               ((uint64_t)1 << g) * reduce_teams(1u << h, pl.G, cap)})
+            pl.rc_blocks += (teams + bt - 1) / bt;
         pl.groups += (1u << h) + (1u << g);
         for (uint32_t t = 0; t < sg.ntiles; t++) pl.tile_seg.push_back(s);
         for (uint32_t t = 0; t < sg.nchunks; t++) pl.chunk_seg.push_back(s);
         if (s + 1 == pt.seg_hi) {
             pt.lane_hi = pl.lanes;
-            pt.rcw_hi = pl.rc_waves;
         }
     }
     pl.seg_lane0[nseg] = pl.lanes;
     pl.seg_grp0[nseg] = pl.groups;
-    pl.seg_rcw0[nseg] = pl.rc_waves;
+    pl.seg_rcb0[nseg] = pl.rc_blocks;
     return kOk;
 }
 
@@ -383,7 +393,7 @@ int32_t Engine::create(Engine** out) {
 
 void Engine::account_buffers() {
     for (DevBuf* b : {&desc_, &digits_, &keysA_, &valsA_, &keysB_, &valsB_, &hist_, &part_, &segvalid_,
-                      &buckets_, &recAk_, &recAp_, &recBk_, &rc_, &winsum_, &err_, &wins_, &res_,
+                      &buckets_, &recAk_, &recAp_, &lists_, &rc_, &winsum_, &err_, &wins_, &res_,
                       &pts_in_, &ptable_, &scalars_, &srs_, &gtab_, &gtab_gk_, &gtab_g2_, &tmp_})
         b->acct = &ws_;
 }
@@ -409,7 +419,7 @@ Engine::~Engine() {
 
 // pack the plan's descriptor arrays into one blob (16-byte aligned sections)
 struct DescLayout {
-    size_t msms, msm_scalar0, msm_dtile0, segs, seg_lane0, seg_grp0, seg_rcw0, tile_seg, chunk_seg, part_T,
+    size_t msms, msm_scalar0, msm_dtile0, segs, seg_lane0, seg_grp0, seg_rcb0, tile_seg, chunk_seg, part_T,
         total;
 };
 
@@ -427,7 +437,7 @@ static DescLayout layout_for(const Plan& pl) {
     L.segs = take(pl.segs.size() * sizeof(SegDesc));
     L.seg_lane0 = take(pl.seg_lane0.size() * 8);
     L.seg_grp0 = take(pl.seg_grp0.size() * 8);
-    L.seg_rcw0 = take(pl.seg_rcw0.size() * 8);
+    L.seg_rcb0 = take(pl.seg_rcb0.size() * 8);
     L.tile_seg = take(pl.tile_seg.size() * 4);
     L.chunk_seg = take(pl.chunk_seg.size() * 4);
     L.part_T = take(kMaxParts * 4);  // entries per lane of each part (k_lane_plan)
@@ -435,7 +445,10 @@ static DescLayout layout_for(const Plan& pl) {
     return L;
 }
 
-static constexpr uint32_t kRunLimit = 8;
+// Device tail: the host normalises the copied sums of up to this many MSMs
+// (0.15 us each and one inversion of 7 us per 64); above, a device lane per
+// MSM does (150 us whatever their number, its inversion's chain).
+static constexpr uint32_t kHostNormMsms = 1024;
 
 // Host tail of a call: per MSM, result = sum_w 2^(c w) (U_w + sum_{t < c-1}
 // 2^t Q_{w,t}) by one Horner over the bit positions b = c w + t (Q_{w,t} =
@@ -460,16 +473,29 @@ struct HostG1 {
     static bool is_id(const Pt& p) { return H::is_id(p); }
     static Pt xdbl(const Pt& p) { return H::xdbl(p); }
     static Pt xadd(const Pt& a, const Pt& b) { return H::xadd(a, b); }
-    static void finish(const std::vector<Pt>& res, uint8_t* out) {
-        std::vector<zkh::Fp> xs, ys;
-        H::batch_to_affine(res, xs, ys);
+    // 64 at a time on the stack: the no-allocation path ends here too
+    static void finish(const Pt* res, size_t n, uint8_t* out) {
         const zkh::Fp one = H::one(), zero = zkh::zero();
-        for (size_t j = 0; j < res.size(); j++) {
-            uint8_t* o = out + j * kOut;
-            const bool id = H::is_id(res[j]);
-            memcpy(o, (id ? one : xs[j]).v, 32);
-            memcpy(o + 32, (id ? one : ys[j]).v, 32);
-            memcpy(o + 64, (id ? zero : one).v, 32);
+        for (size_t j0 = 0; j0 < n; j0 += 64) {
+            const size_t m = std::min<size_t>(64, n - j0);
+            zkh::Fp xs[64], ys[64], pre[129];
+            H::batch_to_affine(res + j0, m, xs, ys, pre);
+            for (size_t j = 0; j < m; j++) {
+                uint8_t* o = out + (j0 + j) * kOut;
+                const bool id = H::is_id(res[j0 + j]);
+                memcpy(o, (id ? one : xs[j]).v, 32);
+                memcpy(o + 32, (id ? one : ys[j]).v, 32);
+                memcpy(o + 64, (id ? zero : one).v, 32);
+            }
+        }
+    }
+    // the same for sums as copied back (kIn bytes each)
+    static void finish_sums(const uint8_t* hw, size_t n, uint8_t* out) {
+        Pt res[64];
+        for (size_t j0 = 0; j0 < n; j0 += 64) {
+            const size_t m = std::min<size_t>(64, n - j0);
+            for (size_t j = 0; j < m; j++) res[j] = load(hw + (j0 + j) * kIn);
+            finish(res, m, out + j0 * kOut);
         }
     }
 };
@@ -492,9 +518,9 @@ struct HostG2View {
     static bool is_id(const Pt& p) { return G::is_id(p); }
     static Pt xdbl(const Pt& p) { return G::xdbl(p); }
     static Pt xadd(const Pt& a, const Pt& b) { return G::xadd(a, b); }
-    static void finish(const std::vector<Pt>& res, uint8_t* out) {
+    static void finish(const Pt* res, size_t n, uint8_t* out) {
         const zkh::Fp2 one = G::one2(), zero = G::zero2();
-        for (size_t j = 0; j < res.size(); j++) {
+        for (size_t j = 0; j < n; j++) {
             uint8_t* o = out + j * kOut;
             zkh::Fp2 x, y, z = one;
             if (G::is_id(res[j])) {
@@ -550,7 +576,7 @@ static void host_tail(const Plan& pl, const uint8_t* hw, uint8_t* out) {
     } else {
         tail(0, nmsm);
     }
-    HC::finish(res, out);
+    HC::finish(res.data(), res.size(), out);
 }
 
 WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
@@ -568,18 +594,20 @@ WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
     z.buckets = pl.buckets * ptb;
     z.rec_keys = rec_cap * 4;
     z.rec_pts = rec_cap * ptb;
+    z.lists = merge_lists_bytes(rec_cap, pl.curve);
     z.rc = pl.groups * ptb;
     // bit-plane points: host form for the host tail, stored form for the device's
     z.bits = nseg * 16 * (dev_tail ? ptb : hpb);
-    z.err = 16;  // the decomposition flag, the merge's long and mid run counters
+    z.err = 32;  // the decomposition flag, the merge's list counters
     z.wins = dev_tail ? nseg * ptb : 0;
-    z.res = dev_tail ? nmsm * result_bytes(pl.curve) : 0;
-    // copied back: the results (device tail) or the bit planes, then err, then
+    // device tail: the sums, normalised on the host, or (many) the results
+    z.res = dev_tail ? nmsm * (nmsm <= kHostNormMsms ? hpb : result_bytes(pl.curve)) : 0;
+    // copied back: those (device tail) or the bit planes, then err, then
     // the per-segment valid-entry counts
     z.back = dev_tail ? z.res : z.bits;
     z.host = z.back + z.err + nseg * 4;
     const uint64_t parts[] = {z.desc, z.digits, z.keys, z.vals, z.keys, z.vals, z.hist, z.part,
-                              z.segvalid, z.buckets, z.rec_keys, z.rec_pts, z.rec_keys, z.rc, z.bits,
+                              z.segvalid, z.buckets, z.rec_keys, z.rec_pts, z.lists, z.rc, z.bits,
                               z.err, z.wins, z.res};
     for (uint64_t b : parts) z.device += (b + 255) & ~uint64_t(255);
     return z;
@@ -604,7 +632,7 @@ int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, 
     ZK_ALLOC(buckets_, z.buckets);
     ZK_ALLOC(recAk_, z.rec_keys);
     ZK_ALLOC(recAp_, z.rec_pts);
-    ZK_ALLOC(recBk_, z.rec_keys);
+    ZK_ALLOC(lists_, z.lists);
     ZK_ALLOC(rc_, z.rc);
     ZK_ALLOC(winsum_, z.bits);
     if (dev_tail) {
@@ -626,7 +654,7 @@ int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, 
     ws.buckets = buckets_.p;
     ws.recAk = recAk_.p;
     ws.recAp = recAp_.p;
-    ws.recBk = recBk_.p;
+    ws.lists = lists_.p;
     ws.rc = rc_.p;
     ws.bits = winsum_.p;
     ws.err = err_.p;
@@ -653,7 +681,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     memcpy(hb + L.segs, pl.segs.data(), pl.segs.size() * sizeof(SegDesc));
     memcpy(hb + L.seg_lane0, pl.seg_lane0.data(), pl.seg_lane0.size() * 8);
     memcpy(hb + L.seg_grp0, pl.seg_grp0.data(), pl.seg_grp0.size() * 8);
-    memcpy(hb + L.seg_rcw0, pl.seg_rcw0.data(), pl.seg_rcw0.size() * 8);
+    memcpy(hb + L.seg_rcb0, pl.seg_rcb0.data(), pl.seg_rcb0.size() * 8);
     memcpy(hb + L.tile_seg, pl.tile_seg.data(), pl.tile_seg.size() * 4);
     memcpy(hb + L.chunk_seg, pl.chunk_seg.data(), pl.chunk_seg.size() * 4);
     for (uint32_t p = 0; p < kMaxParts; p++)
@@ -668,17 +696,14 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     uint64_t* d_seg_lane0 = (uint64_t*)(db + L.seg_lane0);
     uint32_t* d_part_T = (uint32_t*)(db + L.part_T);
     const uint64_t* d_seg_grp0 = (const uint64_t*)(db + L.seg_grp0);
-    const uint64_t* d_seg_rcw0 = (const uint64_t*)(db + L.seg_rcw0);
+    const uint64_t* d_seg_rcb0 = (const uint64_t*)(db + L.seg_rcb0);
     const uint32_t* d_tile_seg = (const uint32_t*)(db + L.tile_seg);
     const uint32_t* d_chunk_seg = (const uint32_t*)(db + L.chunk_seg);
     uint32_t* d_err = (uint32_t*)ws.err;
     hipStream_t st = stream_;
     const uint32_t P = pl.nparts;
-    // the merge lists (long and mid runs): a listed run has more than
-    // kRunLimit records, so each list holds at most nrec / (kRunLimit + 1)
-    // runs; both sit in recBk (2 * lanes + 2 words)
     const uint64_t nrec = 2 * pl.parts[P - 1].lane_hi;
-    const uint32_t list_cap = (uint32_t)std::min<uint64_t>(nrec / (kRunLimit + 1) + 1, 1u << 29);
+    const bool norm = nmsm > kHostNormMsms;  // device tail: normalise there too
     uint8_t* hw = ws.hw;
     // The device part of the call.  Stream A (the engine stream): descriptors,
     // decomposition, then the accumulation of each part, one merge of every
@@ -737,26 +762,24 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         // their first lane, longer runs (heavy buckets) by lane groups.  One
         // merge after the last part instead of one after each keeps the
         // accumulations back to back.
-        launch_merge_runs(pl.curve, (const uint32_t*)ws.recAk, (const uint8_t*)ws.recAp, nrec, kRunLimit,
-                          ws.buckets, d_err + 1, (uint32_t*)ws.recBk, list_cap, st);
+        launch_merge_runs(pl.curve, (const uint32_t*)ws.recAk, ws.recAp, nrec, ws.buckets, d_err + 1, ws.lists, st);
         ZK_TRY(rec(ev_m1_[0], st));
         // the bucket reduction of all parts at once, after the last merge: as
         // a kernel beside the next part's accumulation it finds no free slots
         // (its waves need as many registers as the accumulation's) and
         // measured slower
         ZK_TRY(rec(ev_r0_[0], st));
-        launch_bucket_reduce(pl.curve, d_segs, d_seg_rcw0, d_seg_grp0, nseg, 0, nseg, 0, pl.rc_waves, pl.G,
+        launch_bucket_reduce(pl.curve, d_segs, d_seg_rcb0, d_seg_grp0, nseg, pl.rc_blocks, pl.G, pl.reduce_lanes,
                              ws.buckets, ws.rc, ws.bits, !dev_tail, st);
         ZK_TRY(rec(ev_r1_[0], st));
         if (dev_tail) {
-            launch_tail(pl.curve, d_segs, d_msms, nseg, nmsm, ws.bits, ws.wins, ws.res, st);
+            launch_tail(pl.curve, d_segs, d_msms, nseg, nmsm, ws.bits, ws.wins, ws.res, norm, st);
             ZK_TRY(rec(ev_tail_, st));
         }
         ZK_TRY(rec(ev_[kStCopyOut], st));
         ZK_TRY(hipMemcpyAsync(hw, dev_tail ? ws.res : ws.bits, back_bytes, hipMemcpyDeviceToHost, st));
-        // err[0]: decomposition error flag; err[1], err[2]: long / mid run
-        // counts of the merge (above list_cap: listed runs were dropped)
-        ZK_TRY(hipMemcpyAsync(hw + back_bytes, ws.err, 4 * 3, hipMemcpyDeviceToHost, st));
+        // err[0]: decomposition error flag; err[1..4]: the merge's list counts
+        ZK_TRY(hipMemcpyAsync(hw + back_bytes, ws.err, 4 * 5, hipMemcpyDeviceToHost, st));
         ZK_TRY(hipMemcpyAsync(hw + back_bytes + z.err, ws.segvalid, (uint64_t)nseg * 4,
                               hipMemcpyDeviceToHost, st));
         return kOk;
@@ -777,19 +800,19 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             key.push_back(m.c);
             key.push_back(m.table0);
         }
-        for (uint64_t v : {pl.scalars, pl.entries, pl.buckets, pl.lanes, pl.groups, pl.rc_waves,
+        for (uint64_t v : {pl.scalars, pl.entries, pl.buckets, pl.lanes, pl.groups, pl.rc_blocks,
                            (uint64_t)pl.tiles, (uint64_t)pl.chunks, (uint64_t)pl.T, (uint64_t)pl.dtiles,
                            (uint64_t)pl.G, (uint64_t)nseg})
             key.push_back(v);
         key.push_back(table_n);  // places the table's identity bitmap
         for (uint32_t p = 0; p < P; p++) {
             const PlanPart& pt = pl.parts[p];
-            for (uint64_t v : {(uint64_t)pt.seg_hi, (uint64_t)pt.T, pt.lane_hi, pt.rcw_hi}) key.push_back(v);
+            for (uint64_t v : {(uint64_t)pt.seg_hi, (uint64_t)pt.T, pt.lane_hi}) key.push_back(v);
         }
         key.push_back(dev_tail ? 1 : 0);
         for (const void* p : std::initializer_list<const void*>{
                  d_scalars, d_table, ws.desc, ws.hdesc, ws.digits, ws.keysA, ws.valsA, ws.keysB, ws.valsB,
-                 ws.hist, ws.part, ws.segvalid, ws.buckets, ws.recAk, ws.recAp, ws.recBk, ws.rc, ws.bits,
+                 ws.hist, ws.part, ws.segvalid, ws.buckets, ws.recAk, ws.recAp, ws.lists, ws.rc, ws.bits,
                  ws.err, ws.hw, ws.wins, ws.res})
             key.push_back((uint64_t)(uintptr_t)p);
         graph = graph_mode == kGraphOn || key == last_key_ || (graph_exec_ && key == graph_key_);
@@ -830,10 +853,11 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     }
     ZK_TRY(hipStreamSynchronize(st));
     ZK_TRY(hipGetLastError());
-    uint32_t err[3];
-    memcpy(err, hw + back_bytes, 4 * 3);
+    uint32_t err[5];
+    memcpy(err, hw + back_bytes, 4 * 5);
     if (err[0]) return kGpuError;
-    if (err[1] > list_cap || err[2] > list_cap) return kGpuError;
+    const MergeCaps cap = merge_caps(nrec);
+    if (err[1] > cap.mid || err[2] > cap.spans || err[3] > cap.parts || err[4] > cap.runs) return kGpuError;
 
     // stage times: each stage's kernels summed over the parts (they overlap
     // across streams; a graph replay has only the device total)
@@ -858,14 +882,16 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     (void)hipEventElapsedTime(&timing_.device_ms, ev_[0], ev_[kNumStages]);
 
     // host tail: Horner over windows, then affine normalisation; the device
-    // tail left the normalised results
+    // tail left the sums (the host normalises them) or the results
     auto t_tail0 = std::chrono::steady_clock::now();
-    if (dev_tail) memcpy(out96, hw, back_bytes);
+    if (dev_tail && norm) memcpy(out96, hw, back_bytes);
+    else if (dev_tail && pl.curve == CurveId::Grumpkin) HostG1<zkh::HR>::finish_sums(hw, nmsm, out96);
+    else if (dev_tail) HostG1<zkh::HP>::finish_sums(hw, nmsm, out96);
     else if (pl.curve == CurveId::Grumpkin) host_tail<HostG1<zkh::HR>>(pl, hw, out96);
     else if (pl.curve == CurveId::Bn254G2) host_tail<HostG2View>(pl, hw, out96);
     else host_tail<HostG1<zkh::HP>>(pl, hw, out96);
     auto t_end = std::chrono::steady_clock::now();
-    timing_.host_tail_ms = dev_tail ? 0.f : std::chrono::duration<float, std::milli>(t_end - t_tail0).count();
+    timing_.host_tail_ms = std::chrono::duration<float, std::milli>(t_end - t_tail0).count();
     timing_.wall_ms = std::chrono::duration<float, std::milli>(t_end - t_wall0).count();
     timing_.nmsm = nmsm;
     timing_.window_bits_first = nmsm ? pl.msms[0].c : 0;
@@ -1537,7 +1563,7 @@ int32_t Engine::noalloc_setup() {
     na_plan_.segs.reserve(kNoAllocMaxSegs);
     na_plan_.seg_lane0.reserve(kNoAllocMaxSegs + 1);
     na_plan_.seg_grp0.reserve(kNoAllocMaxSegs + 1);
-    na_plan_.seg_rcw0.reserve(kNoAllocMaxSegs + 1);
+    na_plan_.seg_rcb0.reserve(kNoAllocMaxSegs + 1);
     na_plan_.tile_seg.reserve(4 * kNoAllocMaxSegs);
     na_plan_.chunk_seg.reserve(2 * kNoAllocMaxSegs);
     na_host_.reserve(kNoAllocHostBytes);
@@ -1612,7 +1638,7 @@ int32_t Engine::msm_resident_noalloc(const void* d_scalars, const uint32_t* coun
     ws.buckets = take(z.buckets);
     ws.recAk = take(z.rec_keys);
     ws.recAp = take(z.rec_pts);
-    ws.recBk = take(z.rec_keys);
+    ws.lists = take(z.lists);
     ws.rc = take(z.rc);
     ws.bits = take(z.bits);
     ws.err = take(z.err);
@@ -1700,14 +1726,16 @@ int32_t Engine::test_xyzz(int op, const uint8_t* p, const uint8_t* q, uint8_t* o
     ZK_ALLOC(dout, (uint64_t)n * 128);
     ZK_TRY(hipMemcpy(dp.p, p, (uint64_t)n * 128, hipMemcpyHostToDevice));
     ZK_TRY(hipMemcpy(dq.p, q, (uint64_t)n * 128, hipMemcpyHostToDevice));
-    launch_test_xyzz(op, dp.p, dq.p, dout.p, n, stream_);
+    if (op >= 9)
+        launch_test_team(op >= 11 ? CurveId::Grumpkin : CurveId::Bn254, op % 2 == 0, dp.p, dq.p, dout.p, n, stream_);
+    else launch_test_xyzz(op, dp.p, dq.p, dout.p, n, stream_);
     ZK_TRY(hipStreamSynchronize(stream_));
     ZK_TRY(hipMemcpy(out, dout.p, (uint64_t)n * 128, hipMemcpyDeviceToHost));
     return kOk;
 }
 
 int32_t Engine::test_g2(int op, const uint8_t* p, const uint8_t* q, uint8_t* out, uint32_t n) {
-    if (!p || !q || !out || n == 0 || op < 0 || op > 6) return kInvalidInput;
+    if (!p || !q || !out || n == 0 || op < 0 || op > 8) return kInvalidInput;
     DevBuf dp, dq, dout;
     const uint64_t bytes = (uint64_t)n * 256;
     ZK_ALLOC(dp, bytes);
@@ -1715,7 +1743,8 @@ int32_t Engine::test_g2(int op, const uint8_t* p, const uint8_t* q, uint8_t* out
     ZK_ALLOC(dout, bytes);
     ZK_TRY(hipMemcpy(dp.p, p, bytes, hipMemcpyHostToDevice));
     ZK_TRY(hipMemcpy(dq.p, q, bytes, hipMemcpyHostToDevice));
-    launch_test_g2(op, dp.p, dq.p, dout.p, n, stream_);
+    if (op >= 7) launch_test_team(CurveId::Bn254G2, op == 8, dp.p, dq.p, dout.p, n, stream_);
+    else launch_test_g2(op, dp.p, dq.p, dout.p, n, stream_);
     ZK_TRY(hipStreamSynchronize(stream_));
     ZK_TRY(hipMemcpy(out, dout.p, bytes, hipMemcpyDeviceToHost));
     return kOk;

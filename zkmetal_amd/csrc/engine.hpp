@@ -79,7 +79,7 @@ constexpr uint32_t kMaxParts = 8;
 struct PlanPart {
     uint32_t seg_lo, seg_hi, tile_lo, tile_hi, chunk_lo, chunk_hi;
     uint32_t T;  // entries per accumulation lane in this part
-    uint64_t lane_lo, lane_hi, rcw_lo, rcw_hi, entries;
+    uint64_t lane_lo, lane_hi, entries;
 };
 
 struct Plan {
@@ -91,15 +91,16 @@ struct Plan {
     std::vector<SegDesc> segs;
     std::vector<uint64_t> seg_lane0;  // nseg + 1
     std::vector<uint64_t> seg_grp0;   // nseg + 1: first row/column sum of the segment
-    std::vector<uint64_t> seg_rcw0;   // nseg + 1: first row/column wave of the segment
+    std::vector<uint64_t> seg_rcb0;   // nseg + 1: first row/column block of the segment
     std::vector<uint32_t> tile_seg;
     std::vector<uint32_t> chunk_seg;
-    uint64_t scalars = 0, entries = 0, buckets = 0, lanes = 0, groups = 0, rc_waves = 0;
+    uint64_t scalars = 0, entries = 0, buckets = 0, lanes = 0, groups = 0, rc_blocks = 0;
     uint32_t tiles = 0, chunks = 0, T = 0, dtiles = 0;  // T: the first part's
     uint32_t nparts = 1;
     PlanPart parts[kMaxParts];
     CurveId curve = CurveId::Bn254;
-    uint32_t G = 8;  // buckets per bucket-reduction lane (a power of 2, 8..32)
+    uint32_t G = 8;  // buckets per bucket-reduction lane or team (a power of 2)
+    bool reduce_lanes = false;  // rows and columns summed by lanes, else by teams
 };
 
 // Device buffers of one call (and the host staging it copies through).
@@ -107,7 +108,7 @@ struct Workspace {
     uint8_t* desc = nullptr;  // packed descriptor tables
     void *digits = nullptr, *keysA = nullptr, *valsA = nullptr, *keysB = nullptr, *valsB = nullptr;
     void *hist = nullptr, *part = nullptr, *segvalid = nullptr, *buckets = nullptr;
-    void *recAk = nullptr, *recAp = nullptr, *recBk = nullptr, *rc = nullptr, *bits = nullptr;
+    void *recAk = nullptr, *recAp = nullptr, *lists = nullptr, *rc = nullptr, *bits = nullptr;
     void *err = nullptr, *wins = nullptr, *res = nullptr;
     uint8_t* hdesc = nullptr;  // host: descriptors before upload
     uint8_t* hw = nullptr;     // host: copy-back area
@@ -116,7 +117,7 @@ struct Workspace {
 // bytes of each buffer of a planned call; device = all device buffers, each
 // rounded up to 256 bytes; host = the copy-back area
 struct WsSizes {
-    uint64_t desc, digits, keys, vals, hist, part, segvalid, buckets, rec_keys, rec_pts, rc, bits, err,
+    uint64_t desc, digits, keys, vals, hist, part, segvalid, buckets, rec_keys, rec_pts, lists, rc, bits, err,
         wins, res, back, host, device;
 };
 WsSizes ws_sizes(const Plan& pl, bool dev_tail);
@@ -126,8 +127,8 @@ uint32_t default_window_bits(uint64_t n, CurveId cv = CurveId::Bn254);
 
 // Launch schedule by size class ceil(log2 entries) of a call (its sorted
 // entries before the zero digits are dropped): parts[k] the pipeline parts
-// (1..kMaxParts), per[k] the buckets each bucket-reduction lane sums before
-// the shuffle tree (4..64, a power of two); 0 keeps the built-in rule.
+// (1..kMaxParts), per[k] the buckets each bucket-reduction team sums before
+// the tree (4..64, a power of two); 0 keeps the built-in rule.
 struct Schedule {
     uint8_t parts[33];
     uint8_t per[33];
@@ -368,7 +369,7 @@ class Engine {
     Timing timing_{};
 
     DevBuf desc_, digits_, keysA_, valsA_, keysB_, valsB_, hist_, part_, segvalid_, buckets_;
-    DevBuf recAk_, recAp_, recBk_, rc_, winsum_, err_;  // recBk_: long-run list
+    DevBuf recAk_, recAp_, lists_, rc_, winsum_, err_;  // lists_: the merge's run lists
     DevBuf wins_, res_;  // device tail: window sums, results
     DevBuf pts_in_, ptable_, scalars_, srs_, gtab_, gtab_gk_, gtab_g2_, tmp_;
     HostBuf hdesc_, hwin_;

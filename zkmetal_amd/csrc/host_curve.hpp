@@ -196,10 +196,14 @@ struct HostArith {
     // Batch normalisation: every point needs 1/ZZ and 1/ZZZ; one inversion.
     static void batch_to_affine(const std::vector<Xyzz>& pts, std::vector<Fp>& xs,
                                 std::vector<Fp>& ys) {
-        size_t n = pts.size();
-        xs.assign(n, zero());
-        ys.assign(n, zero());
-        std::vector<Fp> pre(2 * n + 1);
+        xs.assign(pts.size(), zero());
+        ys.assign(pts.size(), zero());
+        std::vector<Fp> pre(2 * pts.size() + 1);
+        batch_to_affine(pts.data(), pts.size(), xs.data(), ys.data(), pre.data());
+    }
+
+    // the same over arrays (xs, ys zeroed by the caller; pre: 2n + 1 elements)
+    static void batch_to_affine(const Xyzz* pts, size_t n, Fp* xs, Fp* ys, Fp* pre) {
         pre[0] = Mod::one();
         for (size_t i = 0; i < n; i++) {
             Fp zz = is_id(pts[i]) ? Mod::one() : pts[i].ZZ;

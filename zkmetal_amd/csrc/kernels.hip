@@ -9,10 +9,7 @@
 //                     (replaces the CPU counting sort, MSMEngine.swift:595-661)
 //   k_accumulate      load-balanced XYZZ mixed additions into buckets
 //                     (replaces msm_kernels.metal:16-62)
-//   k_merge_runs / k_merge_long   bucket partials that crossed lane boundaries
-//   k_br_rowcol / k_br_bits  bucket reduction: window sum = U + sum_b 2^b Q_b,
-//                     Q_b bit-plane sums of the bucket index (replaces the
-//                     running sums of msm_kernels.metal:152-248)
+// then the merge, the bucket reduction and the window combine (reduce.hip).
 // The weighting by 2^b, the window combine (Horner over windows) and the
 // affine normalisation are a short serial tail that runs on the host
 // (MSMEngine.swift:899-904 does its Horner there too).
@@ -26,6 +23,7 @@
 #include "glv.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
+#include "segments.hpp"
 
 namespace zk {
 
@@ -35,17 +33,6 @@ using Ap = Arith<Bn254Fp>;
 using Ar = Arith<Bn254Fr>;
 
 // ------------------------------------------------------------------ helpers
-
-// largest j in [0, n) with pre[j] <= x (pre ascending, pre[0] == 0)
-__device__ __forceinline__ uint32_t upper_index(const uint64_t* pre, uint32_t n, uint64_t x) {
-    uint32_t lo = 0, hi = n;  // invariant: pre[lo] <= x < pre[hi] (pre[n] = inf)
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (pre[mid] <= x) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
 
 // Sort key of a bucket index x < 2^15: low 7 bits in byte 0, the rest in
 // byte 1.  A real key's low byte is then <= 0x7f, so the first radix pass
@@ -83,28 +70,8 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* l
     return off + inc - v;
 }
 
-// Sum over aligned groups of P lanes (P a power of two <= 64, uniform across
-// the wave); the group's first lane returns the group total.  Cross-lane data
-// moves with ds_bpermute shuffles, no LDS, no barriers.
-__device__ __forceinline__ Fq shfl_down_fq(const Fq& a, uint32_t d) {
-    Fq r;
-#pragma unroll
-    for (int i = 0; i < 9; i++) r.v[i] = __shfl_down(a.v[i], d);
-    return r;
-}
-
-__device__ __forceinline__ QXyzz shfl_down_qxyzz(const QXyzz& a, uint32_t d) {
-    QXyzz r;
-    r.X = shfl_down_fq(a.X, d);
-    r.Y = shfl_down_fq(a.Y, d);
-    r.ZZ = shfl_down_fq(a.ZZ, d);
-    r.ZZZ = shfl_down_fq(a.ZZZ, d);
-    return r;
-}
-
-// Curve policies of the bucket kernels (accumulation, merge, reduction): the
-// stored point type and its loads / stores, the affine table point, and the
-// additions.  G1Curve<F>: XYZZ over one field (BN254 G1 over Fp, Grumpkin
+// Curve policies of the accumulation: the stored point type and its store, the
+// affine table point, and the addition.  G1Curve<F>: XYZZ over one field (BN254 G1 over Fp, Grumpkin
 // over Fr), one 128-byte table slot per entry, 144-byte points.  G2Curve:
 // XYZZ over Fp2 (BN254 G2), two slots per entry, two 144-byte halves per
 // point.  kSlots: table slots per entry.
@@ -114,43 +81,12 @@ struct G1Curve {
     using Af = QAff;
     static constexpr uint32_t kSlots = 1;
     static constexpr uint64_t kPtBytes = kBucketBytes;
-    static __device__ __forceinline__ Pt identity() { return qxyzz_identity(); }
-    static __device__ __forceinline__ Pt select(bool c, const Pt& a, const Pt& b) { return qxyzz_select(c, a, b); }
     static __device__ __forceinline__ Pt run_start() { return Arith<F>::qxyzz_run_start(); }
     static __device__ __forceinline__ void madd_run(Pt& a, bool& id, const Af& q) {
         Arith<F>::qxyzz_madd_run(a, id, q.x, q.y);
     }
-    static __device__ __forceinline__ void add(Pt& a, const Pt& b) { Arith<F>::qxyzz_add(a, b); }
-    static __device__ __forceinline__ Pt shfl_down(const Pt& a, uint32_t d) { return shfl_down_qxyzz(a, d); }
     static __device__ __forceinline__ Af load_tab(const uint4* t, uint64_t e, bool neg) { return load_qtab(t, e, neg); }
-    static __device__ __forceinline__ Pt load(const uint4* b, uint64_t i) { return load_qxyzz(b, i); }
     static __device__ __forceinline__ void store(uint4* b, uint64_t i, const Pt& p) { store_qxyzz(b, i, p); }
-    static __device__ __forceinline__ void store_host(uint4* b, uint64_t i, const Pt& p) {
-        store_xyzz(b, i, Arith<F>::qxyzz_to_xyzz(p));
-    }
-    static __device__ __forceinline__ Pt dbl(const Pt& p) { return Arith<F>::qxyzz_dbl(p); }
-    static __device__ __forceinline__ Pt dbl_k(const Pt& p, uint32_t k) { return Arith<F>::qxyzz_dbl_k(p, k); }
-    // result slot i (96 B): the normalised Jacobian X | Y | Z in the 2^256
-    // Montgomery form, canonical: (x, y, 1), the identity (1, 1, 0)
-    static __device__ __forceinline__ void store_result(uint4* b, uint64_t i, const Pt& p) {
-        using A = Arith<F>;
-        const Fp one = A::fq_to_fp(A::fq_one());
-        Fp x = one, y = one, z = fp_zero();
-        if (!A::qxyzz_is_id(p)) {
-            // 1/ZZ = ZZZ / (ZZ ZZZ), 1/ZZZ = ZZ / (ZZ ZZZ): one inversion
-            const Fq inv = A::fq_inv(A::fq_mul(p.ZZ, p.ZZZ));
-            x = A::fq_to_fp(A::fq_mul(p.X, A::fq_mul(p.ZZZ, inv)));
-            y = A::fq_to_fp(A::fq_mul(p.Y, A::fq_mul(p.ZZ, inv)));
-            z = one;
-        }
-        uint4* o = b + i * 6;
-        const Fp* f[3] = {&x, &y, &z};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            o[2 * k] = make_uint4(f[k]->v[0], f[k]->v[1], f[k]->v[2], f[k]->v[3]);
-            o[2 * k + 1] = make_uint4(f[k]->v[4], f[k]->v[5], f[k]->v[6], f[k]->v[7]);
-        }
-    }
 };
 
 struct G2Curve {
@@ -158,63 +94,13 @@ struct G2Curve {
     using Af = QAff2;
     static constexpr uint32_t kSlots = 2;
     static constexpr uint64_t kPtBytes = 2 * kBucketBytes;
-    static __device__ __forceinline__ Pt identity() { return G2Arith::identity(); }
-    static __device__ __forceinline__ Pt select(bool c, const Pt& a, const Pt& b) { return G2Arith::select(c, a, b); }
     static __device__ __forceinline__ Pt run_start() { return G2Arith::run_start(); }
     static __device__ __forceinline__ void madd_run(Pt& a, bool& id, const Af& q) {
         G2Arith::madd_run(a, id, q.x, q.y);
     }
-    static __device__ __forceinline__ void add(Pt& a, const Pt& b) { G2Arith::add(a, b); }
-    static __device__ __forceinline__ Pt shfl_down(const Pt& a, uint32_t d) {
-        const QXyzz x = shfl_down_qxyzz(QXyzz{a.X.c0, a.Y.c0, a.ZZ.c0, a.ZZZ.c0}, d);
-        const QXyzz y = shfl_down_qxyzz(QXyzz{a.X.c1, a.Y.c1, a.ZZ.c1, a.ZZZ.c1}, d);
-        return Pt{Fq2{x.X, y.X}, Fq2{x.Y, y.Y}, Fq2{x.ZZ, y.ZZ}, Fq2{x.ZZZ, y.ZZZ}};
-    }
     static __device__ __forceinline__ Af load_tab(const uint4* t, uint64_t e, bool neg) { return load_qtab2(t, e, neg); }
-    static __device__ __forceinline__ Pt load(const uint4* b, uint64_t i) { return load_qxyzz2(b, i); }
     static __device__ __forceinline__ void store(uint4* b, uint64_t i, const Pt& p) { store_qxyzz2(b, i, p); }
-    static __device__ __forceinline__ void store_host(uint4* b, uint64_t i, const Pt& p) { store_host_xyzz2(b, i, p); }
 };
-
-// Lane-sum then group tree with ONE addition site: steps 0..nload-1 add the
-// lane's own elements (load(e) returns the e-th, or the identity), the next
-// log2(P) steps add the partner's partial (shuffle tree over aligned groups of
-// P lanes).  nload and P must be wave-uniform.  Keeping a single inlined
-// addition halves the code of the latency-bound reduction kernels.
-__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = max(v, (uint32_t)__shfl_xor(v, d));
-    return v;
-}
-
-// point i of b where `valid`, else the identity: limb-wise selects (a
-// conditional load of a whole point as one value made the compiler stage it
-// through scratch memory); an invalid lane reads point 0, which every such
-// buffer holds
-template <class C>
-__device__ __forceinline__ typename C::Pt load_or_id(const uint4* b, uint64_t i, bool valid) {
-    return C::select(valid, C::load(b, valid ? i : 0), C::identity());
-}
-
-template <class C, class Load>
-__device__ __forceinline__ typename C::Pt sum_then_tree(uint32_t nload, uint32_t P, Load load) {
-    const uint32_t lane = __lane_id();
-    uint32_t levels = 0;
-    while ((1u << levels) < P) levels++;
-    typename C::Pt acc = C::identity();
-#pragma unroll 1
-    for (uint32_t st = 0; st < nload + levels; st++) {
-        typename C::Pt q;
-        if (st < nload) {
-            q = load(st);
-        } else {
-            const uint32_t s = P >> (st - nload + 1);
-            q = C::select((lane & (P - 1)) >= s, C::identity(), C::shfl_down(acc, s));
-        }
-        C::add(acc, q);
-    }
-    return acc;
-}
 
 // -------------------------------------------------------- base table / phi
 // table[2i] = P_i, table[2i+1] = phi(P_i) = (beta x, y): affine, coordinates
@@ -953,298 +839,6 @@ __global__ __launch_bounds__(256) void k_accumulate(
     }
 }
 
-// ------------------------------------------------------ partial merging
-// Records with equal key are contiguous (a bucket's partials come from
-// consecutive lanes; padding of empty lanes carries key 0x7fffffff).
-// k_merge_runs: the lane holding the first record of a run with at most
-// `limit` payload records (and at most 3*limit records in all) sums it and
-// writes dest[key]; a run of at most 64 records is appended to mid_list, a
-// longer one to long_list.  k_merge_mid: eight lanes per listed run (eight
-// runs per wave), each summing every eighth record, then a 3-level shuffle
-// tree.  k_merge_long: one 256-lane workgroup per listed run, a shuffle tree
-// per wave, then one lane adds the four wave partials: depth len/256 + 9.
-
-template <class C>
-__global__ __launch_bounds__(256) void k_merge_runs(const uint32_t* __restrict__ keys,
-                                                    const uint4* __restrict__ pts, uint64_t nrec,
-                                                    uint32_t limit, uint4* __restrict__ dest,
-                                                    uint32_t* __restrict__ long_count,
-                                                    uint32_t* __restrict__ long_list,
-                                                    uint32_t* __restrict__ mid_count,
-                                                    uint32_t* __restrict__ mid_list,
-                                                    uint32_t list_cap) {
-    // lane i looks at records 2i and 2i+1 (one accumulation lane's head and
-    // tail slots); at most one of them starts a run with a payload
-    const uint64_t i2 = 2 * ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (i2 >= nrec) return;
-    for (uint64_t i = i2; i < i2 + 2 && i < nrec; i++) {
-        const uint32_t k = keys[i] & ZK_REC_KEYMASK;
-        if (k == ZK_REC_KEYMASK) continue;  // padding
-        if (i > 0 && (keys[i - 1] & ZK_REC_KEYMASK) == k) continue;
-        uint64_t j = i;
-        uint32_t valid = 0;
-        while (j < nrec && valid <= limit && j - i <= 3 * limit) {
-            const uint32_t kj = keys[j];
-            if ((kj & ZK_REC_KEYMASK) != k) break;
-            valid += (kj & ZK_REC_INVALID) ? 0u : 1u;
-            j++;
-        }
-        if (valid > limit || (j - i > 3 * limit && j < nrec && (keys[j] & ZK_REC_KEYMASK) == k)) {
-            // records are sorted by key: the run is longer than 64 records
-            // iff record i + 64 still carries its key
-            const bool is_long = i + 64 < nrec && (keys[i + 64] & ZK_REC_KEYMASK) == k;
-            const uint32_t slot = atomicAdd(is_long ? long_count : mid_count, 1u);
-            if (slot < list_cap) (is_long ? long_list : mid_list)[slot] = (uint32_t)i;
-            continue;
-        }
-        bool has = false;
-        typename C::Pt acc = C::identity();
-        for (uint64_t p = i; p < j; p++) {
-            if (!(keys[p] & ZK_REC_INVALID)) {
-                typename C::Pt q = C::load(pts, p);
-                if (has) C::add(acc, q);
-                else acc = q;
-                has = true;
-            }
-        }
-        if (has) C::store(dest, k, acc);
-    }
-}
-
-template <class C>
-__global__ __launch_bounds__(256) void k_merge_mid(const uint32_t* __restrict__ keys,
-                                                   const uint4* __restrict__ pts, uint64_t nrec,
-                                                   const uint32_t* __restrict__ mid_count,
-                                                   const uint32_t* __restrict__ mid_list,
-                                                   uint32_t list_cap, uint4* __restrict__ dest) {
-    const uint32_t n = min(*mid_count, list_cap);
-    const uint32_t lane = __lane_id(), sub = lane & 7u;
-    const uint64_t wave = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const uint64_t nwaves = (uint64_t)gridDim.x * 4;
-    for (uint64_t base = wave * 8; base < n; base += nwaves * 8) {  // uniform per wave
-        const uint64_t run = base + (lane >> 3);
-        uint64_t start = 0;
-        uint32_t k = 0, cnt = 0;
-        bool has = false;
-        if (run < n) {
-            start = mid_list[run];
-            k = keys[start] & ZK_REC_KEYMASK;
-            for (uint64_t p = start + sub; p < start + 64 && p < nrec; p += 8) {
-                const uint32_t kr = keys[p];
-                if ((kr & ZK_REC_KEYMASK) != k) break;
-                cnt++;
-                has |= !(kr & ZK_REC_INVALID);
-            }
-        }
-        const typename C::Pt acc = sum_then_tree<C>(wave_max(cnt), 8, [&](uint32_t e) {
-            const uint64_t p = start + sub + 8ull * e;
-            return load_or_id<C>(pts, p, e < cnt && !(keys[p] & ZK_REC_INVALID));
-        });
-        // the group's first lane stores if any lane of the group had a payload
-        const uint64_t hb = __ballot(has);
-        if (run < n && sub == 0 && ((hb >> (lane & ~7u)) & 0xffull)) C::store(dest, k, acc);
-    }
-}
-
-template <class C>
-__global__ __launch_bounds__(256) void k_merge_long(const uint32_t* __restrict__ keys,
-                                                    const uint4* __restrict__ pts, uint64_t nrec,
-                                                    const uint32_t* __restrict__ long_count,
-                                                    const uint32_t* __restrict__ long_list,
-                                                    uint32_t long_cap, uint4* __restrict__ dest) {
-    __shared__ uint4 part[4][C::kPtBytes / 16];
-    __shared__ uint32_t part_has[4];
-    const uint32_t n = min(*long_count, long_cap);
-    const uint32_t t = threadIdx.x, wv = t >> 6, lane = __lane_id();
-    for (uint32_t run = blockIdx.x; run < n; run += gridDim.x) {  // uniform per workgroup
-        const uint64_t start = long_list[run];
-        const uint32_t k = keys[start] & ZK_REC_KEYMASK;
-        uint32_t cnt = 0;
-        bool has = false;
-        for (uint64_t p = start + t; p < nrec; p += 256) {
-            const uint32_t kr = keys[p];
-            if ((kr & ZK_REC_KEYMASK) != k) break;
-            cnt++;
-            has |= !(kr & ZK_REC_INVALID);
-        }
-        typename C::Pt acc = sum_then_tree<C>(wave_max(cnt), 64, [&](uint32_t e) {
-            const uint64_t p = start + t + 256ull * e;
-            return load_or_id<C>(pts, p, e < cnt && !(keys[p] & ZK_REC_INVALID));
-        });
-        const bool wave_has = __ballot(has) != 0;
-        if (lane == 0) {
-            C::store(&part[wv][0], 0, acc);
-            part_has[wv] = wave_has ? 1u : 0u;
-        }
-        __syncthreads();
-        if (t == 0) {
-#pragma unroll 1
-            for (uint32_t w = 1; w < 4; w++) {
-                const typename C::Pt o = C::load(&part[w][0], 0);
-                C::add(acc, o);
-            }
-            if (part_has[0] | part_has[1] | part_has[2] | part_has[3]) C::store(dest, k, acc);
-        }
-        __syncthreads();  // LDS partials are reused by the next run
-    }
-}
-
-// ------------------------------------------------------ bucket reduction
-// Window sum S = sum_k (k+1) B_k over bucket keys k < 2^(c-1).  Write
-// k = hi * 2^g + lo (g = (c-1)/2 low bits, h = c-1-g high bits).  Then
-//   S = U + sum_{b<g} 2^b Pl_b + sum_{b<h} 2^(g+b) Ph_b,
-//   U = sum_lo C_lo,  Pl_b = sum_{lo: bit b} C_lo,  Ph_b = sum_{hi: bit b} R_hi,
-// with row sums R_hi = sum_lo B_{hi,lo} and column sums C_lo = sum_hi B_{hi,lo}
-// (two additions per bucket in all).  k_br_rowcol: a row of 2^g buckets is
-// summed by P_r = max(1, 2^g/per) lanes (`per` buckets each, then a
-// log2(P_r) shuffle tree), a column of 2^h buckets by P_c = max(1, 2^h/per)
-// lanes; rows and columns of a segment start on wave boundaries so P is
-// wave-uniform.  per = 8..32 is chosen by the planner from the call's size.
-// k_br_bits: one wave per output point, bits[s*16 + j]: j = 0 -> U,
-// 1..g -> Pl_{j-1}, g+1..c-1 -> Ph_{j-1-g}.  The host applies the powers of 2.
-
-__device__ __forceinline__ void seg_shape(uint32_t nbk, uint32_t& g, uint32_t& h) {
-    const uint32_t cb = 31 - __clz(nbk);  // c - 1
-    g = cb >> 1;
-    h = cb - g;
-}
-
-__device__ __forceinline__ uint32_t lanes_per(uint32_t len, uint32_t per) { return len >= per ? len / per : 1; }
-
-template <class C>
-__global__ __launch_bounds__(256) void k_br_rowcol(const SegDesc* __restrict__ segs,
-                                                   const uint64_t* __restrict__ seg_wave0,
-                                                   const uint64_t* __restrict__ seg_rc0,
-                                                   uint32_t nseg, uint64_t wave_lo, uint64_t wave_hi,
-                                                   uint32_t per, const uint4* __restrict__ buckets,
-                                                   uint4* __restrict__ rc) {
-    const uint64_t wave = wave_lo + (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wave >= wave_hi) return;
-    const uint32_t lane = __lane_id();
-    const uint32_t s = upper_index(seg_wave0, nseg, wave);
-    const SegDesc sg = segs[s];
-    uint32_t g, h;
-    seg_shape(sg.nbk, g, h);
-    const uint32_t nrow = 1u << h, ncol = 1u << g;
-    const uint32_t Pr = lanes_per(ncol, per), Pc = lanes_per(nrow, per);
-    const uint32_t row_waves = (nrow * Pr + 63) / 64;
-    uint32_t w = (uint32_t)(wave - seg_wave0[s]);
-    const bool rows = w < row_waves;
-    if (!rows) w -= row_waves;
-    const uint32_t P = rows ? Pr : Pc;
-    const uint32_t li = w * 64 + lane;
-    const uint32_t item = li / P, part = li % P;
-    const uint32_t nitem = rows ? nrow : ncol;
-    const uint32_t len = rows ? ncol : nrow;  // buckets per item
-    const uint32_t cnt = len / P;  // buckets this lane sums
-    const typename C::Pt acc = sum_then_tree<C>(cnt, P, [&](uint32_t e) {
-        const uint32_t x = part * cnt + e;
-        const uint64_t kk = rows ? ((uint64_t)item << g) + x : ((uint64_t)x << g) + item;
-        return load_or_id<C>(buckets, sg.bkt0 + kk, item < nitem);
-    });
-    if (item < nitem && part == 0) C::store(rc, seg_rc0[s] + (rows ? item : nrow + item), acc);
-}
-
-// index of the i-th value with bit b set: insert a 1 at bit position b
-__device__ __forceinline__ uint32_t with_bit(uint32_t i, uint32_t b) {
-    return ((i >> b) << (b + 1)) | (1u << b) | (i & ((1u << b) - 1u));
-}
-
-template <class C>
-__global__ __launch_bounds__(256) void k_br_bits(const SegDesc* __restrict__ segs,
-                                                 const uint64_t* __restrict__ seg_rc0,
-                                                 uint32_t seg_lo, uint32_t seg_hi, const uint4* __restrict__ rc,
-                                                 uint4* __restrict__ bits, int host_form) {
-    const uint64_t item = (uint64_t)seg_lo * 16 + (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const uint32_t s = (uint32_t)(item >> 4), j = (uint32_t)(item & 15u);
-    if (s >= seg_hi) return;
-    const uint32_t lane = __lane_id();
-    const SegDesc sg = segs[s];
-    uint32_t g, h;
-    seg_shape(sg.nbk, g, h);
-    if (j > g + h) return;
-    const uint64_t R0 = seg_rc0[s], C0 = R0 + (1u << h);
-    // element list: U -> all columns; Pl_b -> columns with bit b; Ph_b -> rows with bit b
-    uint64_t base;
-    uint32_t count, b = 0;
-    bool masked;
-    if (j == 0) {
-        base = C0; count = 1u << g; masked = false;
-    } else if (j <= g) {
-        base = C0; b = j - 1; count = 1u << (g - 1); masked = true;
-    } else {
-        base = R0; b = j - 1 - g; count = 1u << (h - 1); masked = true;
-    }
-    // count is a power of 2: lanes take elements lane, lane+64, ...
-    const uint32_t P = count >= 64 ? 64u : count;
-    const typename C::Pt acc = sum_then_tree<C>((count + 63) / 64, P, [&](uint32_t e) {
-        const uint32_t i = lane + 64 * e;
-        return load_or_id<C>(rc, base + (masked ? with_bit(i, b) : i), i < count);
-    });
-    if (lane == 0) {
-        if (host_form) C::store_host(bits, item, acc);  // for the host tail
-        else C::store(bits, item, acc);                 // for k_tail_windows
-    }
-}
-
-// ------------------------------------------------ window combine on the device
-// The device form of the call's tail (the host form is Engine::run's
-// host_tail): result_j = sum_w 2^(cstep w) S_w over the MSM's segments w,
-// S_w = U_w + sum_{t < c-1} 2^t Q_{w,t}, the planes k_br_bits stored
-// (bits[s*16] = U, bits[s*16 + 1 + t] = Q_t), then the affine normalisation;
-// cstep = c for plain windows, 0 for window-shifted segments (a plain sum).
-// The reference does its window combine on the host
-// (Sources/zkMetal/MSM/MSMEngine.swift:899-904); on the device it lets a
-// captured graph end with final results.  The doubling chain is inherently
-// serial (2^127 S_top needs 127 doublings), so sixteen lanes per segment
-// compute S_w, then one lane per MSM runs the Horner over segments and the
-// inversion.
-
-// k_tail_windows: sixteen lanes per segment (four segments per wave): lane
-// t < c - 1 doubles plane Q_t t times (a Jacobian chain), lane 15 holds U,
-// then a 4-level shuffle tree sums the sixteen.  The longest chain is c - 2
-// doublings and four additions, against c - 2 doublings and c - 1 additions
-// one after another in a Horner over the planes.
-template <class C>
-__global__ __launch_bounds__(64) void k_tail_windows(const SegDesc* __restrict__ segs,
-                                                     const MsmDesc* __restrict__ msms, uint32_t nseg,
-                                                     const uint4* __restrict__ bits,
-                                                     uint4* __restrict__ wins) {
-    const uint32_t t = threadIdx.x & 15u;
-    const uint32_t sidx = (blockIdx.x * 64 + threadIdx.x) >> 4;
-    const bool valid = sidx < nseg;
-    const uint32_t s = valid ? sidx : 0u;
-    const uint32_t c = msms[segs[s].msm].c;
-    const uint64_t b0 = (uint64_t)s * 16;
-    typename C::Pt v = C::identity();
-    if (valid && t + 1 < c) v = C::dbl_k(C::load(bits, b0 + 1 + t), t);  // 2^t Q_t
-    if (valid && t == 15) v = C::load(bits, b0);                         // U (c - 1 <= 15 planes)
-#pragma unroll
-    for (uint32_t d = 8; d >= 1; d >>= 1) {
-        const typename C::Pt o = C::shfl_down(v, d);
-        if (t < d) C::add(v, o);
-    }
-    if (valid && t == 0) C::store(wins, s, v);
-}
-
-template <class C>
-__global__ __launch_bounds__(64) void k_tail_combine(const MsmDesc* __restrict__ msms, uint32_t nmsm,
-                                                     const uint4* __restrict__ wins,
-                                                     uint4* __restrict__ out) {
-    const uint32_t j = blockIdx.x * 64 + threadIdx.x;
-    if (j >= nmsm) return;
-    const MsmDesc m = msms[j];
-    typename C::Pt acc = C::load(wins, m.seg0 + m.nseg - 1);
-#pragma unroll 1
-    for (int w = (int)m.nseg - 2; w >= 0; w--) {
-        // 2^c acc, in Jacobian coordinates (window-shifted segments: cstep = 0,
-        // their sums already carry the window weights)
-        if (m.cstep) acc = C::dbl_k(acc, m.cstep);
-        C::add(acc, C::load(wins, m.seg0 + w));
-    }
-    C::store_result(out, j, acc);
-}
-
 // ------------------------------------------------ synthetic base table
 // table[t0 + 2i] = k_i * G, table[t0 + 2i + 1] = phi(k_i * G), from a host
 // table gtab[w*256 + b] = b * 2^(8w) * G (affine, entry 0 = (0,0)).
@@ -1709,80 +1303,6 @@ void launch_accumulate(CurveId cv, const SegDesc* segs, const uint64_t* seg_lane
     else if (cv == CurveId::Bn254G2) ZK_ACC(G2Curve);
     else ZK_ACC(G1Curve<Bn254Fp>);
 #undef ZK_ACC
-}
-
-template <class C>
-static void merge_runs_t(const uint32_t* keys, const void* pts, uint64_t nrec, uint32_t limit,
-                         void* dest, uint32_t* counts, uint32_t* lists, uint32_t list_cap,
-                         hipStream_t st) {
-    uint32_t* long_list = lists;
-    uint32_t* mid_list = lists + list_cap;
-    hipLaunchKernelGGL(k_merge_runs<C>, dim3(blocks_for((nrec + 1) / 2, 256)), dim3(256), 0, st, keys,
-                       (const uint4*)pts, nrec, limit, (uint4*)dest, counts, long_list,
-                       counts + 1, mid_list, list_cap);
-    // grid-stride over the lists (their lengths are known on the device only)
-    hipLaunchKernelGGL(k_merge_mid<C>, dim3(std::min<uint32_t>(blocks_for(list_cap, 32), 1024)), dim3(256),
-                       0, st, keys, (const uint4*)pts, nrec, (const uint32_t*)(counts + 1),
-                       (const uint32_t*)mid_list, list_cap, (uint4*)dest);
-    hipLaunchKernelGGL(k_merge_long<C>, dim3(std::min<uint32_t>(list_cap, 2048)), dim3(256), 0, st, keys,
-                       (const uint4*)pts, nrec, (const uint32_t*)counts,
-                       (const uint32_t*)long_list, list_cap, (uint4*)dest);
-}
-
-void launch_merge_runs(CurveId cv, const uint32_t* keys, const void* pts, uint64_t nrec,
-                       uint32_t limit, void* dest, uint32_t* counts, uint32_t* lists,
-                       uint32_t list_cap, hipStream_t st) {
-    if (!nrec || !list_cap) return;
-    if (cv == CurveId::Grumpkin)
-        merge_runs_t<G1Curve<Bn254Fr>>(keys, pts, nrec, limit, dest, counts, lists, list_cap, st);
-    else if (cv == CurveId::Bn254G2)
-        merge_runs_t<G2Curve>(keys, pts, nrec, limit, dest, counts, lists, list_cap, st);
-    else
-        merge_runs_t<G1Curve<Bn254Fp>>(keys, pts, nrec, limit, dest, counts, lists, list_cap, st);
-}
-
-template <class C>
-static void bucket_reduce_t(const SegDesc* segs, const uint64_t* seg_wave0, const uint64_t* seg_rc0,
-                            uint32_t nseg, uint32_t seg_lo, uint32_t seg_hi, uint64_t wave_lo,
-                            uint64_t wave_hi, uint32_t per, const void* buckets, void* rc, void* bits,
-                            bool host_form, hipStream_t st) {
-    hipLaunchKernelGGL(k_br_rowcol<C>, dim3(blocks_for(wave_hi - wave_lo, 4)), dim3(256), 0, st, segs,
-                       seg_wave0, seg_rc0, nseg, wave_lo, wave_hi, per, (const uint4*)buckets, (uint4*)rc);
-    const uint64_t bit_items = (uint64_t)(seg_hi - seg_lo) * 16;
-    hipLaunchKernelGGL(k_br_bits<C>, dim3(blocks_for(bit_items, 4)), dim3(256), 0, st, segs,
-                       seg_rc0, seg_lo, seg_hi, (const uint4*)rc, (uint4*)bits, host_form ? 1 : 0);
-}
-
-void launch_bucket_reduce(CurveId cv, const SegDesc* segs, const uint64_t* seg_wave0,
-                          const uint64_t* seg_rc0, uint32_t nseg, uint32_t seg_lo, uint32_t seg_hi,
-                          uint64_t wave_lo, uint64_t wave_hi, uint32_t per, const void* buckets, void* rc,
-                          void* bits, bool host_form, hipStream_t st) {
-    if (wave_hi <= wave_lo || seg_hi <= seg_lo) return;
-    if (cv == CurveId::Grumpkin)
-        bucket_reduce_t<G1Curve<Bn254Fr>>(segs, seg_wave0, seg_rc0, nseg, seg_lo, seg_hi, wave_lo, wave_hi, per,
-                                          buckets, rc, bits, host_form, st);
-    else if (cv == CurveId::Bn254G2)
-        bucket_reduce_t<G2Curve>(segs, seg_wave0, seg_rc0, nseg, seg_lo, seg_hi, wave_lo, wave_hi, per, buckets,
-                                 rc, bits, true, st);
-    else
-        bucket_reduce_t<G1Curve<Bn254Fp>>(segs, seg_wave0, seg_rc0, nseg, seg_lo, seg_hi, wave_lo, wave_hi, per,
-                                          buckets, rc, bits, host_form, st);
-}
-
-void launch_tail(CurveId cv, const SegDesc* segs, const MsmDesc* msms, uint32_t nseg, uint32_t nmsm,
-                 const void* bits, void* wins, void* out, hipStream_t st) {
-    if (!nseg || !nmsm) return;
-    if (cv == CurveId::Grumpkin) {
-        hipLaunchKernelGGL(k_tail_windows<G1Curve<Bn254Fr>>, dim3((nseg + 3) / 4), dim3(64), 0, st, segs,
-                           msms, nseg, (const uint4*)bits, (uint4*)wins);
-        hipLaunchKernelGGL(k_tail_combine<G1Curve<Bn254Fr>>, dim3((nmsm + 63) / 64), dim3(64), 0, st, msms,
-                           nmsm, (const uint4*)wins, (uint4*)out);
-    } else if (cv == CurveId::Bn254) {
-        hipLaunchKernelGGL(k_tail_windows<G1Curve<Bn254Fp>>, dim3((nseg + 3) / 4), dim3(64), 0, st, segs,
-                           msms, nseg, (const uint4*)bits, (uint4*)wins);
-        hipLaunchKernelGGL(k_tail_combine<G1Curve<Bn254Fp>>, dim3((nmsm + 63) / 64), dim3(64), 0, st, msms,
-                           nmsm, (const uint4*)wins, (uint4*)out);
-    }
 }
 
 void launch_gen_bases(const void* ks, const void* gtab, uint64_t n, void* table,

@@ -1,4 +1,4 @@
-// Host-callable launchers for the MSM kernels (kernels.hip).
+// Host-callable launchers for the MSM kernels (kernels.hip, reduce.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -52,24 +52,31 @@ void launch_accumulate(CurveId cv, const SegDesc* segs, const uint64_t* seg_lane
                        uint32_t nseg, const MsmDesc* msms, const uint32_t* seg_valid, const uint16_t* keys,
                        const uint32_t* vals, const void* table, const uint32_t* T, uint64_t lane_lo,
                        uint64_t lane_hi, void* buckets, uint32_t* rec_keys, void* rec_pts, hipStream_t st);
-// counts[0] / counts[1]: long / mid run counts (zeroed by the caller);
-// lists: 2 * list_cap words (long list, then mid list)
-void launch_merge_runs(CurveId cv, const uint32_t* keys, const void* pts, uint64_t nrec, uint32_t limit,
-                       void* dest, uint32_t* counts, uint32_t* lists, uint32_t list_cap,
-                       hipStream_t st);
+// what the merge of nrec records can list at most: mid runs, spans of long
+// runs, runs of several spans and their partial sums
+struct MergeCaps {
+    uint32_t mid, spans, runs, parts;
+};
+MergeCaps merge_caps(uint64_t nrec);
+// bytes of the merge's lists and partial sums
+uint64_t merge_lists_bytes(uint64_t nrec, CurveId cv);
+// counts: mid runs, spans, partial sums, runs of several spans listed (zeroed
+// by the caller; more than merge_caps(nrec) means that some were dropped)
+void launch_merge_runs(CurveId cv, const uint32_t* keys, const void* pts, uint64_t nrec, void* dest,
+                       uint32_t* counts, void* lists, hipStream_t st);
 // bits: 16 points per segment (U and the bit-plane sums), in the host form
 // (Xyzz, 2^256 Montgomery, 128 B) for the host tail or in the stored form
-// (144 B) for launch_tail
-// segments [seg_lo, seg_hi) and their row/column waves [wave_lo, wave_hi)
-void launch_bucket_reduce(CurveId cv, const SegDesc* segs, const uint64_t* seg_wave0,
-                          const uint64_t* seg_rc0, uint32_t nseg, uint32_t seg_lo, uint32_t seg_hi,
-                          uint64_t wave_lo, uint64_t wave_hi, uint32_t per, const void* buckets, void* rc,
+// (144 B) for launch_tail; seg_blk0: first row/column block of each segment,
+// blocks: their number; by_lanes: the plan's reduce_lanes
+void launch_bucket_reduce(CurveId cv, const SegDesc* segs, const uint64_t* seg_blk0, const uint64_t* seg_rc0,
+                          uint32_t nseg, uint64_t blocks, uint32_t per, bool by_lanes, const void* buckets, void* rc,
                           void* bits, bool host_form, hipStream_t st);
-// window combine and normalisation on the device (BN254 G1 and Grumpkin):
-// bits in the stored form, wins: nseg stored points (scratch), out: nmsm
-// results of 96 B (normalised Jacobian X | Y | Z, 2^256 Montgomery form)
+// window combine on the device (BN254 G1 and Grumpkin): bits in the stored
+// form, wins: nseg stored points (scratch), out: nmsm sums in the host form
+// (Xyzz, 128 B), or with norm nmsm results of 96 B (normalised Jacobian
+// X | Y | Z, 2^256 Montgomery form)
 void launch_tail(CurveId cv, const SegDesc* segs, const MsmDesc* msms, uint32_t nseg, uint32_t nmsm,
-                 const void* bits, void* wins, void* out, hipStream_t st);
+                 const void* bits, void* wins, void* out, bool norm, hipStream_t st);
 void launch_gen_bases(const void* ks, const void* gtab, uint64_t n, void* table,
                       hipStream_t st);
 // out[i] = k_i * G on Grumpkin, 64-byte affine points (x, y in Fr Montgomery form)
@@ -83,6 +90,8 @@ void launch_test_fp(int op, const void* a, const void* b, void* out, uint64_t n,
                     hipStream_t st);
 void launch_test_xyzz(int op, const void* p, const void* q, void* out, uint64_t n,
                       hipStream_t st);
+// points in the host form: p + q (or 2 p) by lane teams
+void launch_test_team(CurveId cv, bool dbl, const void* p, const void* q, void* out, uint64_t n, hipStream_t st);
 void launch_test_glv(const void* scalars, void* out, uint64_t n, hipStream_t st);
 void launch_copy(const void* src, void* dst, uint64_t bytes, hipStream_t st);
 void launch_probe(int mode, uint32_t blocks, uint32_t iters, uint64_t* out, hipStream_t st);

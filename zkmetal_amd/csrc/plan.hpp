@@ -83,6 +83,15 @@ struct SegDesc {
 // pos + v * wadj + wbase relative to the MSM's table0: for a plain segment
 // (v = 0, wadj = wbase = 0) the position itself.
 
+// Teams (or lanes) that sum one row or column of len buckets: about per
+// buckets each, at most as many as a block has teams (all powers of two).
+constexpr uint32_t reduce_teams(uint32_t len, uint32_t per, uint32_t block_teams) {
+    return len <= per ? 1 : len / per < block_teams ? len / per : block_teams;
+}
+// lanes that share one point in the merge and reduction kernels (team29.hpp):
+// a block of 256 holds 256 / this many teams
+constexpr uint32_t team_lanes(CurveId cv) { return cv == CurveId::Bn254G2 ? 8u : 4u; }
+
 // Merge records: key bit 31 set = no payload (padding); bits 0..30 = index of
 // the bucket (or window sum) the payload belongs to.
 #define ZK_REC_INVALID 0x80000000u

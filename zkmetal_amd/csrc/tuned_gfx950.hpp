@@ -7,10 +7,10 @@
 // start from these tables; zkmsm_set_window_table / _batch_ replace them.
 //
 // kTunedParts / kTunedPer: the launch schedule by call size class ceil(log2
-// entries) -- pipeline parts and buckets per bucket-reduction lane -- for
+// entries) -- pipeline parts and buckets per bucket-reduction lane or team -- for
 // calls of one MSM ([0]) and of several ([1]), from the same sweep; 0 = the
-// built-in rule (default_parts, and 8 to 32 buckets per lane by bucket
-// count).  zkmsm_set_schedule_table replaces them.
+// built-in rule (default_parts, and buckets per lane or team by bucket
+// count, at least 8).  zkmsm_set_schedule_table replaces them.
 #pragma once
 #include <stdint.h>
 
@@ -21,13 +21,12 @@ static const uint32_t kTunedPlain[33] = {0, 0, 0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 10,
 static const uint32_t kTunedBatch[33] = {0, 0, 0, 0, 0, 0, 0, 0, 6, 7, 8, 8, 9, 10, 11, 12, 13,
                                          13, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
-// The sweep kept the built-in parts everywhere and the built-in reduction
-// tile for batched calls; single MSMs of entry classes 2^13 and 2^17 .. 2^21
-// (2^12 .. 2^17 points) ran 4-7% faster with 4 buckets per reduction lane
-// (their reduction is latency-bound: shorter chains before the tree).
+// Small calls leave most of the chip idle, so a shorter chain before the tree
+// wins: with 4 against 8 buckets, 256 points 255 against 263 us, 4097 points
+// 322 against 332, 2^16 points the same.
 static const uint8_t kTunedParts[2][33] = {};
 static const uint8_t kTunedPer[2][33] = {
-    {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 4, 0, 0, 0, 4, 4, 4, 4, 4, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0},
-    {}};
+    {4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0},
+    {4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
 
 }  // namespace zk
