@@ -269,9 +269,11 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
     for (uint32_t k = 0; k < pl.nparts; k++) {
         PlanPart& pt = pl.parts[k];
         uint64_t ent = 0, bk = 0;
+        pt.max_tiles = 0;
         for (uint32_t s = pt.seg_lo; s < pt.seg_hi; s++) {
             ent += pl.segs[s].len;
             bk += pl.segs[s].nbk;
+            pt.max_tiles = std::max(pt.max_tiles, pl.segs[s].ntiles);
         }
         const uint64_t ns_p = pt.seg_hi - pt.seg_lo;
         const uint64_t half_bucket = ent / (2 * std::max<uint64_t>(1, bk));
@@ -285,6 +287,9 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
         pt.chunk_hi = pl.segs[pt.seg_hi - 1].chunk0 + pl.segs[pt.seg_hi - 1].nchunks;
     }
     pl.T = pl.parts[0].T;
+    pl.small_sort = pl.nparts == 1;
+    for (const SegDesc& s : pl.segs)
+        pl.small_sort = pl.small_sort && s.len <= kSmallSortLen && s.nbk <= kSmallSortBuckets;
     // bucket reduction: buckets per lane or team before the tree.  Two
     // additions per bucket on one wave per SIMD (1024 waves) is the least
     // chain that fills the chip; a shorter one only adds tree levels (down to
@@ -722,7 +727,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         ZK_TRY(rec(ev_[0], st));
         // the decomposition also counts the first sort pass's tile histograms
         launch_decompose(pl.curve, d_msms, d_msm_dtile0, nmsm, pl.dtiles, d_segs, d_scalars, d_table, table_n,
-                         ws.digits, (uint32_t*)ws.hist, d_err, st);
+                         ws.digits, pl.small_sort ? nullptr : (uint32_t*)ws.hist, d_err, st);
         ZK_TRY(rec(ev_dec_, st));
         if (P > 1) {  // the sorts need the digits, not the cleared buckets
             ZK_TRY(hipEventRecord(dep_fork_, st));
@@ -733,14 +738,19 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             const PlanPart& pt = pl.parts[p];
             const uint32_t ns_p = pt.seg_hi - pt.seg_lo;
             ZK_TRY(rec(ev_s0_[p], S));
-            launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo, d_chunk_seg,
-                             pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.digits, nullptr, 0, (uint32_t*)ws.hist,
-                             (uint32_t*)ws.part, (uint32_t*)ws.segvalid, (uint16_t*)ws.keysA,
-                             (uint32_t*)ws.valsA, S, false);
-            launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo, d_chunk_seg,
-                             pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.keysA, (const uint32_t*)ws.valsA, 1,
-                             (uint32_t*)ws.hist, (uint32_t*)ws.part, (uint32_t*)ws.segvalid,
-                             (uint16_t*)ws.keysB, (uint32_t*)ws.valsB, S);
+            if (pl.small_sort) {
+                launch_sort_small(d_segs, ns_p, ws.digits, (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB,
+                                  (uint32_t*)ws.valsB, S);
+            } else {
+                launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
+                                 d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.digits, nullptr, 0,
+                                 (uint32_t*)ws.hist, (uint32_t*)ws.part, (uint32_t*)ws.segvalid,
+                                 (uint16_t*)ws.keysA, (uint32_t*)ws.valsA, S, pt.max_tiles, false);
+                launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
+                                 d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.keysA,
+                                 (const uint32_t*)ws.valsA, 1, (uint32_t*)ws.hist, (uint32_t*)ws.part,
+                                 (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB, (uint32_t*)ws.valsB, S, pt.max_tiles);
+            }
             launch_lane_plan(d_segs, (const uint32_t*)ws.segvalid, pt.seg_lo, ns_p, pt.lane_lo, pt.lane_hi,
                              d_seg_lane0, d_part_T + p, S);
             ZK_TRY(rec(ev_s1_[p], S));

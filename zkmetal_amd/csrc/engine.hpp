@@ -79,6 +79,7 @@ constexpr uint32_t kMaxParts = 8;
 struct PlanPart {
     uint32_t seg_lo, seg_hi, tile_lo, tile_hi, chunk_lo, chunk_hi;
     uint32_t T;  // entries per accumulation lane in this part
+    uint32_t max_tiles;  // sort tiles of its longest segment
     uint64_t lane_lo, lane_hi, entries;
 };
 
@@ -99,6 +100,7 @@ struct Plan {
     uint32_t nparts = 1;
     PlanPart parts[kMaxParts];
     CurveId curve = CurveId::Bn254;
+    bool small_sort = false;  // every segment fits k_sort_small (one part)
     uint32_t G = 8;  // buckets per bucket-reduction lane or team (a power of 2)
     bool reduce_lanes = false;  // rows and columns summed by lanes, else by teams
 };

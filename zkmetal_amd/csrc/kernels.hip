@@ -345,10 +345,14 @@ __device__ __forceinline__ uint32_t window_bits256(const uint32_t k[8], uint32_t
 // v = w % wps, i.e. tiles v * ntw + tin and positions v * ntw * kSortTile +
 // (entry) of the segment, ntw = the window's tiles; a window-shifted MSM
 // (wps > 1) pads each window to whole tiles with "no bucket" digits.
-constexpr int kDecThreads = 256;
-static_assert(kSortTile <= (1 << 15) && kSortTile / 2 / kDecThreads >= 1, "decomposition tiling");
+// A block has kThreads threads.  Each walks its scalars one after another, a
+// chain of ~600 instructions each, so a call too small to fill the chip takes
+// 1024 threads, 2 scalars deep (2^16 points: 43 us with 256 threads, 27 with
+// 512, 20 with 1024); a large one is bound by its LDS atomics and runs best
+// with 512 (2^22 points: 150, 131, 160 us).
+static_assert(kSortTile <= (1 << 15) && kSortTile / 2 / 1024 >= 1, "decomposition tiling");
 
-template <int EPS, bool kModR>
+template <int EPS, bool kModR, int kDecThreads>
 __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __restrict__ msms,
                                                           const uint64_t* __restrict__ msm_dtile0,
                                                           uint32_t nmsm,
@@ -361,17 +365,21 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
     // windows (nwin <= 64) x key byte 0, two 16-bit counts per word (a tile
     // has at most kSortTile <= 2^15 entries, so no count reaches 2^16)
     __shared__ uint32_t cnt[kMaxWindows * 128];
+    __shared__ uint64_t pos0[kMaxWindows];  // first position of window w's entries
     const uint32_t b = blockIdx.x;
     const uint32_t j = upper_index(msm_dtile0, nmsm, b);
     const MsmDesc m = msms[j];
     const uint32_t tin = b - (uint32_t)msm_dtile0[j];
-    for (uint32_t x = threadIdx.x; x < m.nwin * 128u; x += kDecThreads) cnt[x] = 0;
+    const uint32_t ntw = (EPS * m.n + kSortTile - 1) / kSortTile;  // tiles per window
+    if (hist)
+        for (uint32_t x = threadIdx.x; x < m.nwin * 128u; x += kDecThreads) cnt[x] = 0;
+    if (threadIdx.x < m.nwin)
+        pos0[threadIdx.x] = segs[m.seg0 + threadIdx.x / m.wps].ent0 +
+                            (uint64_t)(threadIdx.x % m.wps) * ntw * kSortTile;
     __syncthreads();
     const uint32_t c = m.c, half = 1u << (c - 1), full = 1u << c;
     bool carry_left = false;
     constexpr int kPer = kSortTile / EPS / kDecThreads;  // scalars per thread
-    const uint32_t ntw = (EPS * m.n + kSortTile - 1) / kSortTile;  // tiles per window
-    const uint64_t vstride = (uint64_t)ntw * kSortTile;             // positions per local window
     for (int r = 0; r < kPer; r++) {
         const uint64_t i = (uint64_t)tin * (kSortTile / EPS) + (uint64_t)r * kDecThreads + threadIdx.x;
         const bool live = i < m.n;
@@ -400,15 +408,15 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
                 carry = d > half;
                 if (carry) { d = full - d; neg = 1u; }
                 const uint32_t wd = d ? (key_encode(d - 1u) | (neg << 31)) : ZK_KEY_NONE;
-                reinterpret_cast<uint32_t*>(digits)[segs[m.seg0 + w].ent0 + i] = wd;
-                atomicAdd(&cnt[w * 128 + ((wd & 0xffu) >> 1)], 1u << ((wd & 1u) * 16));
+                reinterpret_cast<uint32_t*>(digits)[pos0[w] + i] = wd;
+                if (hist) atomicAdd(&cnt[w * 128 + ((wd & 0xffu) >> 1)], 1u << ((wd & 1u) * 16));
             }
             carry_left |= carry != 0;
             continue;
         }
         GlvSplit sp = glv_split(k);
         uint32_t carry1 = 0, carry2 = 0;
-        uint32_t v = 0, sg = m.seg0;  // window w: local window v of segment sg
+        uint32_t v = 0;  // local window of w's segment
         for (uint32_t w = 0; w < m.nwin; w++) {
             uint32_t d1 = window_bits128(sp.k1, w, c) + carry1;
             uint32_t d2 = window_bits128(sp.k2, w, c) + carry2;
@@ -420,18 +428,17 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
             const uint32_t vt = v << 16;
             uint32_t w1 = d1 ? (key_encode(d1 - 1u) | vt | (neg1 << 31)) : ZK_KEY_NONE;
             uint32_t w2 = d2 ? (key_encode(d2 - 1u) | vt | (neg2 << 31)) : ZK_KEY_NONE;
-            const uint64_t e = segs[sg].ent0 + v * vstride + 2 * i;
-            digits[e >> 1] = make_uint2(w1, w2);
-            atomicAdd(&cnt[w * 128 + ((w1 & 0xffu) >> 1)], 1u << ((w1 & 1u) * 16));
-            atomicAdd(&cnt[w * 128 + ((w2 & 0xffu) >> 1)], 1u << ((w2 & 1u) * 16));
-            if (++v == m.wps) {
-                v = 0;
-                sg++;
+            digits[(pos0[w] + 2 * i) >> 1] = make_uint2(w1, w2);
+            if (hist) {
+                atomicAdd(&cnt[w * 128 + ((w1 & 0xffu) >> 1)], 1u << ((w1 & 1u) * 16));
+                atomicAdd(&cnt[w * 128 + ((w2 & 0xffu) >> 1)], 1u << ((w2 & 1u) * 16));
             }
+            if (++v == m.wps) v = 0;
         }
         carry_left |= (carry1 | carry2) != 0;
     }
     if (carry_left) atomicOr(err, 1u);
+    if (!hist) return;  // k_sort_small counts for itself
     __syncthreads();
     for (uint32_t x = threadIdx.x; x < m.nwin * 256u; x += kDecThreads) {
         const uint32_t w = x >> 8, d = x & 255u;
@@ -586,6 +593,98 @@ __global__ __launch_bounds__(256) void k_scan_down(const SegDesc* __restrict__ s
         uint4* q = reinterpret_cast<uint4*>(h);
 #pragma unroll
         for (int i = 0; i < 4; i++) q[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+    }
+}
+
+// The three steps in one launch, a block per segment, for segments of few
+// tiles (kScanSegTiles): a segment's counts are walked kScanChunk * 4 at a
+// time, 1.2 us each, against three launches of 4 to 5 us (2^16 points: 4 us
+// against 13).
+__global__ __launch_bounds__(1024) void k_scan_seg(const SegDesc* __restrict__ segs, uint32_t seg_lo,
+                                                   uint32_t* __restrict__ hist, int pass,
+                                                   uint32_t* __restrict__ seg_valid) {
+    __shared__ uint32_t lds16[16];
+    const uint32_t s = seg_lo + blockIdx.x;
+    const SegDesc sg = segs[s];
+    const uint32_t M = 256u * sg.ntiles, none_bin = 0xffu * sg.ntiles;
+    uint32_t carry = 0;
+    for (uint32_t b = 0; b < M; b += 4 * kScanChunk) {
+        const uint32_t i0 = b + 16u * threadIdx.x;
+        uint32_t v[16];
+        uint32_t sum = 0;
+        uint32_t* h = hist + (uint64_t)sg.tile0 * 256 + i0;
+        if (i0 < M) {
+            load16(h, v);
+#pragma unroll
+            for (int i = 0; i < 16; i++) sum += v[i];
+        }
+        uint32_t tot;
+        uint32_t acc = carry + block_exclusive_scan<16>(sum, lds16, &tot);
+        carry += tot;
+        if (i0 < M) {
+            uint32_t o[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                if (pass == 0 && i0 + i == none_bin) seg_valid[s] = acc;
+                o[i] = (uint32_t)sg.ent0 + acc;
+                acc += v[i];
+            }
+            uint4* q = reinterpret_cast<uint4*>(h);
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+        }
+    }
+}
+
+// A whole segment in one block: entries are ranked within their bucket by LDS
+// atomics, the bucket counts scanned, and every entry written to its place.
+// Replaces ten launches of the two passes for a call whose segments all fit
+// (Plan::small_sort): what a small call pays for is the launches and the
+// latency of the scans, not the entries (4097 points: 12 us against 55; the
+// whole call 310 -> 280 us, 256 points 246 -> 213).
+__global__ __launch_bounds__(1024) void k_sort_small(const SegDesc* __restrict__ segs,
+                                                     const uint32_t* __restrict__ digits,
+                                                     uint32_t* __restrict__ seg_valid,
+                                                     uint16_t* __restrict__ out_keys,
+                                                     uint32_t* __restrict__ out_vals) {
+    constexpr uint32_t kPer = kSmallSortLen / 1024;
+    __shared__ uint32_t cnt[kSmallSortBuckets];
+    __shared__ uint32_t lds16[16];
+    const uint32_t s = blockIdx.x;
+    const SegDesc sg = segs[s];
+    for (uint32_t x = threadIdx.x; x < sg.nbk; x += 1024) cnt[x] = 0;
+    uint32_t wd[kPer], rank[kPer];
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; r++) {
+        const uint32_t pos = r * 1024 + threadIdx.x;
+        wd[r] = pos < sg.len ? digits[sg.ent0 + pos] : ZK_KEY_NONE;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; r++) {
+        const uint32_t key = wd[r] & 0xffffu;
+        rank[r] = key != ZK_KEY_NONE ? atomicAdd(&cnt[key_decode(key)], 1u) : 0u;
+    }
+    __syncthreads();
+    uint32_t carry = 0;
+    for (uint32_t b = 0; b < sg.nbk; b += 1024) {
+        const uint32_t x = b + threadIdx.x;
+        const uint32_t c = x < sg.nbk ? cnt[x] : 0u;
+        uint32_t tot;
+        const uint32_t ex = block_exclusive_scan<16>(c, lds16, &tot);
+        if (x < sg.nbk) cnt[x] = carry + ex;
+        carry += tot;
+    }
+    if (threadIdx.x == 0) seg_valid[s] = carry;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; r++) {
+        const uint32_t key = wd[r] & 0xffffu;
+        if (key == ZK_KEY_NONE) continue;
+        const uint64_t g = sg.ent0 + cnt[key_decode(key)] + rank[r];
+        out_keys[g] = (uint16_t)key;
+        // the table entry: the position, shifted to its window's copy
+        out_vals[g] = (r * 1024 + threadIdx.x + ((wd[r] >> 16) & 0xffu) * sg.wadj + sg.wbase) | (wd[r] & 0x80000000u);
     }
 }
 
@@ -1233,33 +1332,51 @@ void launch_decompose(CurveId cv, const MsmDesc* msms, const uint64_t* msm_dtile
                       uint32_t* err, hipStream_t st) {
     if (!dtiles) return;
     const uint64_t* idm = table_idmask(const_cast<void*>(table), table_n, cv);
-    if (cv == CurveId::Grumpkin)
-        hipLaunchKernelGGL((k_decompose<1, false>), dim3(dtiles), dim3(kDecThreads), 0, st, msms, msm_dtile0,
-                           nmsm, segs, (const uint4*)scalars, idm, (uint2*)digits, hist, err);
-    else if (cv == CurveId::Bn254G2)
-        hipLaunchKernelGGL((k_decompose<1, true>), dim3(dtiles), dim3(kDecThreads), 0, st, msms, msm_dtile0,
-                           nmsm, segs, (const uint4*)scalars, idm, (uint2*)digits, hist, err);
-    else
-        hipLaunchKernelGGL((k_decompose<2, false>), dim3(dtiles), dim3(kDecThreads), 0, st, msms, msm_dtile0,
-                           nmsm, segs, (const uint4*)scalars, idm, (uint2*)digits, hist, err);
+    // up to a block per CU: the wide blocks (see k_decompose)
+#define ZK_DEC(EPS, MODR, THREADS)                                                                       \
+    hipLaunchKernelGGL((k_decompose<EPS, MODR, THREADS>), dim3(dtiles), dim3(THREADS), 0, st, msms, msm_dtile0, \
+                       nmsm, segs, (const uint4*)scalars, idm, (uint2*)digits, hist, err)
+    const bool wide = dtiles <= 256;
+    if (cv == CurveId::Grumpkin) {
+        if (wide) ZK_DEC(1, false, 1024);
+        else ZK_DEC(1, false, 512);
+    } else if (cv == CurveId::Bn254G2) {
+        if (wide) ZK_DEC(1, true, 1024);
+        else ZK_DEC(1, true, 512);
+    } else {
+        if (wide) ZK_DEC(2, false, 1024);
+        else ZK_DEC(2, false, 512);
+    }
+#undef ZK_DEC
 }
 
 void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const uint32_t* tile_seg,
                       uint32_t tile_lo, uint32_t ntiles, const uint32_t* chunk_seg, uint32_t chunk_lo,
                       uint32_t nchunks, const void* in_keys, const uint32_t* in_vals, int pass,
                       uint32_t* hist, uint32_t* part, uint32_t* seg_valid, uint16_t* out_keys,
-                      uint32_t* out_vals, hipStream_t st, bool count) {
+                      uint32_t* out_vals, hipStream_t st, uint32_t max_tiles, bool count) {
     if (!ntiles) return;
     if (count)  // else the tile histograms are already in hist
         hipLaunchKernelGGL(k_sort_hist, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
                            in_keys, pass, (const uint32_t*)seg_valid, hist);
-    hipLaunchKernelGGL(k_scan_up, dim3(nchunks), dim3(256), 0, st, segs, chunk_seg, chunk_lo,
-                       (const uint32_t*)hist, part);
-    hipLaunchKernelGGL(k_scan_spine, dim3(nseg), dim3(256), 0, st, segs, seg_lo, part);
-    hipLaunchKernelGGL(k_scan_down, dim3(nchunks), dim3(256), 0, st, segs, chunk_seg, chunk_lo, hist,
-                       (const uint32_t*)part, pass, seg_valid);
+    if (max_tiles <= kScanSegTiles) {
+        hipLaunchKernelGGL(k_scan_seg, dim3(nseg), dim3(1024), 0, st, segs, seg_lo, hist, pass, seg_valid);
+    } else {
+        hipLaunchKernelGGL(k_scan_up, dim3(nchunks), dim3(256), 0, st, segs, chunk_seg, chunk_lo,
+                           (const uint32_t*)hist, part);
+        hipLaunchKernelGGL(k_scan_spine, dim3(nseg), dim3(256), 0, st, segs, seg_lo, part);
+        hipLaunchKernelGGL(k_scan_down, dim3(nchunks), dim3(256), 0, st, segs, chunk_seg, chunk_lo, hist,
+                           (const uint32_t*)part, pass, seg_valid);
+    }
     hipLaunchKernelGGL(k_sort_scatter, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
                        in_keys, in_vals, pass, (const uint32_t*)hist, (const uint32_t*)seg_valid,
+                       out_keys, out_vals);
+}
+
+void launch_sort_small(const SegDesc* segs, uint32_t nseg, const void* digits, uint32_t* seg_valid,
+                       uint16_t* out_keys, uint32_t* out_vals, hipStream_t st) {
+    if (!nseg) return;
+    hipLaunchKernelGGL(k_sort_small, dim3(nseg), dim3(1024), 0, st, segs, (const uint32_t*)digits, seg_valid,
                        out_keys, out_vals);
 }
 

@@ -24,18 +24,23 @@ void launch_build_table(CurveId cv, const void* pts, void* table, uint64_t n, hi
 void launch_shift_windows(void* table, uint64_t n, uint64_t stride, uint32_t c, uint32_t nwin,
                           hipStream_t st);
 // one block per first-pass sort tile of each MSM (msm_dtile0, dtiles blocks):
-// digits, and the first sort pass's tile histograms into hist
+// digits, and the first sort pass's tile histograms into hist (null: none)
 void launch_decompose(CurveId cv, const MsmDesc* msms, const uint64_t* msm_dtile0, uint32_t nmsm,
                       uint32_t dtiles, const SegDesc* segs, const void* scalars,
                       const void* table, uint64_t table_n, void* digits, uint32_t* hist,
                       uint32_t* err, hipStream_t st);
 // one radix pass over segments [seg_lo, seg_lo + nseg): their tiles
-// [tile_lo, tile_lo + ntiles) and scan chunks [chunk_lo, chunk_lo + nchunks)
+// [tile_lo, tile_lo + ntiles) and scan chunks [chunk_lo, chunk_lo + nchunks);
+// max_tiles: the most tiles of one of them
 void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const uint32_t* tile_seg,
                       uint32_t tile_lo, uint32_t ntiles, const uint32_t* chunk_seg, uint32_t chunk_lo,
                       uint32_t nchunks, const void* in_keys, const uint32_t* in_vals, int pass,
                       uint32_t* hist, uint32_t* part, uint32_t* seg_valid, uint16_t* out_keys,
-                      uint32_t* out_vals, hipStream_t st, bool count = true);
+                      uint32_t* out_vals, hipStream_t st, uint32_t max_tiles, bool count = true);
+// segments [0, nseg) sorted by a block each, both passes in one (every segment
+// within kSmallSortLen entries and kSmallSortBuckets buckets)
+void launch_sort_small(const SegDesc* segs, uint32_t nseg, const void* digits, uint32_t* seg_valid,
+                       uint16_t* out_keys, uint32_t* out_vals, hipStream_t st);
 void launch_fill_zero(void* p, uint64_t bytes, hipStream_t st);
 // lanes of k_accumulate resident at once on the device (CUs x workgroups per
 // CU at its register use x 256): a lane count just above it leaves a second,

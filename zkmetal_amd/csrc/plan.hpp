@@ -103,6 +103,10 @@ constexpr int kSortThreads = 512;
 constexpr int kSortWaves = kSortThreads / 64;
 constexpr int kSortItems = 8;
 constexpr int kSortTile = kSortThreads * kSortItems;
+// one-block sort of a whole segment (k_sort_small): entries and buckets at most
+constexpr uint32_t kSmallSortLen = 16384, kSmallSortBuckets = 4096;
+// tiles of a segment up to which one block scans its histogram (k_scan_seg)
+constexpr uint32_t kScanSegTiles = 256;
 constexpr int kScanChunk = 4096;  // histogram counts per scan block (16 per thread)
 
 }  // namespace zk
