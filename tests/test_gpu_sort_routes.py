@@ -1,6 +1,6 @@
 """The sort's routes at their edges against the closed form: a segment just
 within and just past the one-block sort (16384 entries, 4096 buckets), and
-segments on either side of the one-block histogram scan (256 tiles)."""
+segments on either side of the one-block histogram scan (128 tiles)."""
 import pytest
 
 import zkmetal_amd as zk
@@ -17,7 +17,7 @@ SEED = 0x50B7
 def eng():
     e = zk.MetalMSM()
     e.set_window_shift(e.SHIFT_OFF)
-    e.srs_generate(SEED, (1 << 19) + 1)
+    e.srs_generate(SEED, (1 << 18) + 1)
     yield e
     e.close()
 
@@ -39,7 +39,7 @@ def test_one_block_sort_edges(eng, n, c):
         eng.set_window_bits(0)
 
 
-@pytest.mark.parametrize("n", [1 << 19, (1 << 19) + 1])
+@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1])
 def test_one_block_scan_edges(eng, n):
     for parts in (1, 2):
         eng.set_pipeline_parts(parts)

@@ -281,6 +281,7 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
         pt.T = (uint32_t)std::max<uint64_t>(std::max<uint64_t>(4, std::min<uint64_t>(32, half_bucket)),
                                             (ent + cap - 1) / cap);
         pt.entries = ent;
+        pt.nbk = (uint32_t)bk;
         pt.tile_lo = pl.segs[pt.seg_lo].tile0;
         pt.tile_hi = pl.segs[pt.seg_hi - 1].tile0 + pl.segs[pt.seg_hi - 1].ntiles;
         pt.chunk_lo = pl.segs[pt.seg_lo].chunk0;
@@ -290,6 +291,7 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
     pl.small_sort = pl.nparts == 1;
     for (const SegDesc& s : pl.segs)
         pl.small_sort = pl.small_sort && s.len <= kSmallSortLen && s.nbk <= kSmallSortBuckets;
+    pl.parts[0].scan_seg = pl.nparts == 1 && pl.parts[0].max_tiles <= kScanSegTiles;
     // bucket reduction: buckets per lane or team before the tree.  Two
     // additions per bucket on one wave per SIMD (1024 waves) is the least
     // chain that fills the chip; a shorter one only adds tree levels (down to
@@ -398,7 +400,7 @@ int32_t Engine::create(Engine** out) {
 
 void Engine::account_buffers() {
     for (DevBuf* b : {&desc_, &digits_, &keysA_, &valsA_, &keysB_, &valsB_, &hist_, &part_, &segvalid_,
-                      &buckets_, &recAk_, &recAp_, &lists_, &rc_, &winsum_, &err_, &wins_, &res_,
+                      &buckets_, &recAk_, &recAp_, &lists_, &rc_, &winsum_, &err_, &wins_,
                       &pts_in_, &ptable_, &scalars_, &srs_, &gtab_, &gtab_gk_, &gtab_g2_, &tmp_})
         b->acct = &ws_;
 }
@@ -544,8 +546,10 @@ struct HostG2View {
     }
 };
 
+// windows: hw holds the window sums S_w themselves (BN254 G2), one point per
+// segment.
 template <class HC>
-static void host_tail(const Plan& pl, const uint8_t* hw, uint8_t* out) {
+static void host_tail(const Plan& pl, const uint8_t* hw, uint8_t* out, bool windows = false) {
     const uint32_t nmsm = (uint32_t)pl.msms.size();
     std::vector<typename HC::Pt> res(nmsm);
     auto tail = [&](uint32_t jb, uint32_t je) {
@@ -553,6 +557,14 @@ static void host_tail(const Plan& pl, const uint8_t* hw, uint8_t* out) {
             const MsmDesc& m = pl.msms[j];
             const int cb = (int)m.c - 1;  // planes per segment (bucket index bits)
             typename HC::Pt acc = HC::identity();
+            for (int w = (int)m.nseg - 1; windows && w >= 0; w--) {
+                for (uint32_t k = 0; k < m.cstep && !HC::is_id(acc); k++) acc = HC::xdbl(acc);
+                acc = HC::xadd(acc, HC::load(hw + (uint64_t)(m.seg0 + w) * HC::kIn));
+            }
+            if (windows) {
+                res[j] = acc;
+                continue;
+            }
             // Horner over the bits of sum_w 2^(cstep w) S_w: at bit b, segment
             // w adds its plane t = b - cstep w (and U_w at t = 0); plain
             // windows (cstep = c) meet one segment per bit, window-shifted
@@ -602,14 +614,16 @@ WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
     z.lists = merge_lists_bytes(rec_cap, pl.curve);
     z.rc = pl.groups * ptb;
     // bit-plane points: host form for the host tail, stored form for the device's
-    z.bits = nseg * 16 * (dev_tail ? ptb : hpb);
+    // and for BN254 G2, whose window sums (host form) the device makes of them
+    const bool g2 = pl.curve == CurveId::Bn254G2;
+    z.bits = nseg * 16 * (dev_tail || g2 ? ptb : hpb);
     z.err = 32;  // the decomposition flag, the merge's list counters
     z.wins = dev_tail ? nseg * ptb : 0;
     // device tail: the sums, normalised on the host, or (many) the results
     z.res = dev_tail ? nmsm * (nmsm <= kHostNormMsms ? hpb : result_bytes(pl.curve)) : 0;
     // copied back: those (device tail) or the bit planes, then err, then
     // the per-segment valid-entry counts
-    z.back = dev_tail ? z.res : z.bits;
+    z.back = dev_tail ? z.res : g2 ? nseg * hpb : z.bits;
     z.host = z.back + z.err + nseg * 4;
     const uint64_t parts[] = {z.desc, z.digits, z.keys, z.vals, z.keys, z.vals, z.hist, z.part,
                               z.segvalid, z.buckets, z.rec_keys, z.rec_pts, z.lists, z.rc, z.bits,
@@ -639,11 +653,9 @@ int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, 
     ZK_ALLOC(recAp_, z.rec_pts);
     ZK_ALLOC(lists_, z.lists);
     ZK_ALLOC(rc_, z.rc);
-    ZK_ALLOC(winsum_, z.bits);
-    if (dev_tail) {
-        ZK_ALLOC(wins_, z.wins);
-        ZK_ALLOC(res_, z.res);
-    }
+    const bool dev_bits = dev_tail || pl.curve == CurveId::Bn254G2;
+    if (dev_bits) ZK_ALLOC(winsum_, z.bits);
+    if (dev_tail) ZK_ALLOC(wins_, z.wins);
     ZK_ALLOC(err_, z.err);
     ZK_ALLOC(hwin_, z.host);
     Workspace ws;
@@ -661,12 +673,13 @@ int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, 
     ws.recAp = recAp_.p;
     ws.lists = lists_.p;
     ws.rc = rc_.p;
-    ws.bits = winsum_.p;
     ws.err = err_.p;
     ws.wins = wins_.p;
-    ws.res = res_.p;
     ws.hdesc = (uint8_t*)hdesc_.p;
     ws.hw = (uint8_t*)hwin_.p;
+    ws.mapped = true;
+    ws.bits = dev_bits ? winsum_.p : hwin_.p;
+    ws.res = hwin_.p;
     return run_ws(pl, ws, z, dev_tail, graph_mode_, d_scalars, d_table, table_n, out96);
 }
 
@@ -693,7 +706,6 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         reinterpret_cast<uint32_t*>(hb + L.part_T)[p] = p < pl.nparts ? pl.parts[p].T : 0u;
     uint8_t* db = ws.desc;
     const MsmDesc* d_msms = (const MsmDesc*)(db + L.msms);
-    const uint64_t* d_msm_scalar0 = (const uint64_t*)(db + L.msm_scalar0);
     const uint64_t* d_msm_dtile0 = (const uint64_t*)(db + L.msm_dtile0);
     const SegDesc* d_segs = (const SegDesc*)(db + L.segs);
     // seg_lane0 and part_T: the host plan's values, rewritten on the device
@@ -710,6 +722,10 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     const uint64_t nrec = 2 * pl.parts[P - 1].lane_hi;
     const bool norm = nmsm > kHostNormMsms;  // device tail: normalise there too
     uint8_t* hw = ws.hw;
+    // err[0]: decomposition error flag; err[1..4]: the merge's list counts;
+    // from 32 bytes on the segments' valid-entry counts
+    const CallBack back{d_err, (const uint32_t*)ws.segvalid, nseg,
+                        ws.mapped ? (uint32_t*)(hw + back_bytes) : nullptr};
     // The device part of the call.  Stream A (the engine stream): descriptors,
     // decomposition, then the accumulation of each part, one merge of every
     // part's records, the bucket reduction and the device tail; stream S: the
@@ -722,8 +738,12 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         auto rec = [&](hipEvent_t e, hipStream_t s) -> hipError_t { return events ? hipEventRecord(e, s) : hipSuccess; };
         // one part: everything on stream A (no cross-stream waits)
         hipStream_t S = P > 1 ? stream_sort_ : st;
-        ZK_TRY(hipMemcpyAsync(ws.desc, ws.hdesc, L.total, hipMemcpyHostToDevice, st));
-        launch_fill_zero(ws.err, z.err, st);
+        if (ws.mapped) {
+            launch_prologue(ws.hdesc, ws.desc, L.total, ws.err, z.err, ws.buckets, P == 1 ? pl.buckets * ptb : 0, st);
+        } else {
+            ZK_TRY(hipMemcpyAsync(ws.desc, ws.hdesc, L.total, hipMemcpyHostToDevice, st));
+            launch_fill_zero(ws.err, z.err, st);
+        }
         ZK_TRY(rec(ev_[0], st));
         // the decomposition also counts the first sort pass's tile histograms
         launch_decompose(pl.curve, d_msms, d_msm_dtile0, nmsm, pl.dtiles, d_segs, d_scalars, d_table, table_n,
@@ -733,7 +753,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             ZK_TRY(hipEventRecord(dep_fork_, st));
             ZK_TRY(hipStreamWaitEvent(S, dep_fork_, 0));
         }
-        launch_fill_zero(ws.buckets, pl.buckets * ptb, st);
+        if (P > 1 || !ws.mapped) launch_fill_zero(ws.buckets, pl.buckets * ptb, st);
         for (uint32_t p = 0; p < P; p++) {
             const PlanPart& pt = pl.parts[p];
             const uint32_t ns_p = pt.seg_hi - pt.seg_lo;
@@ -745,14 +765,15 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
                 launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
                                  d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.digits, nullptr, 0,
                                  (uint32_t*)ws.hist, (uint32_t*)ws.part, (uint32_t*)ws.segvalid,
-                                 (uint16_t*)ws.keysA, (uint32_t*)ws.valsA, S, pt.max_tiles, false);
+                                 (uint16_t*)ws.keysA, (uint32_t*)ws.valsA, S, pt.scan_seg, false);
                 launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
                                  d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.keysA,
                                  (const uint32_t*)ws.valsA, 1, (uint32_t*)ws.hist, (uint32_t*)ws.part,
-                                 (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB, (uint32_t*)ws.valsB, S, pt.max_tiles);
+                                 (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB, (uint32_t*)ws.valsB, S, pt.scan_seg);
             }
-            launch_lane_plan(d_segs, (const uint32_t*)ws.segvalid, pt.seg_lo, ns_p, pt.lane_lo, pt.lane_hi,
-                             d_seg_lane0, d_part_T + p, S);
+            if (ns_p > kPlanSegs)
+                launch_lane_plan(d_segs, (const uint32_t*)ws.segvalid, pt.seg_lo, ns_p, pt.lane_lo, pt.lane_hi,
+                                 d_seg_lane0, d_part_T + p, S);
             ZK_TRY(rec(ev_s1_[p], S));
             if (P > 1) ZK_TRY(hipEventRecord(dep_sort_[p], S));
         }
@@ -762,8 +783,8 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             ZK_TRY(rec(ev_a0_[p], st));
             launch_accumulate(pl.curve, d_segs, d_seg_lane0, pt.seg_lo, pt.seg_hi - pt.seg_lo, d_msms,
                               (const uint32_t*)ws.segvalid, (const uint16_t*)ws.keysB, (const uint32_t*)ws.valsB,
-                              d_table, d_part_T + p, pt.lane_lo, pt.lane_hi, ws.buckets, (uint32_t*)ws.recAk,
-                              ws.recAp, st);
+                              d_table, pt.seg_hi - pt.seg_lo > kPlanSegs ? d_part_T + p : nullptr, pt.nbk, pt.lane_lo,
+                              pt.lane_hi, ws.buckets, (uint32_t*)ws.recAk, ws.recAp, st);
             ZK_TRY(rec(ev_a1_[p], st));
         }
         // bucket partials that crossed lane boundaries, every part's at once
@@ -779,16 +800,18 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         // (its waves need as many registers as the accumulation's) and
         // measured slower
         ZK_TRY(rec(ev_r0_[0], st));
+        const bool bits_end = !dev_tail && pl.curve != CurveId::Bn254G2;  // the planes go to the host
         launch_bucket_reduce(pl.curve, d_segs, d_seg_rcb0, d_seg_grp0, nseg, pl.rc_blocks, pl.G, pl.reduce_lanes,
-                             ws.buckets, ws.rc, ws.bits, !dev_tail, st);
+                             ws.buckets, ws.rc, ws.bits, bits_end, bits_end ? back : CallBack{}, st);
+        if (pl.curve == CurveId::Bn254G2) launch_g2_windows(d_segs, d_msms, nseg, ws.bits, hw, back, st);
         ZK_TRY(rec(ev_r1_[0], st));
         if (dev_tail) {
-            launch_tail(pl.curve, d_segs, d_msms, nseg, nmsm, ws.bits, ws.wins, ws.res, norm, st);
+            launch_tail(pl.curve, d_segs, d_msms, nseg, nmsm, ws.bits, ws.wins, ws.res, norm, back, st);
             ZK_TRY(rec(ev_tail_, st));
         }
         ZK_TRY(rec(ev_[kStCopyOut], st));
+        if (ws.mapped) return kOk;
         ZK_TRY(hipMemcpyAsync(hw, dev_tail ? ws.res : ws.bits, back_bytes, hipMemcpyDeviceToHost, st));
-        // err[0]: decomposition error flag; err[1..4]: the merge's list counts
         ZK_TRY(hipMemcpyAsync(hw + back_bytes, ws.err, 4 * 5, hipMemcpyDeviceToHost, st));
         ZK_TRY(hipMemcpyAsync(hw + back_bytes + z.err, ws.segvalid, (uint64_t)nseg * 4,
                               hipMemcpyDeviceToHost, st));
@@ -898,7 +921,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     else if (dev_tail && pl.curve == CurveId::Grumpkin) HostG1<zkh::HR>::finish_sums(hw, nmsm, out96);
     else if (dev_tail) HostG1<zkh::HP>::finish_sums(hw, nmsm, out96);
     else if (pl.curve == CurveId::Grumpkin) host_tail<HostG1<zkh::HR>>(pl, hw, out96);
-    else if (pl.curve == CurveId::Bn254G2) host_tail<HostG2View>(pl, hw, out96);
+    else if (pl.curve == CurveId::Bn254G2) host_tail<HostG2View>(pl, hw, out96, true);
     else host_tail<HostG1<zkh::HP>>(pl, hw, out96);
     auto t_end = std::chrono::steady_clock::now();
     timing_.host_tail_ms = std::chrono::duration<float, std::milli>(t_end - t_tail0).count();
@@ -1335,8 +1358,8 @@ int32_t Engine::ensure_gtab_g2() {
         if (G::is_id(pts[i])) continue;
         const zkh::Fp2 dinv = G::mul2(acc, pre[i]);
         acc = G::mul2(acc, G::mul2(pts[i].ZZ, pts[i].ZZZ));
-        const zkh::Fp2 x = G::mul2(pts[i].X, G::mul2(dinv, pts[i].ZZZ));
-        const zkh::Fp2 y = G::mul2(pts[i].Y, G::mul2(dinv, pts[i].ZZ));
+        const zkh::Fp2 x = G::canon2(G::mul2(pts[i].X, G::mul2(dinv, pts[i].ZZZ)));
+        const zkh::Fp2 y = G::canon2(G::mul2(pts[i].Y, G::mul2(dinv, pts[i].ZZ)));
         const zkh::Fp* c[4] = {&x.c0, &x.c1, &y.c0, &y.c1};
         for (int k = 0; k < 4; k++) memcpy(&blob[i * 128 + 32 * k], c[k]->v, 32);
     }

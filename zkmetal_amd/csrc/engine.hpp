@@ -80,6 +80,8 @@ struct PlanPart {
     uint32_t seg_lo, seg_hi, tile_lo, tile_hi, chunk_lo, chunk_hi;
     uint32_t T;  // entries per accumulation lane in this part
     uint32_t max_tiles;  // sort tiles of its longest segment
+    uint32_t nbk;        // buckets of all its segments
+    bool scan_seg;       // histograms scanned by a block per segment
     uint64_t lane_lo, lane_hi, entries;
 };
 
@@ -114,6 +116,9 @@ struct Workspace {
     void *err = nullptr, *wins = nullptr, *res = nullptr;
     uint8_t* hdesc = nullptr;  // host: descriptors before upload
     uint8_t* hw = nullptr;     // host: copy-back area
+    // hdesc and hw are pinned, and bits (host tail) or res point into hw: the
+    // kernels read and write them, no copies
+    bool mapped = false;
 };
 
 // bytes of each buffer of a planned call; device = all device buffers, each
@@ -372,7 +377,7 @@ class Engine {
 
     DevBuf desc_, digits_, keysA_, valsA_, keysB_, valsB_, hist_, part_, segvalid_, buckets_;
     DevBuf recAk_, recAp_, lists_, rc_, winsum_, err_;  // lists_: the merge's run lists
-    DevBuf wins_, res_;  // device tail: window sums, results
+    DevBuf wins_;  // device tail: window sums
     DevBuf pts_in_, ptable_, scalars_, srs_, gtab_, gtab_gk_, gtab_g2_, tmp_;
     HostBuf hdesc_, hwin_;
     uint32_t srs_n_ = 0;

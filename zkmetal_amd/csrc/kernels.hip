@@ -811,6 +811,18 @@ __global__ __launch_bounds__(256) void k_fill_zero(uint4* __restrict__ p, uint64
     for (; i < n16; i += stride) p[i] = make_uint4(0, 0, 0, 0);
 }
 
+// The start of a call in one launch: the descriptors from the pinned host
+// image, the error flag and counters, and (one part) the buckets.  A copy and
+// two fills take three launches and the copy engine's latency.
+__global__ __launch_bounds__(256) void k_prologue(const uint4* __restrict__ hdesc, uint4* __restrict__ desc,
+                                                  uint64_t ndesc, uint4* __restrict__ err, uint64_t nerr,
+                                                  uint4* __restrict__ buckets, uint64_t nbuckets) {
+    const uint64_t i0 = (uint64_t)blockIdx.x * 256 + threadIdx.x, stride = (uint64_t)gridDim.x * 256;
+    for (uint64_t i = i0; i < ndesc; i += stride) desc[i] = hdesc[i];
+    for (uint64_t i = i0; i < nerr; i += stride) err[i] = make_uint4(0, 0, 0, 0);
+    for (uint64_t i = i0; i < nbuckets; i += stride) buckets[i] = make_uint4(0, 0, 0, 0);
+}
+
 // --------------------------------------------------- bucket accumulation
 // Lane L of segment s (l = L - seg_lane0[s]; T and seg_lane0 as k_lane_plan
 // set them for the part) owns sorted entries [ent0 + l*T, ent0 + (l+1)*T)
@@ -835,6 +847,14 @@ __device__ __forceinline__ void put_record(uint32_t* keys, uint4* pts, uint64_t 
 // are all busy again, and seg_lane0[s] = lane_lo + sum over the earlier
 // segments of ceil(valid / T) (at most lanes in all: each segment rounds up
 // by less than one lane).  One workgroup; T goes to *Tout for k_accumulate.
+// (A part of up to kPlanSegs segments is planned by the accumulation's blocks
+// themselves, each for itself: a microsecond there against a launch here.)
+__device__ __forceinline__ uint32_t lane_entries(uint32_t valid, uint32_t nbk, uint64_t lanes, uint32_t nseg) {
+    const uint64_t cap = lanes > nseg ? lanes - nseg : 1;
+    const uint32_t T = max(4u, min(32u, valid / (2u * max(nbk, 1u))));
+    return max(T, (uint32_t)((valid + cap - 1) / cap));
+}
+
 __global__ __launch_bounds__(256) void k_lane_plan(const SegDesc* __restrict__ segs,
                                                    const uint32_t* __restrict__ seg_valid, uint32_t seg_lo,
                                                    uint32_t nseg, uint64_t lane_lo, uint64_t lanes,
@@ -848,9 +868,7 @@ __global__ __launch_bounds__(256) void k_lane_plan(const SegDesc* __restrict__ s
     uint32_t V, B;
     (void)block_exclusive_scan(v, lds4, &V);
     (void)block_exclusive_scan(b, lds4, &B);
-    const uint64_t cap = lanes > nseg ? lanes - nseg : 1;
-    uint32_t T = max(4u, min(32u, V / (2u * max(B, 1u))));
-    T = max(T, (uint32_t)((V + cap - 1) / cap));
+    const uint32_t T = lane_entries(V, B, lanes, nseg);
     if (threadIdx.x == 0) *Tout = T;
     uint64_t carry = 0;
     for (uint32_t base = 0; base < nseg; base += 256) {
@@ -868,14 +886,36 @@ __global__ __launch_bounds__(256) void k_accumulate(
     const SegDesc* __restrict__ segs, const uint64_t* __restrict__ seg_lane0, uint32_t seg_lo, uint32_t nseg,
     const MsmDesc* __restrict__ msms, const uint32_t* __restrict__ seg_valid,
     const uint16_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-    const uint4* __restrict__ table, const uint32_t* __restrict__ Tp, uint64_t lane_lo, uint64_t lane_hi,
-    uint4* __restrict__ buckets, uint32_t* __restrict__ rec_keys, uint4* __restrict__ rec_pts) {
+    const uint4* __restrict__ table, const uint32_t* __restrict__ Tp, uint32_t nbk, uint64_t lane_lo,
+    uint64_t lane_hi, uint4* __restrict__ buckets, uint32_t* __restrict__ rec_keys, uint4* __restrict__ rec_pts) {
     const uint64_t L = lane_lo + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t T, s;  // entries per lane in this part; this lane's segment
+    uint64_t l;     // its index in the segment
+    if (Tp) {       // planned by k_lane_plan
+        T = *Tp;
+        s = seg_lo + upper_index(seg_lane0 + seg_lo, nseg, L);
+        l = L - seg_lane0[s];
+    } else {
+        __shared__ uint32_t lane0[kPlanSegs], lds4[4];
+        const uint32_t t = threadIdx.x, v = t < nseg ? seg_valid[seg_lo + t] : 0u;
+        uint32_t V, n;
+        (void)block_exclusive_scan(v, lds4, &V);
+        T = lane_entries(V, nbk, lane_hi - lane_lo, nseg);
+        const uint32_t ex = block_exclusive_scan((v + T - 1) / T, lds4, &n);
+        if (t < nseg) lane0[t] = ex;
+        __syncthreads();
+        const uint32_t x = (uint32_t)(L - lane_lo);
+        uint32_t lo = 0, hi = nseg;  // largest lo with lane0[lo] <= x
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (lane0[mid] <= x) lo = mid;
+            else hi = mid;
+        }
+        s = seg_lo + lo;
+        l = x - lane0[lo];
+    }
     if (L >= lane_hi) return;
-    const uint32_t T = *Tp;  // k_lane_plan's entries per lane for this part
-    const uint32_t s = seg_lo + upper_index(seg_lane0 + seg_lo, nseg, L);
     const SegDesc sg = segs[s];
-    const uint64_t l = L - seg_lane0[s];
     const uint64_t segend = sg.ent0 + seg_valid[s];
     const uint64_t b = sg.ent0 + l * T;
     const uint64_t e = min(b + T, segend);
@@ -1354,12 +1394,12 @@ void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const
                       uint32_t tile_lo, uint32_t ntiles, const uint32_t* chunk_seg, uint32_t chunk_lo,
                       uint32_t nchunks, const void* in_keys, const uint32_t* in_vals, int pass,
                       uint32_t* hist, uint32_t* part, uint32_t* seg_valid, uint16_t* out_keys,
-                      uint32_t* out_vals, hipStream_t st, uint32_t max_tiles, bool count) {
+                      uint32_t* out_vals, hipStream_t st, bool scan_seg, bool count) {
     if (!ntiles) return;
     if (count)  // else the tile histograms are already in hist
         hipLaunchKernelGGL(k_sort_hist, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
                            in_keys, pass, (const uint32_t*)seg_valid, hist);
-    if (max_tiles <= kScanSegTiles) {
+    if (scan_seg) {
         hipLaunchKernelGGL(k_scan_seg, dim3(nseg), dim3(1024), 0, st, segs, seg_lo, hist, pass, seg_valid);
     } else {
         hipLaunchKernelGGL(k_scan_up, dim3(nchunks), dim3(256), 0, st, segs, chunk_seg, chunk_lo,
@@ -1378,6 +1418,14 @@ void launch_sort_small(const SegDesc* segs, uint32_t nseg, const void* digits, u
     if (!nseg) return;
     hipLaunchKernelGGL(k_sort_small, dim3(nseg), dim3(1024), 0, st, segs, (const uint32_t*)digits, seg_valid,
                        out_keys, out_vals);
+}
+
+void launch_prologue(const void* hdesc, void* desc, uint64_t desc_bytes, void* err, uint64_t err_bytes,
+                     void* buckets, uint64_t bucket_bytes, hipStream_t st) {
+    const uint64_t n = std::max(desc_bytes, bucket_bytes) / 16;
+    const unsigned blocks = (unsigned)std::min<uint64_t>(std::max<uint64_t>(blocks_for(n, 256), 1), 16384);
+    hipLaunchKernelGGL(k_prologue, dim3(blocks), dim3(256), 0, st, (const uint4*)hdesc, (uint4*)desc,
+                       desc_bytes / 16, (uint4*)err, err_bytes / 16, (uint4*)buckets, bucket_bytes / 16);
 }
 
 void launch_fill_zero(void* p, uint64_t bytes, hipStream_t st) {
@@ -1409,13 +1457,13 @@ void launch_lane_plan(const SegDesc* segs, const uint32_t* seg_valid, uint32_t s
 
 void launch_accumulate(CurveId cv, const SegDesc* segs, const uint64_t* seg_lane0, uint32_t seg_lo,
                        uint32_t nseg, const MsmDesc* msms, const uint32_t* seg_valid, const uint16_t* keys,
-                       const uint32_t* vals, const void* table, const uint32_t* T, uint64_t lane_lo,
+                       const uint32_t* vals, const void* table, const uint32_t* T, uint32_t nbk, uint64_t lane_lo,
                        uint64_t lane_hi, void* buckets, uint32_t* rec_keys, void* rec_pts, hipStream_t st) {
     if (lane_hi <= lane_lo) return;
 #define ZK_ACC(C)                                                                                  \
     hipLaunchKernelGGL(k_accumulate<C>, dim3(blocks_for(lane_hi - lane_lo, 256)), dim3(256), 0, st, \
                        segs, seg_lane0, seg_lo, nseg, msms, seg_valid, keys, vals, (const uint4*)table, \
-                       T, lane_lo, lane_hi, (uint4*)buckets, rec_keys, (uint4*)rec_pts)
+                       T, nbk, lane_lo, lane_hi, (uint4*)buckets, rec_keys, (uint4*)rec_pts)
     if (cv == CurveId::Grumpkin) ZK_ACC(G1Curve<Bn254Fr>);
     else if (cv == CurveId::Bn254G2) ZK_ACC(G2Curve);
     else ZK_ACC(G1Curve<Bn254Fp>);

@@ -105,8 +105,14 @@ constexpr int kSortItems = 8;
 constexpr int kSortTile = kSortThreads * kSortItems;
 // one-block sort of a whole segment (k_sort_small): entries and buckets at most
 constexpr uint32_t kSmallSortLen = 16384, kSmallSortBuckets = 4096;
-// tiles of a segment up to which one block scans its histogram (k_scan_seg)
-constexpr uint32_t kScanSegTiles = 256;
+// segments of a part up to which k_accumulate plans its lanes itself (one per
+// thread of a block)
+constexpr uint32_t kPlanSegs = 256;
+// tiles of a segment up to which one block scans its histogram (k_scan_seg),
+// in calls of one part: 1.2 us per 64 tiles against 13 us of three launches.
+// Beside an accumulation its 1024 threads find no room on any CU, and the
+// part's sort waits the accumulation out (G2 at 2^20 points: 1.7 ms).
+constexpr uint32_t kScanSegTiles = 128;
 constexpr int kScanChunk = 4096;  // histogram counts per scan block (16 per thread)
 
 }  // namespace zk

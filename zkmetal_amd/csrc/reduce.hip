@@ -20,6 +20,13 @@
 
 namespace zk {
 
+// the call's last kernel, block 0: err and counts to pinned host memory
+__device__ __forceinline__ void write_back(const CallBack& b) {
+    if (blockIdx.x != 0 || !b.out) return;
+    if (threadIdx.x < 5) b.out[threadIdx.x] = b.err[threadIdx.x];
+    for (uint32_t i = threadIdx.x; i < b.nseg; i += blockDim.x) b.out[8 + i] = b.seg_valid[i];
+}
+
 // sum over aligned groups of P teams of a wave (P a power of two, uniform):
 // a butterfly, so every team ends with the group's total
 template <class T>
@@ -420,8 +427,9 @@ template <class T>
 __global__ __launch_bounds__(256) void k_br_bits(const SegDesc* __restrict__ segs,
                                                  const uint64_t* __restrict__ seg_rc0,
                                                  const uint4* __restrict__ rc, uint4* __restrict__ bits,
-                                                 int host_form) {
+                                                 int host_form, CallBack back) {
     __shared__ uint4 lds[4 * T::kPtBytes / 16];
+    write_back(back);
     const uint32_t s = blockIdx.x >> 4, j = blockIdx.x & 15u;
     const SegDesc sg = segs[s];
     uint32_t g, h;
@@ -473,7 +481,10 @@ template <class T>
 __global__ __launch_bounds__(16 * T::kLanes) void k_tail_windows(const SegDesc* __restrict__ segs,
                                                                 const MsmDesc* __restrict__ msms,
                                                                 const uint4* __restrict__ bits,
-                                                                uint4* __restrict__ wins) {
+                                                                uint4* __restrict__ wins, int host_form,
+                                                                CallBack back) {
+    __shared__ uint4 lds[4 * T::kPtBytes / 16];
+    write_back(back);
     const uint32_t s = blockIdx.x, t = threadIdx.x / T::kLanes;
     const uint32_t c = msms[segs[s].msm].c;
     const uint64_t b0 = (uint64_t)s * 16;
@@ -484,8 +495,10 @@ __global__ __launch_bounds__(16 * T::kLanes) void k_tail_windows(const SegDesc* 
     const uint32_t n = plane ? t : 0;
 #pragma unroll 1
     for (uint32_t i = 0; i < n; i++) v = T::dbl(v);
-    wave_tree<T>(v, 16);
-    if (t == 0) T::store(wins, s, v);
+    block_tree<T>(v, 16, lds);
+    if (t != 0) return;
+    if (host_form) T::store_host(wins, s, v);
+    else T::store(wins, s, v);
 }
 
 // one team per MSM: the MSM's sum in the host form (128 B) into out, or (norm)
@@ -495,7 +508,8 @@ __global__ __launch_bounds__(16 * T::kLanes) void k_tail_windows(const SegDesc* 
 template <class T>
 __global__ __launch_bounds__(64) void k_tail_combine(const MsmDesc* __restrict__ msms, uint32_t nmsm,
                                                      uint4* __restrict__ wins, uint4* __restrict__ out,
-                                                     int norm) {
+                                                     int norm, CallBack back) {
+    if (!norm) write_back(back);
     const uint32_t j = (blockIdx.x * 64 + threadIdx.x) / T::kLanes;
     if (j >= nmsm) return;
     const MsmDesc m = msms[j];
@@ -518,8 +532,9 @@ __global__ __launch_bounds__(64) void k_tail_combine(const MsmDesc* __restrict__
 template <class F>
 __global__ __launch_bounds__(64) void k_tail_normalise(const MsmDesc* __restrict__ msms, uint32_t nmsm,
                                                        const uint4* __restrict__ wins,
-                                                       uint4* __restrict__ out) {
+                                                       uint4* __restrict__ out, CallBack back) {
     using A = Arith<F>;
+    write_back(back);
     const uint32_t j = blockIdx.x * 64 + threadIdx.x;
     if (j >= nmsm) return;
     const QXyzz p = load_qxyzz(wins, msms[j].seg0);
@@ -624,7 +639,7 @@ void launch_merge_runs(CurveId cv, const uint32_t* keys, const void* pts, uint64
 template <class C>
 static void bucket_reduce_t(const SegDesc* segs, const uint64_t* seg_blk0, const uint64_t* seg_rc0,
                             uint32_t nseg, uint64_t blocks, uint32_t per, bool by_lanes, const void* buckets,
-                            void* rc, void* bits, bool host_form, hipStream_t st) {
+                            void* rc, void* bits, bool host_form, const CallBack& back, hipStream_t st) {
     using T = typename C::Team;
     if (by_lanes)
         hipLaunchKernelGGL(k_br_rowcol_lanes<C>, dim3((unsigned)blocks), dim3(256), 0, st, segs, seg_blk0, seg_rc0,
@@ -634,42 +649,49 @@ static void bucket_reduce_t(const SegDesc* segs, const uint64_t* seg_blk0, const
                            per, (const uint4*)buckets, (uint4*)rc);
     const uint32_t waves = nseg > 32 ? 1 : nseg > 16 ? 2 : 4;  // of one of ~1000 points
     hipLaunchKernelGGL(k_br_bits<T>, dim3(nseg * 16), dim3(64 * waves), 0, st, segs, seg_rc0, (const uint4*)rc,
-                       (uint4*)bits, host_form ? 1 : 0);
+                       (uint4*)bits, host_form ? 1 : 0, back);
 }
 
 void launch_bucket_reduce(CurveId cv, const SegDesc* segs, const uint64_t* seg_blk0, const uint64_t* seg_rc0,
                           uint32_t nseg, uint64_t blocks, uint32_t per, bool by_lanes, const void* buckets, void* rc,
-                          void* bits, bool host_form, hipStream_t st) {
+                          void* bits, bool host_form, const CallBack& back, hipStream_t st) {
     if (!blocks || !nseg) return;
     if (cv == CurveId::Grumpkin)
         bucket_reduce_t<LaneG1<Bn254Fr>>(segs, seg_blk0, seg_rc0, nseg, blocks, per, by_lanes, buckets, rc, bits,
-                                             host_form, st);
+                                             host_form, back, st);
     else if (cv == CurveId::Bn254G2)
         bucket_reduce_t<LaneG2>(segs, seg_blk0, seg_rc0, nseg, blocks, per, by_lanes, buckets, rc, bits, host_form,
-                                st);
+                                back, st);
     else
         bucket_reduce_t<LaneG1<Bn254Fp>>(segs, seg_blk0, seg_rc0, nseg, blocks, per, by_lanes, buckets, rc, bits,
-                                             host_form, st);
+                                             host_form, back, st);
 }
 
 template <class F>
 static void tail_t(const SegDesc* segs, const MsmDesc* msms, uint32_t nseg, uint32_t nmsm, const void* bits,
-                   void* wins, void* out, bool norm, hipStream_t st) {
+                   void* wins, void* out, bool norm, const CallBack& back, hipStream_t st) {
     using T = TeamG1<F>;
     hipLaunchKernelGGL(k_tail_windows<T>, dim3(nseg), dim3(16 * T::kLanes), 0, st, segs, msms, (const uint4*)bits,
-                       (uint4*)wins);
+                       (uint4*)wins, 0, CallBack{});
     hipLaunchKernelGGL(k_tail_combine<T>, dim3((nmsm + T::kPerWave - 1) / T::kPerWave), dim3(64), 0, st, msms, nmsm,
-                       (uint4*)wins, (uint4*)out, norm ? 1 : 0);
+                       (uint4*)wins, (uint4*)out, norm ? 1 : 0, back);
     if (norm)
         hipLaunchKernelGGL(k_tail_normalise<F>, dim3((nmsm + 63) / 64), dim3(64), 0, st, msms, nmsm,
-                           (const uint4*)wins, (uint4*)out);
+                           (const uint4*)wins, (uint4*)out, back);
 }
 
 void launch_tail(CurveId cv, const SegDesc* segs, const MsmDesc* msms, uint32_t nseg, uint32_t nmsm,
-                 const void* bits, void* wins, void* out, bool norm, hipStream_t st) {
+                 const void* bits, void* wins, void* out, bool norm, const CallBack& back, hipStream_t st) {
     if (!nseg || !nmsm) return;
-    if (cv == CurveId::Grumpkin) tail_t<Bn254Fr>(segs, msms, nseg, nmsm, bits, wins, out, norm, st);
-    else if (cv == CurveId::Bn254) tail_t<Bn254Fp>(segs, msms, nseg, nmsm, bits, wins, out, norm, st);
+    if (cv == CurveId::Grumpkin) tail_t<Bn254Fr>(segs, msms, nseg, nmsm, bits, wins, out, norm, back, st);
+    else if (cv == CurveId::Bn254) tail_t<Bn254Fp>(segs, msms, nseg, nmsm, bits, wins, out, norm, back, st);
+}
+
+void launch_g2_windows(const SegDesc* segs, const MsmDesc* msms, uint32_t nseg, const void* bits, void* out,
+                       const CallBack& back, hipStream_t st) {
+    if (!nseg) return;
+    hipLaunchKernelGGL(k_tail_windows<TeamG2>, dim3(nseg), dim3(16 * TeamG2::kLanes), 0, st, segs, msms,
+                       (const uint4*)bits, (uint4*)out, 1, back);
 }
 
 }  // namespace zk
