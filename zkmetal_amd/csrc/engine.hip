@@ -139,12 +139,12 @@ bool shifted_pays(uint64_t n, uint32_t c, uint32_t c_s) {
     return shifted < plain;
 }
 
-// A call of one MSM has a latency-bound reduction (about 0.16 ms from 2^16
-// to 2^22 points whatever its bucket count), and its shifted buckets are
-// deep enough to span several accumulation lanes, which costs merge work:
-// measured on MI355X, one shifted MSM takes 0.42 / 0.74 / 1.81 / 6.23 ms
-// against 0.61 / 0.65 / 1.71 / 6.05 ms plain at 2^16 / 2^18 / 2^20 / 2^22.
-constexpr uint64_t kShiftSingleMax = 1u << 17;
+// A single MSM's shifted buckets are deep enough to span several accumulation
+// lanes, which costs merge work where the reduction it saves no longer counts.
+// Measured on MI355X, one MSM shifted against plain: 2^16 points 290 / 425 us
+// (witness-like scalars 277 / 393), 2^18 586 / 594 (410 / 444), 2^19 883 / 894
+// (576 / 525), 2^20 1594 / 1671 (912 / 808).
+constexpr uint64_t kShiftSingleMax = 1u << 18;
 
 // Row and column sums by lanes from this many additions on (two per bucket),
 // by lane teams below: 2^16 of them make a wave of one-lane chains for every
@@ -634,9 +634,8 @@ WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
 
 int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, uint64_t table_n,
                     uint8_t* out96) {
-    const uint32_t nmsm = (uint32_t)pl.msms.size();
     // window combine on the device (graph mode, large batches) or the host
-    const bool dev_tail = device_tail(nmsm, pl.curve);
+    const bool dev_tail = device_tail(pl);
     const WsSizes z = ws_sizes(pl, dev_tail);
     ZK_ALLOC(desc_, z.desc);
     ZK_ALLOC(hdesc_, z.desc);
@@ -1081,8 +1080,8 @@ int32_t Engine::msm_batch_host(const uint8_t* points, const uint8_t* scalars,
         }
     }
     Plan pl;
-    rc = make_plan(ns.data(), t0.data(), (uint32_t)ns.size(), window_bits_for(ns, cv).data(), pl, 0,
-                   lane_cap(cv), cv, parts_req_, 0, 0, 0, schedule((uint32_t)ns.size()));
+    rc = plan_call(ns, t0, pl, 0, cv, 0,
+                   pts_in_.growth(total * input_point_bytes(cv)) + ptable_.growth(table_bytes(total, cv)));
     if (rc != kOk) return rc;
     ZK_ALLOC(pts_in_, total * input_point_bytes(cv));
     ZK_ALLOC(ptable_, table_bytes(total, cv));
@@ -1136,8 +1135,7 @@ int32_t Engine::msm_device(const void* d_points, const void* d_scalars, const ui
     ZK_ALLOC(ptable_, table_bytes(total, cv));
     launch_build_table(cv, d_points, ptable_.p, total, stream_);
     Plan& pl = plan_;
-    int rc = make_plan(ns.data(), t0.data(), (uint32_t)ns.size(), window_bits_for(ns, cv).data(), pl, 0,
-                       lane_cap(cv), cv, parts_req_, 0, 0, 0, schedule((uint32_t)ns.size()));
+    int rc = plan_call(ns, t0, pl, 0, cv, 0, 0);
     if (rc != kOk) return rc;
     std::vector<uint8_t> res(ns.size() * result_bytes(cv));
     rc = run(pl, d_scalars, ptable_.p, total, res.data());
@@ -1173,9 +1171,36 @@ int32_t Engine::srs_finish(uint64_t n, uint64_t stride) {
     return kOk;
 }
 
-uint32_t Engine::shift_floor(uint32_t nmsm) const {
+uint32_t Engine::shift_floor(const std::vector<uint32_t>& ns, bool lean) const {
     if (shift_mode_ == kShiftAll) return 1;
-    return device_tail(nmsm, CurveId::Bn254) ? kShiftDeviceTailFloor : 0;
+    const uint32_t nmsm = (uint32_t)ns.size();
+    const bool dev = tail_mode_ == kTailDevice ||
+                     (tail_mode_ == kTailAuto && (graph_mode_ == kGraphOn || nmsm >= kDeviceTailMinMsms));
+    if (lean || nmsm > kShiftAlwaysMsms) return dev ? kShiftDeviceTailFloor : 0;
+    if (nmsm == 1 && !dev && ns[0] > kShiftSingleMax) return 0;
+    return kShiftFloor;
+}
+
+// The call's plan: the tuned window widths and the shift rule; where a cap on
+// the engine's memory leaves no room for it, the widths and the rule that need
+// the fewest buckets (lean).  other: bytes the call will allocate besides.
+int32_t Engine::plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
+                          CurveId cv, uint64_t shift_stride, uint64_t other) {
+    const uint32_t nmsm = (uint32_t)ns.size();
+    auto make = [&](bool lean) {
+        return make_plan(ns.data(), t0.data(), nmsm, window_bits_for(ns, cv, lean).data(), pl, form, lane_cap(cv), cv,
+                         parts_req_, shift_stride, kShiftC, shift_floor(ns, lean), schedule(nmsm));
+    };
+    const int32_t rc = make(false);
+    if (rc != kOk || !ws_.limit) return rc;
+    const WsSizes z = ws_sizes(pl, device_tail(pl));
+    const uint64_t need = other + desc_.growth(z.desc) + digits_.growth(z.digits) + keysA_.growth(z.keys) +
+                          valsA_.growth(z.vals) + keysB_.growth(z.keys) + valsB_.growth(z.vals) +
+                          hist_.growth(z.hist) + part_.growth(z.part) + segvalid_.growth(z.segvalid) +
+                          buckets_.growth(z.buckets) + recAk_.growth(z.rec_keys) + recAp_.growth(z.rec_pts) +
+                          lists_.growth(z.lists) + rc_.growth(z.rc) + winsum_.growth(z.bits) +
+                          wins_.growth(z.wins) + err_.growth(z.err);
+    return ws_.used + need > ws_.limit ? make(true) : rc;
 }
 
 uint64_t Engine::plan_shift(const void* table, uint64_t shift_stride) const {
@@ -1488,9 +1513,8 @@ int32_t Engine::msm_table_parts(const void* table, uint32_t table_n,
     if (ns.empty()) return kOk;
     if (total >= (1ull << 30)) return kInvalidInput;
     Plan& pl = plan_;
-    int rc = make_plan(ns.data(), t0.data(), (uint32_t)ns.size(), window_bits_for(ns).data(), pl, form, acc_cap_,
-                       CurveId::Bn254, parts_req_, plan_shift(table, shift_stride), kShiftC,
-                       shift_floor((uint32_t)ns.size()), schedule((uint32_t)ns.size()));
+    int rc = plan_call(ns, t0, pl, form, CurveId::Bn254, plan_shift(table, shift_stride),
+                       host_parts ? scalars_.growth(total * 32) : 0);
     if (rc != kOk) return rc;
     const void* d_sc = d_scalars;
     if (host_parts) {
@@ -1511,21 +1535,28 @@ int32_t Engine::msm_table_parts(const void* table, uint32_t table_n,
     return kOk;
 }
 
-uint32_t Engine::window_bit(uint32_t n, bool batch, CurveId cv) const {
-    uint32_t c = c_override_;
-    if (!c && cv == CurveId::Bn254) {
-        uint32_t cls = 0;
-        while ((1ull << cls) < n) cls++;  // ceil(log2 n)
-        cls = std::min<uint32_t>(cls, 32);
-        if (batch) c = ctab_batch_[cls];
-        if (!c) c = ctab_[cls];
+uint32_t Engine::window_bit(uint32_t n, bool batch, CurveId cv, bool lean) const {
+    if (c_override_) return c_override_;
+    uint32_t cls = 0;
+    while ((1ull << cls) < n) cls++;  // ceil(log2 n)
+    cls = std::min<uint32_t>(cls, 32);
+    uint32_t c = 0;  // 0 = cost-model default
+    if (cv == CurveId::Bn254) {
+        // lean: the narrow widths in place of the tuned ones (not of a caller's)
+        auto entry = [&](const uint32_t* tab, const uint32_t* tuned, const uint32_t* narrow) {
+            return lean && tab[cls] == tuned[cls] ? narrow[cls] : tab[cls];
+        };
+        if (batch) c = entry(ctab_batch_, kTunedBatch, kLeanBatch);
+        if (!c) c = entry(ctab_, kTunedPlain, kLeanPlain);
+    } else if (!batch && !lean) {
+        c = (cv == CurveId::Grumpkin ? kTunedGrumpkin : kTunedG2)[cls];
     }
-    return c;  // 0 = cost-model default
+    return c;
 }
 
-std::vector<uint32_t> Engine::window_bits_for(const std::vector<uint32_t>& ns, CurveId cv) const {
+std::vector<uint32_t> Engine::window_bits_for(const std::vector<uint32_t>& ns, CurveId cv, bool lean) const {
     std::vector<uint32_t> cs(ns.size());
-    for (size_t j = 0; j < ns.size(); j++) cs[j] = window_bit(ns[j], ns.size() > 1, cv);
+    for (size_t j = 0; j < ns.size(); j++) cs[j] = window_bit(ns[j], ns.size() > 1, cv, lean);
     return cs;
 }
 
@@ -1624,32 +1655,41 @@ int32_t Engine::msm_resident_noalloc(const void* d_scalars, const uint32_t* coun
     for (uint32_t j = 0; j < nmsm; j++)
         if (counts[j] == 0) memset(out96 + (uint64_t)j * 96, 0, 96);
     if (k == 0) return kOk;
-    // the plan's array sizes, before planning: within the reserved capacity
-    uint64_t nseg = 0, tiles = 0, chunks = 0;
-    for (uint32_t i = 0; i < k; i++) {
-        cs[i] = window_bit(ns[i], k > 1, CurveId::Bn254);
-        const uint32_t c = cs[i] ? cs[i] : default_window_bits(ns[i]);
-        if (c < 2 || c > 16) return kInvalidInput;
-        const uint64_t w = (128 + c - 1) / c, nt = (2ull * ns[i] + kSortTile - 1) / kSortTile;
-        nseg += w;
-        tiles += w * nt;
-        chunks += w * ((256 * nt + kScanChunk - 1) / kScanChunk);
-    }
-    if (nseg > na_plan_.segs.capacity() || tiles > na_plan_.tile_seg.capacity() ||
-        chunks > na_plan_.chunk_seg.capacity())
-        return kInvalidInput;
-    // at most 2^15 accumulation lanes: a quarter of the device's resident
-    // lanes, ample for <= 2^16 points, and it bounds the merge records (two
-    // per lane), the largest buffer of a small call
-    int rc = make_plan(ns, t0, k, cs, na_plan_, 0, std::min<uint64_t>(acc_cap_, 1u << 15), CurveId::Bn254, 0,
-                       plan_shift(srs_.p, kOwnTable), kShiftC, shift_mode_ == kShiftAll ? 1u : 0u);
-    if (rc != kOk) return rc;
     const Plan& pl = na_plan_;
-    const WsSizes z = ws_sizes(pl, true);
-    const uint64_t desc_host = (z.desc + 255) & ~uint64_t(255);
     const uint64_t res_host = (uint64_t)k * 96;
-    if (z.device > kNoAllocScratchBytes || desc_host + z.host + res_host > na_host_.capacity())
-        return kInvalidInput;  // the call needs more than the array holds
+    WsSizes z{};
+    uint64_t desc_host = 0;
+    auto plan = [&](bool lean) -> int32_t {
+        // the plan's array sizes, before planning: within the reserved capacity
+        uint64_t nseg = 0, tiles = 0, chunks = 0;
+        for (uint32_t i = 0; i < k; i++) {
+            cs[i] = window_bit(ns[i], k > 1, CurveId::Bn254, lean);
+            const uint32_t c = cs[i] ? cs[i] : default_window_bits(ns[i]);
+            if (c < 2 || c > 16) return kInvalidInput;
+            const uint64_t w = (128 + c - 1) / c, nt = (2ull * ns[i] + kSortTile - 1) / kSortTile;
+            nseg += w;
+            tiles += w * nt;
+            chunks += w * ((256 * nt + kScanChunk - 1) / kScanChunk);
+        }
+        if (nseg > na_plan_.segs.capacity() || tiles > na_plan_.tile_seg.capacity() ||
+            chunks > na_plan_.chunk_seg.capacity())
+            return kInvalidInput;
+        // at most 2^15 accumulation lanes: a quarter of the device's resident
+        // lanes, ample for <= 2^16 points, and it bounds the merge records (two
+        // per lane), the largest buffer of a small call
+        const int32_t rc = make_plan(ns, t0, k, cs, na_plan_, 0, std::min<uint64_t>(acc_cap_, 1u << 15),
+                                     CurveId::Bn254, 0, plan_shift(srs_.p, kOwnTable), kShiftC,
+                                     shift_mode_ == kShiftAll ? 1u : 0u);
+        if (rc != kOk) return rc;
+        z = ws_sizes(pl, true);
+        desc_host = (z.desc + 255) & ~uint64_t(255);
+        // else the call needs more than the array holds
+        return z.device > kNoAllocScratchBytes || desc_host + z.host + res_host > na_host_.capacity() ? kInvalidInput
+                                                                                                      : kOk;
+    };
+    int32_t rc = plan(false);
+    if (rc != kOk) rc = plan(true);
+    if (rc != kOk) return rc;
     // carve the call's buffers out of the array, 256-byte aligned, in the
     // order ws_sizes counts them
     uint64_t off = 0;

@@ -39,6 +39,8 @@ struct DevBuf {
     size_t cap = 0;
     WsAccount* acct = nullptr;
     hipError_t ensure(size_t bytes);
+    // bytes that ensure(bytes) would add to the account
+    uint64_t growth(uint64_t bytes) const { return bytes > cap ? std::max<uint64_t>(bytes, 256) - cap : 0; }
     void release();
     ~DevBuf() { release(); }
 };
@@ -271,8 +273,8 @@ class Engine {
     // per-MSM window widths: the override, else the tuned tables (BN254 G1
     // only), else 0 = the cost model
     std::vector<uint32_t> window_bits_for(const std::vector<uint32_t>& ns,
-                                          CurveId cv = CurveId::Bn254) const;
-    uint32_t window_bit(uint32_t n, bool batch, CurveId cv) const;
+                                          CurveId cv = CurveId::Bn254, bool lean = false) const;
+    uint32_t window_bit(uint32_t n, bool batch, CurveId cv, bool lean = false) const;
 
     void set_window_bits(uint32_t c) { c_override_ = c; }
     // cap on the device memory this engine's buffers may grow to (resident
@@ -294,14 +296,21 @@ class Engine {
     // overlap (0: by size); a measurement knob, results are the same
     void set_parts(uint32_t p) { parts_req_ = std::min<uint32_t>(p, kMaxParts); }
     // where a call's window combine and normalisation run: kTailAuto (the
-    // device in graph mode and for calls of at least kDeviceTailMinMsms MSMs,
+    // device in graph mode, for calls of at least kDeviceTailMinMsms MSMs and
+    // for calls of at least kDeviceTailMinPlain that are not window-shifted,
     // else the host), kTailHost, kTailDevice.  BN254 G2 always uses the host.
+    // A plain MSM's combine takes the host 40 us (127 doublings, as many
+    // additions), the device about 260 whatever the number of MSMs (8 MSMs of
+    // 64 points: 489 us by the host, 438 by the device); a shifted one has 15
+    // doublings: 5 us against 47.
     enum TailMode : int32_t { kTailAuto = 0, kTailHost = 1, kTailDevice = 2 };
-    static constexpr uint32_t kDeviceTailMinMsms = 16;
-    bool device_tail(uint32_t nmsm, CurveId cv) const {
-        return cv != CurveId::Bn254G2 &&
-               (tail_mode_ == kTailDevice ||
-                (tail_mode_ == kTailAuto && (graph_mode_ == kGraphOn || nmsm >= kDeviceTailMinMsms)));
+    static constexpr uint32_t kDeviceTailMinMsms = 16, kDeviceTailMinPlain = 8;
+    bool device_tail(const Plan& pl) const {
+        if (pl.curve == CurveId::Bn254G2 || tail_mode_ != kTailAuto)
+            return pl.curve != CurveId::Bn254G2 && tail_mode_ == kTailDevice;
+        uint32_t plain = 0;
+        for (const MsmDesc& m : pl.msms) plain += m.cstep != 0;
+        return graph_mode_ == kGraphOn || pl.msms.size() >= kDeviceTailMinMsms || plain >= kDeviceTailMinPlain;
     }
     int32_t set_tail_mode(int32_t m) {
         if (m < kTailAuto || m > kTailDevice) return kInvalidInput;
@@ -390,12 +399,20 @@ class Engine {
     // after the table's bases are written: the shifted copies, then wait
     int32_t srs_finish(uint64_t n, uint64_t stride);
     uint64_t plan_shift(const void* table, uint64_t shift_stride) const;
-    // make_plan's shift_floor for a call of nmsm MSMs: every MSM in kShiftAll
+    int32_t plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
+                      CurveId cv, uint64_t shift_stride, uint64_t other);
+    // make_plan's shift_floor for a call: in calls of up to kShiftAlwaysMsms
+    // MSMs every MSM of at least kShiftFloor points (a single one up to
+    // kShiftSingleMax): below that a plain reduction of narrow windows is as
+    // quick (one MSM of 256 / 512 / 2048 points 187 / 184 / 175 us shifted,
+    // 172 / 195 / 246 plain; 64 of 512 752 / 916), and beyond so many MSMs
+    // their 2^15 buckets each no longer fill idle lanes but cost time, and the
+    // estimate (shifted_pays) decides.  Otherwise: every MSM in kShiftAll
     // mode; in a call whose window combine runs on the device, every MSM of
     // at least kShiftDeviceTailFloor points (a plain MSM's serial doubling
     // chain would set the combine's latency)
-    static constexpr uint32_t kShiftDeviceTailFloor = 4096;
-    uint32_t shift_floor(uint32_t nmsm) const;
+    static constexpr uint32_t kShiftDeviceTailFloor = 4096, kShiftFloor = 512, kShiftAlwaysMsms = 64;
+    uint32_t shift_floor(const std::vector<uint32_t>& ns, bool lean) const;
     // host image of the resident bases (64 B each) for the prefix check:
     // srs_first_ is filled whenever an SRS is set, srs_host_ on the first
     // call whose first base matches it

@@ -16,10 +16,26 @@
 
 namespace zk {
 
-static const uint32_t kTunedPlain[33] = {0, 0, 0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 10, 10, 10, 12, 15,
-                                         15, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-static const uint32_t kTunedBatch[33] = {0, 0, 0, 0, 0, 0, 0, 0, 6, 7, 8, 8, 9, 10, 11, 12, 13,
+// Widths that divide the 128 bits without a narrow top window (8, 13 with an
+// 11-bit top, 16) win: a narrow one piles its entries into few buckets, whose
+// partials the merge then adds up.  Against the widths between (us): 2^11
+// points 214 at 13 bits, 254 at 8; 2^14 291 at 16, 399 at 10; 2^16 358 at 16,
+// 420 at 15.
+static const uint32_t kTunedPlain[33] = {0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 8, 13, 13, 13, 16, 16, 16,
+                                         16, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+static const uint32_t kTunedBatch[33] = {0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 8, 8, 9, 10, 11, 13, 13,
                                          13, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+// The narrow widths for a call that a memory cap, or the no-allocation
+// array, leaves no room for the tuned ones (a fraction of their buckets).
+static const uint32_t kLeanPlain[33] = {0, 0, 0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 10, 10, 10, 12, 15,
+                                        15, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+static const uint32_t kLeanBatch[33] = {0, 0, 0, 0, 0, 0, 0, 0, 6, 7, 8, 8, 9, 10, 11, 12, 13,
+                                        13, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+// single MSMs on Grumpkin and BN254 G2 (255-bit scalars, no GLV)
+static const uint32_t kTunedGrumpkin[33] = {0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 10, 11, 12, 10, 10, 11, 15,
+                                            15, 16, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+static const uint32_t kTunedG2[33] = {0, 0, 0, 0, 0, 0, 8, 8, 8, 8, 10, 9, 10, 12, 12, 12, 12,
+                                      12, 13, 16, 16, 16, 16, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
 // Small calls leave most of the chip idle, so a shorter chain before the tree
 // wins: with 4 against 8 buckets, 256 points 255 against 263 us, 4097 points
