@@ -1,6 +1,7 @@
 """The sort's routes at their edges against the closed form: a segment just
 within and just past the one-block sort (16384 entries, 4096 buckets), and
 segments on either side of the one-block histogram scan (128 tiles)."""
+import numpy as np
 import pytest
 
 import zkmetal_amd as zk
@@ -47,3 +48,23 @@ def test_one_block_scan_edges(eng, n):
             _check(eng, n, 1)
         finally:
             eng.set_pipeline_parts(0)
+
+
+@pytest.mark.parametrize("n", [8193, 12320, 40000])
+@pytest.mark.parametrize("odd", [None, 63, 64, 8192])
+def test_second_pass_with_one_low_byte(eng, n, odd):
+    # keys that differ in their high bytes only (ranked without matching), and
+    # the same with one entry of another low byte (matched) at a wave's edge
+    rng = np.random.default_rng(SEED + n)
+    k = 1 + 256 * rng.integers(0, 120, n, dtype=np.uint64)
+    if odd is not None:
+        k[odd] += 77
+    sc = np.zeros((n, 4), np.uint64)
+    sc[:, 0] = k
+    sc = sc.reshape(-1).view(np.uint8)
+    eng.set_window_bits(16)
+    try:
+        got = result_affine(eng.msm_batch_resident(sc, [n])[0])
+    finally:
+        eng.set_window_bits(0)
+    assert got == B.mul(B.G, ref.scalar_dot(sc.tobytes(), zk.gen_scalars(SEED, n, 0).tobytes(), n))

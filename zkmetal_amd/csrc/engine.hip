@@ -764,7 +764,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
                 launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
                                  d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.digits, nullptr, 0,
                                  (uint32_t*)ws.hist, (uint32_t*)ws.part, (uint32_t*)ws.segvalid,
-                                 (uint16_t*)ws.keysA, (uint32_t*)ws.valsA, S, pt.scan_seg, false);
+                                 (uint16_t*)ws.keysA, (uint32_t*)ws.valsA, S, pt.scan_seg);
                 launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
                                  d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.keysA,
                                  (const uint32_t*)ws.valsA, 1, (uint32_t*)ws.hist, (uint32_t*)ws.part,

@@ -40,14 +40,21 @@ using Ar = Arith<Bn254Fr>;
 __device__ __forceinline__ uint32_t key_encode(uint32_t x) { return (x & 0x7fu) | ((x >> 7) << 8); }
 __device__ __forceinline__ uint32_t key_decode(uint32_t k) { return (k & 0x7fu) | ((k >> 8) << 7); }
 
+// v + the value that the DPP control moves here (0 where no lane is moved)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v) {
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+
+// within rows of 16 lanes by row shifts, then the rows' totals by row
+// broadcasts: six register moves, no trips through the LDS crossbar
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
-    const uint32_t lane = __lane_id();
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        uint32_t t = __shfl_up(v, d);
-        if (lane >= (uint32_t)d) v += t;
-    }
-    return v;
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 
 // Block of NW waves: exclusive prefix of v, block total in *total (lds: NW words)
@@ -448,6 +455,13 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
     }
 }
 
+// block b of n, renumbered so that each XCD (blocks go to the eight in turn)
+// works on consecutive tiles
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t n) {
+    const uint32_t q = n / 8, r = n % 8, x = b % 8, i = b / 8;
+    return x * q + min(x, r) + i;
+}
+
 // ------------------------------------------------------ radix sort passes
 // Two LSD passes of 8 bits over the 16-bit bucket key, independently per
 // segment.  A tile is kSortTile consecutive entries of one segment; wave w of
@@ -460,11 +474,6 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
 // hist[tile0*256 + bin*ntiles + t], so one exclusive scan per segment yields
 // every (bin, tile) destination.
 
-__device__ __forceinline__ uint32_t sort_key(const void* in, int pass, uint64_t pos) {
-    if (pass == 0) return reinterpret_cast<const uint32_t*>(in)[pos] & 0xffffu;
-    return reinterpret_cast<const uint16_t*>(in)[pos];
-}
-
 // Entries of a tile: pass 0 sorts all 2n of the segment; pass 1 only the
 // seg_valid[s] entries with a bucket (pass 0 put them first).
 __device__ __forceinline__ uint32_t tile_len(const SegDesc& sg, uint32_t start, int pass,
@@ -473,28 +482,52 @@ __device__ __forceinline__ uint32_t tile_len(const SegDesc& sg, uint32_t start, 
     return start < n ? min((uint32_t)kSortTile, n - start) : 0u;
 }
 
+// A thread's kSortItems consecutive rounds of a tile, all loads issued before
+// the first is used (clamped to the tile's last entry; the empty asm is where
+// they are waited for): one trip to memory per tile.  With a load per round,
+// waited for in its round, and tiles dealt to the XCDs in turn (xcd_block),
+// the histogram took 45 us and the scatters 131 and 170 us for 2^25 entries;
+// now 27, 97 and 128.
+template <class T>
+__device__ __forceinline__ void load_tile(const T* __restrict__ in, uint64_t base, uint32_t len, uint32_t (&v)[kSortItems]) {
+    const uint32_t p0 = (threadIdx.x >> 6) * (64u * kSortItems) + __lane_id();
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) v[r] = in[base + min(p0 + r * 64u, len - 1)];
+}
+__device__ __forceinline__ void loaded(uint32_t (&v)[kSortItems]) {
+    static_assert(kSortItems == 8, "operands");
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+}
+
+// The second pass's tile histograms (the first pass's come from the
+// decomposition).
 __global__ __launch_bounds__(kSortThreads) void k_sort_hist(const SegDesc* __restrict__ segs,
                                                             const uint32_t* __restrict__ tile_seg,
                                                             uint32_t tile_lo,
-                                                            const void* __restrict__ in, int pass,
+                                                            const uint16_t* __restrict__ in,
                                                             const uint32_t* __restrict__ seg_valid,
                                                             uint32_t* __restrict__ hist) {
     __shared__ uint32_t cnt[kSortWaves][256];
-    const uint32_t t = tile_lo + blockIdx.x;
+    const uint32_t t = tile_lo + xcd_block(blockIdx.x, gridDim.x);
     const uint32_t s = tile_seg[t];
     const SegDesc sg = segs[s];
     const uint32_t tin = t - sg.tile0;
     const uint32_t start = tin * kSortTile;
-    const uint32_t len = tile_len(sg, start, pass, seg_valid, s);
-    const uint32_t shift = pass ? 8u : 0u;
+    const uint32_t len = tile_len(sg, start, 1, seg_valid, s);
     const uint32_t w = threadIdx.x >> 6, lane = __lane_id();
+    uint32_t key[kSortItems];
+    if (len) load_tile(in, sg.ent0 + start, len, key);
     for (uint32_t i = threadIdx.x; i < kSortWaves * 256u; i += kSortThreads) (&cnt[0][0])[i] = 0;
     __syncthreads();
     // counts only (no ranks): one LDS atomic per entry into the wave's own
     // counters is far cheaper than matching equal digits with ballots
-    for (int r = 0; r < kSortItems; r++) {
-        const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
-        if (pos < len) atomicAdd(&cnt[w][(sort_key(in, pass, sg.ent0 + start + pos) >> shift) & 0xffu], 1u);
+    if (len) {
+        loaded(key);
+#pragma unroll
+        for (int r = 0; r < kSortItems; r++) {
+            const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
+            if (pos < len) atomicAdd(&cnt[w][key[r] >> 8], 1u);
+        }
     }
     __syncthreads();
     if (threadIdx.x < 256) {
@@ -692,51 +725,63 @@ __global__ __launch_bounds__(1024) void k_sort_small(const SegDesc* __restrict__
 // from ballot matching in the second pass), sort the tile in LDS, then write
 // each digit's run to its global destination with consecutive threads
 // writing consecutive entries.
+template <int kPass>
 __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
     const SegDesc* __restrict__ segs, const uint32_t* __restrict__ tile_seg, uint32_t tile_lo,
-    const void* __restrict__ in_keys, const uint32_t* __restrict__ in_vals, int pass,
+    const void* __restrict__ in_keys, const uint32_t* __restrict__ in_vals,
     const uint32_t* __restrict__ hist, const uint32_t* __restrict__ seg_valid,
     uint16_t* __restrict__ out_keys, uint32_t* __restrict__ out_vals) {
     __shared__ uint32_t cnt[kSortWaves][256];
-    __shared__ uint32_t dstart[256];
-    __shared__ uint32_t goff[256];
+    __shared__ uint32_t gbase[256];  // a digit's destination less its start in the tile
     __shared__ uint32_t ldsw[kSortWaves];
     __shared__ uint16_t lkey[kSortTile];
     __shared__ uint32_t lval[kSortTile];
-    const uint32_t t = tile_lo + blockIdx.x;
+    constexpr uint32_t shift = kPass ? 8u : 0u;
+    const uint32_t t = tile_lo + xcd_block(blockIdx.x, gridDim.x);
     const uint32_t s = tile_seg[t];
     const SegDesc sg = segs[s];
     const uint32_t tin = t - sg.tile0;
     const uint32_t start = tin * kSortTile;
-    const uint32_t len = tile_len(sg, start, pass, seg_valid, s);
-    const uint32_t shift = pass ? 8u : 0u;
+    const uint32_t len = tile_len(sg, start, kPass, seg_valid, s);
+    if (len == 0) return;
     const uint32_t w = threadIdx.x >> 6, lane = __lane_id();
+    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
+    if (kPass == 0) {
+        load_tile(reinterpret_cast<const uint32_t*>(in_keys), sg.ent0 + start, len, key);
+    } else {
+        load_tile(reinterpret_cast<const uint16_t*>(in_keys), sg.ent0 + start, len, key);
+        load_tile(in_vals, sg.ent0 + start, len, val);
+    }
+    uint32_t gd = 0;
+    if (threadIdx.x < 256) gd = hist[(uint64_t)sg.tile0 * 256 + (uint64_t)threadIdx.x * sg.ntiles + tin];
     for (uint32_t i = threadIdx.x; i < kSortWaves * 256u; i += kSortThreads) (&cnt[0][0])[i] = 0;
     __syncthreads();
-    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
+    loaded(key);
+    // Positions past the end take the key "no bucket": in the first pass its
+    // bin is not written; in the second its low byte comes after every real
+    // one, so the positions rank last in the last bin, past len.
+    uint32_t wd0[kSortItems];
+    bool mixed = false;  // second pass: an instruction's 64 low bytes differ
 #pragma unroll
     for (int r = 0; r < kSortItems; r++) {
         const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
-        const bool act = pos < len;
-        key[r] = ZK_KEY_NONE;
-        val[r] = 0;
-        if (act) {
-            const uint64_t gp = sg.ent0 + start + pos;
-            if (pass == 0) {
-                const uint32_t wd = reinterpret_cast<const uint32_t*>(in_keys)[gp];
-                key[r] = wd & 0xffffu;
-                // the table entry: the position, shifted to its window's copy
-                val[r] = (start + pos + ((wd >> 16) & 0xffu) * sg.wadj + sg.wbase) | (wd & 0x80000000u);
-            } else {
-                key[r] = reinterpret_cast<const uint16_t*>(in_keys)[gp];
-                val[r] = in_vals[gp];
-            }
-        }
-        const uint32_t digit = (key[r] >> shift) & 0xffu;
-        if (pass == 0) {
+        wd0[r] = key[r];
+        key[r] = pos < len ? key[r] & 0xffffu : ZK_KEY_NONE;
+        if (kPass) mixed |= (key[r] & 0xffu) != (__builtin_amdgcn_readfirstlane(key[r]) & 0xffu);
+    }
+    const bool ordered = kPass && __any((int)mixed);
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) {
+        const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
+        if (kPass == 0) {
+            const uint32_t wd = wd0[r];
+            // the table entry: the position, shifted to its window's copy
+            val[r] = (start + pos + ((wd >> 16) & 0xffu) * sg.wadj + sg.wbase) | (wd & 0x80000000u);
             // the first pass need not be stable (the second, stable pass fixes
             // the final order): ranks from LDS atomics, no digit matching
-            rank[r] = act ? atomicAdd(&cnt[w][digit], 1u) : 0u;
+            rank[r] = atomicAdd(&cnt[w][key[r] & 0xffu], 1u);
+        } else if (!ordered) {  // one low byte per instruction: as above
+            rank[r] = atomicAdd(&cnt[w][key[r] >> 8], 1u);
         } else {
             // The second pass must keep the first pass's order between entries
             // of different low bytes; entries with the same low byte and the
@@ -745,8 +790,8 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
             // their low bytes ascend with the lane: the lanes of one low byte
             // at a time take LDS-atomic ranks, lowest low byte first (about
             // two rounds per instruction for uniform digits).
-            const uint32_t lowb = key[r] & 0xffu;
-            bool todo = act;
+            const uint32_t digit = key[r] >> 8, lowb = key[r] & 0xffu;
+            bool todo = true;
             uint32_t rk = 0;
             for (uint64_t m = __ballot(todo); m != 0; m = __ballot(todo)) {
                 const uint32_t lb = __builtin_amdgcn_readlane(lowb, __ffsll((long long)m) - 1);
@@ -770,7 +815,6 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
         uint32_t tot;
         const uint32_t ex = block_exclusive_scan<kSortWaves>(s, ldsw, &tot);
         if (d < 256) {
-            dstart[d] = ex;
             uint32_t run = ex;
 #pragma unroll
             for (int i = 0; i < kSortWaves; i++) {
@@ -778,27 +822,30 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
                 cnt[i][d] = run;
                 run += c;
             }
-            goff[d] = hist[(uint64_t)sg.tile0 * 256 + (uint64_t)d * sg.ntiles + tin];
+            gbase[d] = gd - ex;
         }
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kSortItems; r++) {
-        const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
-        if (pos < len) {
-            const uint32_t j = cnt[w][(key[r] >> shift) & 0xffu] + rank[r];
-            lkey[j] = (uint16_t)key[r];
-            lval[j] = val[r];
-        }
+        const uint32_t j = cnt[w][(key[r] >> shift) & 0xffu] + rank[r];
+        lkey[j] = (uint16_t)key[r];
+        lval[j] = val[r];
     }
     __syncthreads();
-    for (uint32_t j = threadIdx.x; j < len; j += kSortThreads) {
-        const uint32_t k = lkey[j];
-        const uint32_t d = (k >> shift) & 0xffu;
-        const uint32_t g = goff[d] + (j - dstart[d]);
-        if (k != ZK_KEY_NONE) {  // entries without a bucket are not kept
-            out_keys[g] = (uint16_t)k;
-            out_vals[g] = lval[j];
+    uint32_t k[kSortItems], v[kSortItems], g[kSortItems];
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) {
+        const uint32_t j = r * kSortThreads + threadIdx.x;
+        k[r] = lkey[j];
+        v[r] = lval[j];
+        g[r] = gbase[(k[r] >> shift) & 0xffu] + j;
+    }
+#pragma unroll
+    for (int r = 0; r < kSortItems; r++) {
+        if (k[r] != ZK_KEY_NONE) {  // entries without a bucket are not kept
+            out_keys[g[r]] = (uint16_t)k[r];
+            out_vals[g[r]] = v[r];
         }
     }
 }
@@ -1394,11 +1441,11 @@ void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const
                       uint32_t tile_lo, uint32_t ntiles, const uint32_t* chunk_seg, uint32_t chunk_lo,
                       uint32_t nchunks, const void* in_keys, const uint32_t* in_vals, int pass,
                       uint32_t* hist, uint32_t* part, uint32_t* seg_valid, uint16_t* out_keys,
-                      uint32_t* out_vals, hipStream_t st, bool scan_seg, bool count) {
+                      uint32_t* out_vals, hipStream_t st, bool scan_seg) {
     if (!ntiles) return;
-    if (count)  // else the tile histograms are already in hist
+    if (pass)  // the first pass's tile histograms are already in hist
         hipLaunchKernelGGL(k_sort_hist, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
-                           in_keys, pass, (const uint32_t*)seg_valid, hist);
+                           (const uint16_t*)in_keys, (const uint32_t*)seg_valid, hist);
     if (scan_seg) {
         hipLaunchKernelGGL(k_scan_seg, dim3(nseg), dim3(1024), 0, st, segs, seg_lo, hist, pass, seg_valid);
     } else {
@@ -1408,9 +1455,12 @@ void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const
         hipLaunchKernelGGL(k_scan_down, dim3(nchunks), dim3(256), 0, st, segs, chunk_seg, chunk_lo, hist,
                            (const uint32_t*)part, pass, seg_valid);
     }
-    hipLaunchKernelGGL(k_sort_scatter, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
-                       in_keys, in_vals, pass, (const uint32_t*)hist, (const uint32_t*)seg_valid,
-                       out_keys, out_vals);
+    if (pass)
+        hipLaunchKernelGGL(k_sort_scatter<1>, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
+                           in_keys, in_vals, (const uint32_t*)hist, (const uint32_t*)seg_valid, out_keys, out_vals);
+    else
+        hipLaunchKernelGGL(k_sort_scatter<0>, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
+                           in_keys, in_vals, (const uint32_t*)hist, (const uint32_t*)seg_valid, out_keys, out_vals);
 }
 
 void launch_sort_small(const SegDesc* segs, uint32_t nseg, const void* digits, uint32_t* seg_valid,
