@@ -221,6 +221,7 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
             s.nbk = 1u << (c - 1);
             s.tile0 = pl.tiles;
             s.ntiles = sh ? nv * ntw : ntw;
+            s.wtiles = ntw;
             s.msm = j;
             s.wadj = sh ? (uint32_t)(shift_stride - (uint64_t)ntw * kSortTile) : 0u;
             s.wbase = sh ? (uint32_t)(w0 * shift_stride) : 0u;
@@ -602,7 +603,7 @@ WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
     const uint64_t ptb = point_bytes(pl.curve), hpb = host_point_bytes(pl.curve);
     const uint64_t rec_cap = 2 * pl.lanes + 2;
     z.desc = layout_for(pl).total;
-    z.digits = pl.entries * 4;
+    z.digits = pl.entries * 2;
     z.keys = pl.entries * 2;
     z.vals = pl.entries * 4;
     z.hist = (uint64_t)pl.tiles * 256 * 4;
@@ -758,15 +759,15 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             const uint32_t ns_p = pt.seg_hi - pt.seg_lo;
             ZK_TRY(rec(ev_s0_[p], S));
             if (pl.small_sort) {
-                launch_sort_small(d_segs, ns_p, ws.digits, (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB,
+                launch_sort_small(d_segs, ns_p, (const uint16_t*)ws.digits, (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB,
                                   (uint32_t*)ws.valsB, S);
             } else {
                 launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
-                                 d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.digits, nullptr, 0,
+                                 d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, (const uint16_t*)ws.digits, nullptr, 0,
                                  (uint32_t*)ws.hist, (uint32_t*)ws.part, (uint32_t*)ws.segvalid,
                                  (uint16_t*)ws.keysA, (uint32_t*)ws.valsA, S, pt.scan_seg);
                 launch_sort_pass(d_segs, pt.seg_lo, ns_p, d_tile_seg, pt.tile_lo, pt.tile_hi - pt.tile_lo,
-                                 d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, ws.keysA,
+                                 d_chunk_seg, pt.chunk_lo, pt.chunk_hi - pt.chunk_lo, (const uint16_t*)ws.keysA,
                                  (const uint32_t*)ws.valsA, 1, (uint32_t*)ws.hist, (uint32_t*)ws.part,
                                  (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB, (uint32_t*)ws.valsB, S, pt.scan_seg);
             }

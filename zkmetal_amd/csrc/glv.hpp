@@ -93,12 +93,6 @@ __device__ __forceinline__ unsigned sub_n(uint32_t* a, const uint32_t* b) {
     return br;
 }
 
-__device__ __forceinline__ void add_r(uint32_t* a) {
-    unsigned c = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) a[i] = __builtin_addc(a[i], r_limb(i), c, &c);
-}
-
 __device__ __forceinline__ bool geq_r(const uint32_t* a) {
     unsigned br = 0;
 #pragma unroll
@@ -111,6 +105,60 @@ struct GlvSplit {
     bool neg1, neg2;
 };
 
+// hi:lo += a * b (b uniform): the multiply-add's carry goes straight into the
+// third word, two instructions a product where the compiler's rows take four
+__device__ __forceinline__ void mac_uniform(uint64_t& lo, uint32_t& hi, uint32_t a, uint32_t b) {
+    asm("v_mad_u64_u32 %0, vcc, %2, %3, %0\n\tv_addc_co_u32 %1, vcc, 0, %1, vcc"
+        : "+v"(lo), "+v"(hi)
+        : "v"(a), "s"(b)
+        : "vcc");
+}
+
+// Words FROM.. of a * b (NA and NB words, b uniform), column by column; the
+// products of lower columns are left out, so out[FROM] is low by less than
+// min(NA, NB) carries into the column above, which is why the caller starts
+// one column early and looks.  LAST: words past it are not wanted.
+template <int NA, int NB, int FROM, int LAST>
+__device__ __forceinline__ void mul_columns(const uint32_t* a, const uint32_t* b, uint32_t* out) {
+    uint64_t lo = 0;
+#pragma unroll
+    for (int q = FROM; q <= LAST; q++) {
+        uint32_t hi = 0;
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+            if (q - i >= 0 && q - i < NB) {
+                if (q < LAST) mac_uniform(lo, hi, a[i], b[q - i]);
+                else lo = (uint32_t)lo + a[i] * b[q - i];
+            }
+        out[q] = (uint32_t)lo;
+        lo = (lo >> 32) | ((uint64_t)hi << 32);
+    }
+}
+
+// floor(k g / 2^256), NC words.  The products below column 6 add less than
+// (NG + 1) 2^224: unless word 7 is within that of its end, they change
+// nothing above it; else (7 of 2^32 scalars) the whole product is taken.
+template <int NG, int NC>
+__device__ __forceinline__ void mul_high(const uint32_t* k, const uint32_t* g, uint32_t* out) {
+    uint32_t w[8 + NG];
+    mul_columns<8, NG, 6, 7 + NC>(k, g, w);
+    if (w[7] >= 0u - (uint32_t)(NG + 2)) mul_wide<8, NG>(k, g, w);
+#pragma unroll
+    for (int i = 0; i < NC; i++) out[i] = w[8 + i];
+}
+
+// a = |a| of a two's complement value; returns whether it was negative
+__device__ __forceinline__ bool abs128(uint32_t a[4]) {
+    const uint32_t s = (uint32_t)((int32_t)a[3] >> 31);
+    unsigned br = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) a[i] = __builtin_subc(a[i] ^ s, s, br, &br);
+    return s != 0;
+}
+
+// Only the low 128 bits of k1 and k2 are formed: both are below 2^127 in
+// magnitude, so bit 127 is their sign.  With whole products and k1 folded
+// mod r this was two thirds of the decomposition's instructions.
 __device__ inline GlvSplit glv_split(const uint32_t kin[8]) {
     uint32_t k[8];
 #pragma unroll
@@ -124,78 +172,36 @@ __device__ inline GlvSplit glv_split(const uint32_t kin[8]) {
     }
     const uint32_t g1[5] = {0x391eb18du, 0x7a7bd9d4u, 0xa773d2cfu, 0x4ccef014u, 0x2u};
     const uint32_t g2[3] = {0xc7e0b3d7u, 0xd91d232eu, 0x2u};
-    const uint32_t a1[2] = {0x94d213e3u, 0x89d32568u};
+    const uint32_t a1[2] = {0x94d213e3u, 0x89d32568u};  // also b2
     const uint32_t a2[4] = {0x1221250bu, 0x0be4e154u, 0xeeb859fdu, 0x6f4d8248u};
     const uint32_t mb1[4] = {0x7d4f1128u, 0x8211bbebu, 0xeeb859fcu, 0x6f4d8248u};
-    uint32_t w13[13], w11[11];
-    mul_wide<8, 5>(k, g1, w13);
-    mul_wide<8, 3>(k, g2, w11);
-    uint32_t c1[4] = {w13[8], w13[9], w13[10], w13[11]};  // floor(k g1 / 2^256)
-    uint32_t c2[2] = {w11[8], w11[9]};                    // floor(k g2 / 2^256)
+    uint32_t c1[4], c2[2];
+    mul_high<5, 4>(k, g1, c1);
+    mul_high<3, 2>(k, g2, c2);
 
-    // k1 = k - c2 a1 - c1 a2 (mod r)
-    uint32_t t4[4], t8[8];
-    mul_wide<2, 2>(c2, a1, t4);
-    uint32_t s8[8] = {t4[0], t4[1], t4[2], t4[3], 0, 0, 0, 0};
-    uint32_t k1[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) k1[i] = k[i];
-    if (sub_n<8>(k1, s8)) add_r(k1);
-    mul_wide<4, 4>(c1, a2, t8);
-    if (sub_n<8>(k1, t8)) add_r(k1);
-
-    // k2 = c2 (-b1) - c1 b2 as a signed integer
-    uint32_t x6[6], y6[6];
-    mul_wide<2, 4>(c2, mb1, x6);
-    mul_wide<4, 2>(c1, a1, y6);  // b2 == a1
-    bool n2 = sub_n<6>(x6, y6) != 0;
-    if (n2) {
-        unsigned br = 0;
-#pragma unroll
-        for (int i = 0; i < 6; i++) x6[i] = __builtin_subc(0u, x6[i], br, &br);
-    }
-    // fold k1 into [0, r/2]
-    const uint32_t half[8] = {0xf8000000u, 0xa1f0fac9u, 0x3cdcb848u, 0x9419f424u,
-                              0x40c0ac2eu, 0xdc2822dbu, 0x7098d014u, 0x18322739u};
-    unsigned br = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) (void)__builtin_subc(k1[i], half[i], br, &br);
-    bool n1 = (br == 0);
-    if (n1) {
-        uint32_t rr[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) rr[i] = r_limb(i);
-        sub_n<8>(rr, k1);
-#pragma unroll
-        for (int i = 0; i < 8; i++) k1[i] = rr[i];
-    }
     GlvSplit s;
+    uint32_t t[4], u[4];
+    // k1 = k - c1 a2 - c2 a1
+    mul_columns<4, 4, 0, 3>(c1, a2, t);
+    mul_columns<2, 2, 0, 3>(c2, a1, u);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        s.k1[i] = k1[i];
-        s.k2[i] = x6[i];
-    }
-    s.neg1 = n1;
-    s.neg2 = n2;
+    for (int i = 0; i < 4; i++) s.k1[i] = k[i];
+    sub_n<4>(s.k1, t);
+    sub_n<4>(s.k1, u);
+    s.neg1 = abs128(s.k1);
+    // k2 = c2 (-b1) - c1 b2
+    mul_columns<2, 4, 0, 3>(c2, mb1, s.k2);
+    mul_columns<4, 2, 0, 3>(c1, a1, u);
+    sub_n<4>(s.k2, u);
+    s.neg2 = abs128(s.k2);
     return s;
 }
 
-// c-bit window w of a 128-bit value held in 4 little-endian limbs
-// bits [w c, w c + c) of the 128-bit v, from two 64-bit halves by shifts (an
-// indexed register array would be placed in scratch memory)
-__device__ __forceinline__ uint32_t window_bits128(const uint32_t v[4], uint32_t w, uint32_t c) {
-    const uint64_t lo = ((uint64_t)v[1] << 32) | v[0], hi = ((uint64_t)v[3] << 32) | v[2];
-    const uint32_t off = w * c;
-    uint64_t x;
-    if (off >= 128u) x = 0;
-    else if (off >= 64u) x = hi >> (off - 64u);
-    else x = (lo >> off) | (off ? hi << (64u - off) : 0ull);
-    return (uint32_t)x & ((1u << c) - 1u);
-}
-
 // Digit word layout (one per window per half-scalar):
-//   bits 0..15  bucket key = |d| - 1, or 0xFFFF when d == 0 (no bucket)
-//   bit  31     the point is subtracted (digit sign xor GLV sign)
+//   0xFFFF when d == 0 (no bucket), else the sort key of bucket |d| - 1
+//   (key_encode: bit 7 is free), with bit 7 set if the point is subtracted
+//   (digit sign xor GLV sign); never set beside the largest key, 0xFF7F
 #define ZK_KEY_NONE 0xFFFFu
+#define ZK_SIGN 0x80u
 
 }  // namespace zk

@@ -37,7 +37,7 @@ using Ar = Arith<Bn254Fr>;
 // Sort key of a bucket index x < 2^15: low 7 bits in byte 0, the rest in
 // byte 1.  A real key's low byte is then <= 0x7f, so the first radix pass
 // puts every "no bucket" entry (0xFFFF) in bin 0xFF, alone, and can drop them.
-__device__ __forceinline__ uint32_t key_encode(uint32_t x) { return (x & 0x7fu) | ((x >> 7) << 8); }
+__device__ __forceinline__ uint32_t key_encode(uint32_t x) { return x + (x & ~0x7fu); }
 __device__ __forceinline__ uint32_t key_decode(uint32_t k) { return (k & 0x7fu) | ((k >> 8) << 7); }
 
 // v + the value that the DPP control moves here (0 where no lane is moved)
@@ -353,10 +353,13 @@ __device__ __forceinline__ uint32_t window_bits256(const uint32_t k[8], uint32_t
 // (entry) of the segment, ntw = the window's tiles; a window-shifted MSM
 // (wps > 1) pads each window to whole tiles with "no bucket" digits.
 // A block has kThreads threads.  Each walks its scalars one after another, a
-// chain of ~600 instructions each, so a call too small to fill the chip takes
+// chain of ~700 instructions each, so a call too small to fill the chip takes
 // 1024 threads, 2 scalars deep (2^16 points: 43 us with 256 threads, 27 with
-// 512, 20 with 1024); a large one is bound by its LDS atomics and runs best
-// with 512 (2^22 points: 150, 131, 160 us).
+// 512, 20 with 1024); a large one runs best with 512 (2^22 points: 150, 131,
+// 160 us).  Those were with 32-bit digit words, carries from window to window
+// and whole products in the split; with 16-bit words, biased digits and the
+// products that reach the quotients, 2^22 points take 104 us: 78 us of
+// instructions, 52 us of memory traffic.
 static_assert(kSortTile <= (1 << 15) && kSortTile / 2 / 1024 >= 1, "decomposition tiling");
 
 template <int EPS, bool kModR, int kDecThreads>
@@ -366,13 +369,14 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
                                                           const SegDesc* __restrict__ segs,
                                                           const uint4* __restrict__ scalars,
                                                           const uint64_t* __restrict__ idmask,
-                                                          uint2* __restrict__ digits,
+                                                          uint16_t* __restrict__ digits,
                                                           uint32_t* __restrict__ hist,
                                                           uint32_t* __restrict__ err) {
     // windows (nwin <= 64) x key byte 0, two 16-bit counts per word (a tile
     // has at most kSortTile <= 2^15 entries, so no count reaches 2^16)
     __shared__ uint32_t cnt[kMaxWindows * 128];
     __shared__ uint64_t pos0[kMaxWindows];  // first position of window w's entries
+    __shared__ uint32_t bias[2][8];
     const uint32_t b = blockIdx.x;
     const uint32_t j = upper_index(msm_dtile0, nmsm, b);
     const MsmDesc m = msms[j];
@@ -383,9 +387,36 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
     if (threadIdx.x < m.nwin)
         pos0[threadIdx.x] = segs[m.seg0 + threadIdx.x / m.wps].ent0 +
                             (uint64_t)(threadIdx.x % m.wps) * ntw * kSortTile;
+    // Signed digits without carries: a positive half takes half a window's range
+    // less one in every window but the top one, a negative half the whole half
+    // range, and it comes off each digit again, so a digit half a range large
+    // always ends up added (the words have no room for it subtracted when
+    // c = 16).  The top digit is at most half (the values are below 2^126.97,
+    // or 2^253.6; far below it when c = 16).
+    const uint32_t c = m.c, half = 1u << (c - 1), mask = (1u << c) - 1u;
+    if (threadIdx.x < 16) {
+        const uint32_t d = half - 1u + (threadIdx.x >> 3), lo = 32u * (threadIdx.x & 7u);
+        uint32_t x = 0;
+        for (uint32_t w = 0; w + 1 < m.nwin; w++) {
+            const int32_t sh = (int32_t)(c * w - lo);
+            if (sh >= 0 && sh < 32) x += d << sh;
+            else if (sh < 0 && sh > -32) x += d >> -sh;
+        }
+        (&bias[0][0])[threadIdx.x] = x;
+    }
     __syncthreads();
-    const uint32_t c = m.c, half = 1u << (c - 1), full = 1u << c;
-    bool carry_left = false;
+    // The word of biased digit d (off: what the bias added), counted for the
+    // sort.  A "no bucket" word is not: its bin is the last one, whose count
+    // nothing reads, and for witness-like scalars a wave's atomics there were
+    // one serial chain (2^23 such scalars: 361 -> 182 us).
+    auto word = [&](uint32_t w, uint32_t d, uint32_t off, uint32_t neg) {
+        const uint32_t v = d - off;
+        if (v == 0) return ZK_KEY_NONE;
+        const uint32_t key = key_encode((uint32_t)abs((int32_t)v) - 1u);
+        if (hist) atomicAdd(&cnt[w * 128 + ((key & 0x7eu) >> 1)], 1u << ((key << 4) & 31u));
+        return key | (((v ^ neg) >> 24) & ZK_SIGN);
+    };
+    bool over = false;
     constexpr int kPer = kSortTile / EPS / kDecThreads;  // scalars per thread
     for (int r = 0; r < kPer; r++) {
         const uint64_t i = (uint64_t)tin * (kSortTile / EPS) + (uint64_t)r * kDecThreads + threadIdx.x;
@@ -409,42 +440,40 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
         if constexpr (EPS == 1) {
             if constexpr (kModR) reduce_mod_r(k);
             else reduce_mod_p(k);
-            uint32_t carry = 0;
+            unsigned cy = 0;
+#pragma unroll
+            for (int q = 0; q < 8; q++) k[q] = __builtin_addc(k[q], bias[0][q], cy, &cy);
             for (uint32_t w = 0; w < m.nwin; w++) {
-                uint32_t d = window_bits256(k, w, c) + carry, neg = 0;
-                carry = d > half;
-                if (carry) { d = full - d; neg = 1u; }
-                const uint32_t wd = d ? (key_encode(d - 1u) | (neg << 31)) : ZK_KEY_NONE;
-                reinterpret_cast<uint32_t*>(digits)[pos0[w] + i] = wd;
-                if (hist) atomicAdd(&cnt[w * 128 + ((wd & 0xffu) >> 1)], 1u << ((wd & 1u) * 16));
+                const uint32_t d = window_bits256(k, w, c);
+                over |= w + 1 == m.nwin && d > half;
+                digits[pos0[w] + i] = (uint16_t)word(w, d, w + 1 < m.nwin ? half - 1u : 0u, 0);
             }
-            carry_left |= carry != 0;
             continue;
         }
         GlvSplit sp = glv_split(k);
-        uint32_t carry1 = 0, carry2 = 0;
-        uint32_t v = 0;  // local window of w's segment
-        for (uint32_t w = 0; w < m.nwin; w++) {
-            uint32_t d1 = window_bits128(sp.k1, w, c) + carry1;
-            uint32_t d2 = window_bits128(sp.k2, w, c) + carry2;
-            uint32_t neg1 = sp.neg1 ? 1u : 0u, neg2 = sp.neg2 ? 1u : 0u;
-            carry1 = d1 > half;
-            carry2 = d2 > half;
-            if (carry1) { d1 = full - d1; neg1 ^= 1u; }
-            if (carry2) { d2 = full - d2; neg2 ^= 1u; }
-            const uint32_t vt = v << 16;
-            uint32_t w1 = d1 ? (key_encode(d1 - 1u) | vt | (neg1 << 31)) : ZK_KEY_NONE;
-            uint32_t w2 = d2 ? (key_encode(d2 - 1u) | vt | (neg2 << 31)) : ZK_KEY_NONE;
-            digits[(pos0[w] + 2 * i) >> 1] = make_uint2(w1, w2);
-            if (hist) {
-                atomicAdd(&cnt[w * 128 + ((w1 & 0xffu) >> 1)], 1u << ((w1 & 1u) * 16));
-                atomicAdd(&cnt[w * 128 + ((w2 & 0xffu) >> 1)], 1u << ((w2 & 1u) * 16));
-            }
-            if (++v == m.wps) v = 0;
+        unsigned cy1 = 0, cy2 = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            sp.k1[q] = __builtin_addc(sp.k1[q], sp.neg1 ? bias[1][q] : bias[0][q], cy1, &cy1);
+            sp.k2[q] = __builtin_addc(sp.k2[q], sp.neg2 ? bias[1][q] : bias[0][q], cy2, &cy2);
         }
-        carry_left |= (carry1 | carry2) != 0;
+        uint64_t lo1 = ((uint64_t)sp.k1[1] << 32) | sp.k1[0], hi1 = ((uint64_t)sp.k1[3] << 32) | sp.k1[2];
+        uint64_t lo2 = ((uint64_t)sp.k2[1] << 32) | sp.k2[0], hi2 = ((uint64_t)sp.k2[3] << 32) | sp.k2[2];
+        const uint32_t neg1 = sp.neg1 ? 0x80000000u : 0u, neg2 = sp.neg2 ? 0x80000000u : 0u;
+        const uint32_t off1 = half - 1u + (sp.neg1 ? 1u : 0u), off2 = half - 1u + (sp.neg2 ? 1u : 0u);
+        for (uint32_t w = 0; w < m.nwin; w++) {
+            const uint32_t d1 = (uint32_t)lo1 & mask, d2 = (uint32_t)lo2 & mask;
+            lo1 = (lo1 >> c) | (hi1 << (64u - c));
+            lo2 = (lo2 >> c) | (hi2 << (64u - c));
+            hi1 >>= c;
+            hi2 >>= c;
+            over |= w + 1 == m.nwin && max(d1, d2) > half;
+            const uint32_t biased = w + 1 < m.nwin ? ~0u : 0u;
+            const uint32_t w1 = word(w, d1, off1 & biased, neg1), w2 = word(w, d2, off2 & biased, neg2);
+            reinterpret_cast<uint32_t*>(digits)[(pos0[w] + 2 * i) >> 1] = w1 | (w2 << 16);
+        }
     }
-    if (carry_left) atomicOr(err, 1u);
+    if (over) atomicOr(err, 1u);
     if (!hist) return;  // k_sort_small counts for itself
     __syncthreads();
     for (uint32_t x = threadIdx.x; x < m.nwin * 256u; x += kDecThreads) {
@@ -487,7 +516,7 @@ __device__ __forceinline__ uint32_t tile_len(const SegDesc& sg, uint32_t start, 
 // they are waited for): one trip to memory per tile.  With a load per round,
 // waited for in its round, and tiles dealt to the XCDs in turn (xcd_block),
 // the histogram took 45 us and the scatters 131 and 170 us for 2^25 entries;
-// now 27, 97 and 128.
+// now 24, 92 and 126.
 template <class T>
 __device__ __forceinline__ void load_tile(const T* __restrict__ in, uint64_t base, uint32_t len, uint32_t (&v)[kSortItems]) {
     const uint32_t p0 = (threadIdx.x >> 6) * (64u * kSortItems) + __lane_id();
@@ -676,7 +705,7 @@ __global__ __launch_bounds__(1024) void k_scan_seg(const SegDesc* __restrict__ s
 // latency of the scans, not the entries (4097 points: 12 us against 55; the
 // whole call 310 -> 280 us, 256 points 246 -> 213).
 __global__ __launch_bounds__(1024) void k_sort_small(const SegDesc* __restrict__ segs,
-                                                     const uint32_t* __restrict__ digits,
+                                                     const uint16_t* __restrict__ digits,
                                                      uint32_t* __restrict__ seg_valid,
                                                      uint16_t* __restrict__ out_keys,
                                                      uint32_t* __restrict__ out_vals) {
@@ -695,8 +724,8 @@ __global__ __launch_bounds__(1024) void k_sort_small(const SegDesc* __restrict__
     __syncthreads();
 #pragma unroll
     for (uint32_t r = 0; r < kPer; r++) {
-        const uint32_t key = wd[r] & 0xffffu;
-        rank[r] = key != ZK_KEY_NONE ? atomicAdd(&cnt[key_decode(key)], 1u) : 0u;
+        const uint32_t key = wd[r] & ~ZK_SIGN;
+        rank[r] = wd[r] != ZK_KEY_NONE ? atomicAdd(&cnt[key_decode(key)], 1u) : 0u;
     }
     __syncthreads();
     uint32_t carry = 0;
@@ -712,12 +741,13 @@ __global__ __launch_bounds__(1024) void k_sort_small(const SegDesc* __restrict__
     __syncthreads();
 #pragma unroll
     for (uint32_t r = 0; r < kPer; r++) {
-        const uint32_t key = wd[r] & 0xffffu;
-        if (key == ZK_KEY_NONE) continue;
+        if (wd[r] == ZK_KEY_NONE) continue;
+        const uint32_t key = wd[r] & ~ZK_SIGN;
         const uint64_t g = sg.ent0 + cnt[key_decode(key)] + rank[r];
         out_keys[g] = (uint16_t)key;
         // the table entry: the position, shifted to its window's copy
-        out_vals[g] = (r * 1024 + threadIdx.x + ((wd[r] >> 16) & 0xffu) * sg.wadj + sg.wbase) | (wd[r] & 0x80000000u);
+        out_vals[g] = (r * 1024 + threadIdx.x + r * 1024 / kSortTile / sg.wtiles * sg.wadj + sg.wbase) |
+                      ((wd[r] & ZK_SIGN) << 24);
     }
 }
 
@@ -728,7 +758,7 @@ __global__ __launch_bounds__(1024) void k_sort_small(const SegDesc* __restrict__
 template <int kPass>
 __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
     const SegDesc* __restrict__ segs, const uint32_t* __restrict__ tile_seg, uint32_t tile_lo,
-    const void* __restrict__ in_keys, const uint32_t* __restrict__ in_vals,
+    const uint16_t* __restrict__ in_keys, const uint32_t* __restrict__ in_vals,
     const uint32_t* __restrict__ hist, const uint32_t* __restrict__ seg_valid,
     uint16_t* __restrict__ out_keys, uint32_t* __restrict__ out_vals) {
     __shared__ uint32_t cnt[kSortWaves][256];
@@ -736,6 +766,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
     __shared__ uint32_t ldsw[kSortWaves];
     __shared__ uint16_t lkey[kSortTile];
     __shared__ uint32_t lval[kSortTile];
+    static_assert(ZK_SIGN << 24 == 0x80000000u, "digit sign to table entry sign");
     constexpr uint32_t shift = kPass ? 8u : 0u;
     const uint32_t t = tile_lo + xcd_block(blockIdx.x, gridDim.x);
     const uint32_t s = tile_seg[t];
@@ -746,42 +777,42 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
     if (len == 0) return;
     const uint32_t w = threadIdx.x >> 6, lane = __lane_id();
     uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
-    if (kPass == 0) {
-        load_tile(reinterpret_cast<const uint32_t*>(in_keys), sg.ent0 + start, len, key);
-    } else {
-        load_tile(reinterpret_cast<const uint16_t*>(in_keys), sg.ent0 + start, len, key);
-        load_tile(in_vals, sg.ent0 + start, len, val);
-    }
+    load_tile(in_keys, sg.ent0 + start, len, key);
+    if (kPass) load_tile(in_vals, sg.ent0 + start, len, val);
     uint32_t gd = 0;
     if (threadIdx.x < 256) gd = hist[(uint64_t)sg.tile0 * 256 + (uint64_t)threadIdx.x * sg.ntiles + tin];
     for (uint32_t i = threadIdx.x; i < kSortWaves * 256u; i += kSortThreads) (&cnt[0][0])[i] = 0;
     __syncthreads();
     loaded(key);
-    // Positions past the end take the key "no bucket": in the first pass its
-    // bin is not written; in the second its low byte comes after every real
+    // Positions past the end take the key "no bucket".  In the first pass, whose
+    // digits are below 128, a lane counts those entries in a bin of its own
+    // past them (in one bin, a wave's atomics are one serial chain); they
+    // are not written.  In the second their low byte comes after every real
     // one, so the positions rank last in the last bin, past len.
-    uint32_t wd0[kSortItems];
+    auto bin = [&](uint32_t key) { return kPass ? key >> 8 : min(key & 0xffu, 128u + lane); };
+    // First pass: the sign goes to the table entry, the position shifted to its
+    // window's copy (a tile holds one window's entries).
+    const uint32_t entry0 = kPass ? 0u : start + tin / sg.wtiles * sg.wadj + sg.wbase;
     bool mixed = false;  // second pass: an instruction's 64 low bytes differ
 #pragma unroll
     for (int r = 0; r < kSortItems; r++) {
         const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
-        wd0[r] = key[r];
-        key[r] = pos < len ? key[r] & 0xffffu : ZK_KEY_NONE;
+        if (pos >= len) key[r] = ZK_KEY_NONE;
+        if (kPass == 0) {
+            val[r] = (entry0 + pos) | ((key[r] & ZK_SIGN) << 24);
+            if (key[r] != ZK_KEY_NONE) key[r] &= ~ZK_SIGN;
+        }
         if (kPass) mixed |= (key[r] & 0xffu) != (__builtin_amdgcn_readfirstlane(key[r]) & 0xffu);
     }
     const bool ordered = kPass && __any((int)mixed);
 #pragma unroll
     for (int r = 0; r < kSortItems; r++) {
-        const uint32_t pos = w * (64u * kSortItems) + r * 64u + lane;
         if (kPass == 0) {
-            const uint32_t wd = wd0[r];
-            // the table entry: the position, shifted to its window's copy
-            val[r] = (start + pos + ((wd >> 16) & 0xffu) * sg.wadj + sg.wbase) | (wd & 0x80000000u);
             // the first pass need not be stable (the second, stable pass fixes
             // the final order): ranks from LDS atomics, no digit matching
-            rank[r] = atomicAdd(&cnt[w][key[r] & 0xffu], 1u);
+            rank[r] = atomicAdd(&cnt[w][bin(key[r])], 1u);
         } else if (!ordered) {  // one low byte per instruction: as above
-            rank[r] = atomicAdd(&cnt[w][key[r] >> 8], 1u);
+            rank[r] = atomicAdd(&cnt[w][bin(key[r])], 1u);
         } else {
             // The second pass must keep the first pass's order between entries
             // of different low bytes; entries with the same low byte and the
@@ -828,7 +859,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kSortItems; r++) {
-        const uint32_t j = cnt[w][(key[r] >> shift) & 0xffu] + rank[r];
+        const uint32_t j = cnt[w][bin(key[r])] + rank[r];
         lkey[j] = (uint16_t)key[r];
         lval[j] = val[r];
     }
@@ -1422,7 +1453,7 @@ void launch_decompose(CurveId cv, const MsmDesc* msms, const uint64_t* msm_dtile
     // up to a block per CU: the wide blocks (see k_decompose)
 #define ZK_DEC(EPS, MODR, THREADS)                                                                       \
     hipLaunchKernelGGL((k_decompose<EPS, MODR, THREADS>), dim3(dtiles), dim3(THREADS), 0, st, msms, msm_dtile0, \
-                       nmsm, segs, (const uint4*)scalars, idm, (uint2*)digits, hist, err)
+                       nmsm, segs, (const uint4*)scalars, idm, (uint16_t*)digits, hist, err)
     const bool wide = dtiles <= 256;
     if (cv == CurveId::Grumpkin) {
         if (wide) ZK_DEC(1, false, 1024);
@@ -1439,13 +1470,13 @@ void launch_decompose(CurveId cv, const MsmDesc* msms, const uint64_t* msm_dtile
 
 void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const uint32_t* tile_seg,
                       uint32_t tile_lo, uint32_t ntiles, const uint32_t* chunk_seg, uint32_t chunk_lo,
-                      uint32_t nchunks, const void* in_keys, const uint32_t* in_vals, int pass,
+                      uint32_t nchunks, const uint16_t* in_keys, const uint32_t* in_vals, int pass,
                       uint32_t* hist, uint32_t* part, uint32_t* seg_valid, uint16_t* out_keys,
                       uint32_t* out_vals, hipStream_t st, bool scan_seg) {
     if (!ntiles) return;
     if (pass)  // the first pass's tile histograms are already in hist
         hipLaunchKernelGGL(k_sort_hist, dim3(ntiles), dim3(kSortThreads), 0, st, segs, tile_seg, tile_lo,
-                           (const uint16_t*)in_keys, (const uint32_t*)seg_valid, hist);
+                           in_keys, (const uint32_t*)seg_valid, hist);
     if (scan_seg) {
         hipLaunchKernelGGL(k_scan_seg, dim3(nseg), dim3(1024), 0, st, segs, seg_lo, hist, pass, seg_valid);
     } else {
@@ -1463,10 +1494,10 @@ void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const
                            in_keys, in_vals, (const uint32_t*)hist, (const uint32_t*)seg_valid, out_keys, out_vals);
 }
 
-void launch_sort_small(const SegDesc* segs, uint32_t nseg, const void* digits, uint32_t* seg_valid,
+void launch_sort_small(const SegDesc* segs, uint32_t nseg, const uint16_t* digits, uint32_t* seg_valid,
                        uint16_t* out_keys, uint32_t* out_vals, hipStream_t st) {
     if (!nseg) return;
-    hipLaunchKernelGGL(k_sort_small, dim3(nseg), dim3(1024), 0, st, segs, (const uint32_t*)digits, seg_valid,
+    hipLaunchKernelGGL(k_sort_small, dim3(nseg), dim3(1024), 0, st, segs, digits, seg_valid,
                        out_keys, out_vals);
 }
 

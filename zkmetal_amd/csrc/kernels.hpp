@@ -34,12 +34,12 @@ void launch_decompose(CurveId cv, const MsmDesc* msms, const uint64_t* msm_dtile
 // scan_seg: each segment's histogram scanned by one block (PlanPart)
 void launch_sort_pass(const SegDesc* segs, uint32_t seg_lo, uint32_t nseg, const uint32_t* tile_seg,
                       uint32_t tile_lo, uint32_t ntiles, const uint32_t* chunk_seg, uint32_t chunk_lo,
-                      uint32_t nchunks, const void* in_keys, const uint32_t* in_vals, int pass,
+                      uint32_t nchunks, const uint16_t* in_keys, const uint32_t* in_vals, int pass,
                       uint32_t* hist, uint32_t* part, uint32_t* seg_valid, uint16_t* out_keys,
                       uint32_t* out_vals, hipStream_t st, bool scan_seg);
 // segments [0, nseg) sorted by a block each, both passes in one (every segment
 // within kSmallSortLen entries and kSmallSortBuckets buckets)
-void launch_sort_small(const SegDesc* segs, uint32_t nseg, const void* digits, uint32_t* seg_valid,
+void launch_sort_small(const SegDesc* segs, uint32_t nseg, const uint16_t* digits, uint32_t* seg_valid,
                        uint16_t* out_keys, uint32_t* out_vals, hipStream_t st);
 // desc_bytes of descriptors from pinned host memory, err and buckets zeroed
 // (sizes multiples of 16)

@@ -76,10 +76,10 @@ struct SegDesc {
     uint32_t chunk0;  // first histogram-scan chunk (kScanChunk counts each)
     uint32_t nchunks;
     uint32_t wbase;   // window-shifted: table entry of the segment's first window (0 plain)
-    uint32_t pad;
+    uint32_t wtiles;  // window-shifted: sort tiles of one window (ntiles plain)
 };
-// A digit at position pos of segment s, written for the segment's local
-// window v (digit word bits 16..23), addresses table entry
+// A digit at position pos of segment s, in the segment's local window v (its
+// tile over wtiles), addresses table entry
 // pos + v * wadj + wbase relative to the MSM's table0: for a plain segment
 // (v = 0, wadj = wbase = 0) the position itself.
 
