@@ -162,6 +162,20 @@ struct Arith {
         return r;
     }
 
+    // The reduction's multiple of column k, and what m_j adds to column j + d.
+    // Below kRed the multiple is of N = kPinv p, which is -1 mod 2^29: the digit
+    // itself is the multiple (no multiply) and cancels the column exactly, and
+    // the rest of N, (N + 1) / 2^29 (nine limbs), enters from the next column
+    // on.  N < 2^29 p, so seven such steps and two with p add less than
+    // (1 + 2^-29) p to the result, which every stated bound has room for.
+    // (The accumulation of 2^22 points issues 63 v_mul_lo_u32 fewer per mixed
+    // addition: 5.97 -> 5.84 ms per call.)
+    static constexpr int kRed = 7;
+    static __device__ __forceinline__ uint32_t q_m(uint64_t col, int k) {
+        return (k < kRed ? (uint32_t)col : (uint32_t)col * F::kPinv) & ZQ_MASK;
+    }
+    static __device__ __forceinline__ uint32_t q_red(int j, int d) { return j < kRed ? F::n(d - 1) : F::p(d); }
+
     // a * b / 2^261 - c + K*p mod p (K > 0), or a * b / 2^261 (K == 0):
     // result < ab/2^261 + p + K*p with normalised limbs.  The limbs of K*p - c
     // (q_kpr<K, B>) enter the high columns of the product, where they cost one
@@ -179,21 +193,22 @@ struct Arith {
 #pragma unroll
             for (int j = 0; j < k; j++) {
                 qmac(acc, a.v[j], b.v[k - j]);
-                qmac(acc, m[j], F::p(k - j));
+                qmac(acc, m[j], q_red(j, k - j));
             }
             qmac(acc, a.v[k], b.v[0]);
-            m[k] = ((uint32_t)acc * F::kPinv) & ZQ_MASK;
-            qmac(acc, m[k], F::p(0));
+            m[k] = q_m(acc, k);
+            if (k >= kRed) qmac(acc, m[k], F::p(0));
             acc >>= 29;
             carry_fence(acc);
         }
 #pragma unroll
         for (int k = 9; k < 17; k++) {
             if (K > 0) acc += q_kpr<K, B>(k - 9) - c.v[k - 9];
+            if (k - 9 < kRed) qmac(acc, m[k - 9], q_red(k - 9, 9));
 #pragma unroll
             for (int j = k - 8; j < 9; j++) {
                 qmac(acc, a.v[j], b.v[k - j]);
-                qmac(acc, m[j], F::p(k - j));
+                qmac(acc, m[j], q_red(j, k - j));
             }
             t.v[k - 9] = (uint32_t)acc & ZQ_MASK;
             acc >>= 29;
@@ -225,9 +240,9 @@ struct Arith {
             for (int i = 0; 2 * i < k; i++) qmac(acc, a2[i], a.v[k - i]);
             if ((k & 1) == 0) qmac(acc, a.v[k / 2], a.v[k / 2]);
 #pragma unroll
-            for (int j = 0; j < k; j++) qmac(acc, m[j], F::p(k - j));
-            m[k] = ((uint32_t)acc * F::kPinv) & ZQ_MASK;
-            qmac(acc, m[k], F::p(0));
+            for (int j = 0; j < k; j++) qmac(acc, m[j], q_red(j, k - j));
+            m[k] = q_m(acc, k);
+            if (k >= kRed) qmac(acc, m[k], F::p(0));
             acc >>= 29;
             carry_fence(acc);
         }
@@ -237,8 +252,9 @@ struct Arith {
 #pragma unroll
             for (int i = k - 8; 2 * i < k; i++) qmac(acc, a2[i], a.v[k - i]);
             if ((k & 1) == 0) qmac(acc, a.v[k / 2], a.v[k / 2]);
+            if (k - 9 < kRed) qmac(acc, m[k - 9], q_red(k - 9, 9));
 #pragma unroll
-            for (int j = k - 8; j < 9; j++) qmac(acc, m[j], F::p(k - j));
+            for (int j = k - 8; j < 9; j++) qmac(acc, m[j], q_red(j, k - j));
             t.v[k - 9] = (uint32_t)acc & ZQ_MASK;
             acc >>= 29;
             carry_fence(acc);
@@ -253,7 +269,7 @@ struct Arith {
     // multiply-add chains per column, so each hides the other's latency):
     // r1 = fq_mul_sub<K1, B1>(a1, b1, c1), r2 = fq_mul_sub<K2, B2>(a2, b2, c2),
     // same operand conditions.
-    template <int K1, int B1, int K2, int B2>
+    template <int K1, int B1, int K2, int B2, bool kFixed = false>
     static __device__ __forceinline__ void fq_mul_sub_x2(const Fq& a1, const Fq& b1, const Fq& c1, Fq& r1,
                                                          const Fq& a2, const Fq& b2, const Fq& c2, Fq& r2) {
         uint32_t m1[9], m2[9];
@@ -262,17 +278,17 @@ struct Arith {
         for (int k = 0; k < 9; k++) {
 #pragma unroll
             for (int j = 0; j < k; j++) {
-                qmac(s1, a1.v[j], b1.v[k - j]);
-                qmac(s2, a2.v[j], b2.v[k - j]);
-                qmac(s1, m1[j], F::p(k - j));
-                qmac(s2, m2[j], F::p(k - j));
+                qmac4<kFixed>(s1, s2, a1.v[j], b1.v[k - j], a2.v[j], b2.v[k - j], m1[j], m2[j], q_red(j, k - j));
             }
-            qmac(s1, a1.v[k], b1.v[0]);
-            qmac(s2, a2.v[k], b2.v[0]);
-            m1[k] = ((uint32_t)s1 * F::kPinv) & ZQ_MASK;
-            m2[k] = ((uint32_t)s2 * F::kPinv) & ZQ_MASK;
-            qmac(s1, m1[k], F::p(0));
-            qmac(s2, m2[k], F::p(0));
+            if (k) {
+                qmac2<kFixed>(s1, s2, a1.v[k], b1.v[0], a2.v[k], b2.v[0]);
+            } else {
+                s1 = (uint64_t)a1.v[0] * b1.v[0];
+                s2 = (uint64_t)a2.v[0] * b2.v[0];
+            }
+            m1[k] = q_m(s1, k);
+            m2[k] = q_m(s2, k);
+            if (k >= kRed) qred2<kFixed>(s1, s2, m1[k], m2[k], F::p(0));
             s1 >>= 29;
             s2 >>= 29;
             carry_fence(s1);
@@ -282,12 +298,10 @@ struct Arith {
         for (int k = 9; k < 17; k++) {
             if (K1 > 0) s1 += q_kpr<K1, B1>(k - 9) - c1.v[k - 9];
             if (K2 > 0) s2 += q_kpr<K2, B2>(k - 9) - c2.v[k - 9];
+            if (k - 9 < kRed) qred2<kFixed>(s1, s2, m1[k - 9], m2[k - 9], q_red(k - 9, 9));
 #pragma unroll
             for (int j = k - 8; j < 9; j++) {
-                qmac(s1, a1.v[j], b1.v[k - j]);
-                qmac(s2, a2.v[j], b2.v[k - j]);
-                qmac(s1, m1[j], F::p(k - j));
-                qmac(s2, m2[j], F::p(k - j));
+                qmac4<kFixed>(s1, s2, a1.v[j], b1.v[k - j], a2.v[j], b2.v[k - j], m1[j], m2[j], q_red(j, k - j));
             }
             r1.v[k - 9] = (uint32_t)s1 & ZQ_MASK;
             r2.v[k - 9] = (uint32_t)s2 & ZQ_MASK;
@@ -313,19 +327,19 @@ struct Arith {
                 qmac(s1, a1.v[j], b1.v[k - j]);
                 qmac(s2, a2.v[j], b2.v[k - j]);
                 qmac(s3, a3.v[j], b3.v[k - j]);
-                qmac(s1, m1[j], F::p(k - j));
-                qmac(s2, m2[j], F::p(k - j));
-                qmac(s3, m3[j], F::p(k - j));
+                qmac(s1, m1[j], q_red(j, k - j));
+                qmac(s2, m2[j], q_red(j, k - j));
+                qmac(s3, m3[j], q_red(j, k - j));
             }
             qmac(s1, a1.v[k], b1.v[0]);
             qmac(s2, a2.v[k], b2.v[0]);
             qmac(s3, a3.v[k], b3.v[0]);
-            m1[k] = ((uint32_t)s1 * F::kPinv) & ZQ_MASK;
-            m2[k] = ((uint32_t)s2 * F::kPinv) & ZQ_MASK;
-            m3[k] = ((uint32_t)s3 * F::kPinv) & ZQ_MASK;
-            qmac(s1, m1[k], F::p(0));
-            qmac(s2, m2[k], F::p(0));
-            qmac(s3, m3[k], F::p(0));
+            m1[k] = q_m(s1, k);
+            m2[k] = q_m(s2, k);
+            m3[k] = q_m(s3, k);
+            if (k >= kRed) qmac(s1, m1[k], F::p(0));
+            if (k >= kRed) qmac(s2, m2[k], F::p(0));
+            if (k >= kRed) qmac(s3, m3[k], F::p(0));
             s1 >>= 29;
             s2 >>= 29;
             s3 >>= 29;
@@ -335,14 +349,17 @@ struct Arith {
         }
 #pragma unroll
         for (int k = 9; k < 17; k++) {
+            if (k - 9 < kRed) qmac(s1, m1[k - 9], q_red(k - 9, 9));
+            if (k - 9 < kRed) qmac(s2, m2[k - 9], q_red(k - 9, 9));
+            if (k - 9 < kRed) qmac(s3, m3[k - 9], q_red(k - 9, 9));
 #pragma unroll
             for (int j = k - 8; j < 9; j++) {
                 qmac(s1, a1.v[j], b1.v[k - j]);
                 qmac(s2, a2.v[j], b2.v[k - j]);
                 qmac(s3, a3.v[j], b3.v[k - j]);
-                qmac(s1, m1[j], F::p(k - j));
-                qmac(s2, m2[j], F::p(k - j));
-                qmac(s3, m3[j], F::p(k - j));
+                qmac(s1, m1[j], q_red(j, k - j));
+                qmac(s2, m2[j], q_red(j, k - j));
+                qmac(s3, m3[j], q_red(j, k - j));
             }
             r1.v[k - 9] = (uint32_t)s1 & ZQ_MASK;
             r2.v[k - 9] = (uint32_t)s2 & ZQ_MASK;
@@ -360,6 +377,7 @@ struct Arith {
     }
 
     // r1 = a1^2, r2 = a2^2 side by side (as fq_sqr)
+    template <bool kFixed = false>
     static __device__ __forceinline__ void fq_sqr_x2(const Fq& a1, Fq& r1, const Fq& a2, Fq& r2) {
         uint32_t d1[9], d2[9], m1[9], m2[9];
 #pragma unroll
@@ -372,22 +390,21 @@ struct Arith {
         for (int k = 0; k < 9; k++) {
 #pragma unroll
             for (int i = 0; 2 * i < k; i++) {
-                qmac(s1, d1[i], a1.v[k - i]);
-                qmac(s2, d2[i], a2.v[k - i]);
+                qmac2<kFixed>(s1, s2, d1[i], a1.v[k - i], d2[i], a2.v[k - i]);
             }
-            if ((k & 1) == 0) {
-                qmac(s1, a1.v[k / 2], a1.v[k / 2]);
-                qmac(s2, a2.v[k / 2], a2.v[k / 2]);
+            if (k == 0) {
+                s1 = (uint64_t)a1.v[0] * a1.v[0];
+                s2 = (uint64_t)a2.v[0] * a2.v[0];
+            } else if ((k & 1) == 0) {
+                qmac2<kFixed>(s1, s2, a1.v[k / 2], a1.v[k / 2], a2.v[k / 2], a2.v[k / 2]);
             }
 #pragma unroll
             for (int j = 0; j < k; j++) {
-                qmac(s1, m1[j], F::p(k - j));
-                qmac(s2, m2[j], F::p(k - j));
+                qred2<kFixed>(s1, s2, m1[j], m2[j], q_red(j, k - j));
             }
-            m1[k] = ((uint32_t)s1 * F::kPinv) & ZQ_MASK;
-            m2[k] = ((uint32_t)s2 * F::kPinv) & ZQ_MASK;
-            qmac(s1, m1[k], F::p(0));
-            qmac(s2, m2[k], F::p(0));
+            m1[k] = q_m(s1, k);
+            m2[k] = q_m(s2, k);
+            if (k >= kRed) qred2<kFixed>(s1, s2, m1[k], m2[k], F::p(0));
             s1 >>= 29;
             s2 >>= 29;
             carry_fence(s1);
@@ -397,17 +414,13 @@ struct Arith {
         for (int k = 9; k < 17; k++) {
 #pragma unroll
             for (int i = k - 8; 2 * i < k; i++) {
-                qmac(s1, d1[i], a1.v[k - i]);
-                qmac(s2, d2[i], a2.v[k - i]);
+                qmac2<kFixed>(s1, s2, d1[i], a1.v[k - i], d2[i], a2.v[k - i]);
             }
-            if ((k & 1) == 0) {
-                qmac(s1, a1.v[k / 2], a1.v[k / 2]);
-                qmac(s2, a2.v[k / 2], a2.v[k / 2]);
-            }
+            if ((k & 1) == 0) qmac2<kFixed>(s1, s2, a1.v[k / 2], a1.v[k / 2], a2.v[k / 2], a2.v[k / 2]);
+            if (k - 9 < kRed) qred2<kFixed>(s1, s2, m1[k - 9], m2[k - 9], q_red(k - 9, 9));
 #pragma unroll
             for (int j = k - 8; j < 9; j++) {
-                qmac(s1, m1[j], F::p(k - j));
-                qmac(s2, m2[j], F::p(k - j));
+                qred2<kFixed>(s1, s2, m1[j], m2[j], q_red(j, k - j));
             }
             r1.v[k - 9] = (uint32_t)s1 & ZQ_MASK;
             r2.v[k - 9] = (uint32_t)s2 & ZQ_MASK;
@@ -437,8 +450,8 @@ struct Arith {
                 qmac(s2, a2.v[j], b2.v[k - j]);
                 qmac(t1, c1.v[j], d1.v[k - j]);
                 qmac(t2, c2.v[j], d2.v[k - j]);
-                qmac((j & 1) ? t1 : s1, m1[j], F::p(k - j));
-                qmac((j & 1) ? t2 : s2, m2[j], F::p(k - j));
+                qmac((j & 1) ? t1 : s1, m1[j], q_red(j, k - j));
+                qmac((j & 1) ? t2 : s2, m2[j], q_red(j, k - j));
             }
             qmac(s1, a1.v[k], b1.v[0]);
             qmac(s2, a2.v[k], b2.v[0]);
@@ -446,10 +459,10 @@ struct Arith {
             qmac(t2, c2.v[k], d2.v[0]);
             s1 += t1;
             s2 += t2;
-            m1[k] = ((uint32_t)s1 * F::kPinv) & ZQ_MASK;
-            m2[k] = ((uint32_t)s2 * F::kPinv) & ZQ_MASK;
-            qmac(s1, m1[k], F::p(0));
-            qmac(s2, m2[k], F::p(0));
+            m1[k] = q_m(s1, k);
+            m2[k] = q_m(s2, k);
+            if (k >= kRed) qmac(s1, m1[k], F::p(0));
+            if (k >= kRed) qmac(s2, m2[k], F::p(0));
             s1 >>= 29;
             s2 >>= 29;
             t1 = 0;
@@ -461,14 +474,16 @@ struct Arith {
         for (int k = 9; k < 17; k++) {
             if (K1 > 0) s1 += q_kpr<K1, B1>(k - 9) - e1.v[k - 9];
             if (K2 > 0) s2 += q_kpr<K2, B2>(k - 9) - e2.v[k - 9];
+            if (k - 9 < kRed) qmac(s1, m1[k - 9], q_red(k - 9, 9));
+            if (k - 9 < kRed) qmac(s2, m2[k - 9], q_red(k - 9, 9));
 #pragma unroll
             for (int j = k - 8; j < 9; j++) {
                 qmac(s1, a1.v[j], b1.v[k - j]);
                 qmac(s2, a2.v[j], b2.v[k - j]);
                 qmac(t1, c1.v[j], d1.v[k - j]);
                 qmac(t2, c2.v[j], d2.v[k - j]);
-                qmac((j & 1) ? t1 : s1, m1[j], F::p(k - j));
-                qmac((j & 1) ? t2 : s2, m2[j], F::p(k - j));
+                qmac((j & 1) ? t1 : s1, m1[j], q_red(j, k - j));
+                qmac((j & 1) ? t2 : s2, m2[j], q_red(j, k - j));
             }
             s1 += t1;
             s2 += t2;
@@ -492,6 +507,7 @@ struct Arith {
     // c d and the rest in the other), joined before m is taken.  With K > 0
     // (fq_mul_add_sub_x2) the limbs of K p - e enter the high columns as in
     // fq_mul_sub: result < (ab + cd)/2^261 + p + K p - e.
+    template <bool kFixed = false>
     static __device__ __forceinline__ Fq fq_mul_add(const Fq& a, const Fq& b, const Fq& c, const Fq& d) {
         uint32_t m[9];
         Fq t;
@@ -500,26 +516,25 @@ struct Arith {
         for (int k = 0; k < 9; k++) {
 #pragma unroll
             for (int j = 0; j < k; j++) {
-                qmac(s1, a.v[j], b.v[k - j]);
-                qmac(s2, c.v[j], d.v[k - j]);
-                qmac((j & 1) ? s2 : s1, m[j], F::p(k - j));
+                qmac2<kFixed>(s1, s2, a.v[j], b.v[k - j], c.v[j], d.v[k - j]);
+                qmac((j & 1) ? s2 : s1, m[j], q_red(j, k - j));
             }
             qmac(s1, a.v[k], b.v[0]);
             qmac(s2, c.v[k], d.v[0]);
             s1 += s2;
-            m[k] = ((uint32_t)s1 * F::kPinv) & ZQ_MASK;
-            qmac(s1, m[k], F::p(0));
+            m[k] = q_m(s1, k);
+            if (k >= kRed) qmac(s1, m[k], F::p(0));
             s1 >>= 29;
             s2 = 0;
             carry_fence(s1);
         }
 #pragma unroll
         for (int k = 9; k < 17; k++) {
+            if (k - 9 < kRed) qmac(s1, m[k - 9], q_red(k - 9, 9));
 #pragma unroll
             for (int j = k - 8; j < 9; j++) {
-                qmac(s1, a.v[j], b.v[k - j]);
-                qmac(s2, c.v[j], d.v[k - j]);
-                qmac((j & 1) ? s2 : s1, m[j], F::p(k - j));
+                qmac2<kFixed>(s1, s2, a.v[j], b.v[k - j], c.v[j], d.v[k - j]);
+                qmac((j & 1) ? s2 : s1, m[j], q_red(j, k - j));
             }
             s1 += s2;
             t.v[k - 9] = (uint32_t)s1 & ZQ_MASK;
@@ -729,57 +744,48 @@ struct Arith {
         acc = qxyzz_select(q_id, acc, r);
     }
 
-    // Placeholder for an accumulator that starts a bucket run: the value is never
-    // used (the run's first addition selects the point itself), but ZZ = ZZZ = 1
-    // and X = 0 keep P = x2 - X away from 0, so the first addition does not look
-    // exceptional.
-    static __device__ __forceinline__ QXyzz qxyzz_run_start() {
+    // (x, y) as an XYZZ point
+    static __device__ __forceinline__ QXyzz qxyzz_of(const QAff& q) {
         QXyzz r;
-        r.X = fq_zero();
-        r.Y = fq_zero();
+        r.X = q.x;
+        r.Y = q.y;
         r.ZZ = fq_one();
         r.ZZZ = r.ZZ;
         return r;
     }
 
-    // acc += (x2, y2) in the bucket-accumulation loop.  acc_id says acc is the
-    // identity (a run start, or a cancellation earlier in the run); (x2, y2) is
-    // never the identity there.  X3 is left below 6.5p (no final subtraction):
+    // acc += (x2, y2) in the bucket-accumulation loop; neither is the identity
+    // there (a run's first addition assigns).  Returns whether they cancelled.
+    // X3 is left below 6.5p (no final subtraction):
     // every later use of X takes it as a multiplicand or as the subtrahend of a
     // K = 7 form.  Doubling (acc == q) and cancellation (acc == -q) both have
     // PP = 0 mod p; PP < 1.6p is then 0 or p, so its low limb is 0 or p_0.  That one-limb test screens every step; the exact tests run only in
     // lanes that pass it, and a wave branches to them only if one of its lanes
     // does.  After a cancellation acc holds ZZ = 0 mod p, the stored form of the
     // identity.
-    static __device__ __forceinline__ void qxyzz_madd_run(QXyzz& acc, bool& acc_id, const Fq& x2,
-                                                   const Fq& y2) {
+    static __device__ __forceinline__ bool qxyzz_madd_run(QXyzz& acc, const Fq& x2, const Fq& y2) {
         // the ten products in pairs of independent ones, and Y3's two under one
         // reduction: Y3 = (R (Q - X3 + 7p) + Y1 (2p - PPP)) / 2^261
         Fq P, R, PP, RR, PPP, Q;
-        fq_mul_sub_x2<7, 1, 5, 1>(x2, acc.ZZ, acc.X, P, y2, acc.ZZZ, acc.Y, R);  // < 8.5p, < 6.5p
-        fq_sqr_x2(P, PP, R, RR);                                                   // < 1.6p each
-        fq_mul_sub_x2<0, 1, 0, 1>(P, PP, P, PPP, acc.X, PP, P, Q);                 // < 1.5p each
+        fq_mul_sub_x2<7, 1, 5, 1, true>(x2, acc.ZZ, acc.X, P, y2, acc.ZZZ, acc.Y, R);  // < 8.5p, < 6.5p
+        fq_sqr_x2<true>(P, PP, R, RR);                                                   // < 1.6p each
+        fq_mul_sub_x2<0, 1, 0, 1, true>(P, PP, P, PPP, acc.X, PP, P, Q);                 // < 1.5p each
         QXyzz r;
         Fq T;  // 2Q + PPP < 4.5p, limbs sums of three normalised limbs
 #pragma unroll
         for (int i = 0; i < 9; i++) T.v[i] = Q.v[i] + Q.v[i] + PPP.v[i];
         r.X = fq_sub<5>(RR, T);                                                     // < 6.3p
         r.Y = fq_mul_add(R, fq_sub_lazy<7>(Q, r.X), acc.Y, fq_sub_lazy<2>(fq_zero(), PPP));  // < 1.4p
-        fq_mul_sub_x2<0, 1, 0, 1>(acc.ZZ, PP, P, r.ZZ, acc.ZZZ, PPP, P, r.ZZZ);
+        fq_mul_sub_x2<0, 1, 0, 1, true>(acc.ZZ, PP, P, r.ZZ, acc.ZZZ, PPP, P, r.ZZZ);
         bool cancel = false;
         if (__builtin_expect(PP.v[0] == 0u || PP.v[0] == F::p(0), 0)) {
-            const bool z = !acc_id && fq_is_zero2(PP);
+            const bool z = fq_is_zero2(PP);
             const bool d = z && fq_is_zero2(RR);
             cancel = z && !d;
             if (d) r = qxyzz_dbl_aff(x2, y2);
         }
-        QXyzz q;
-        q.X = x2;
-        q.Y = y2;
-        q.ZZ = fq_one();
-        q.ZZZ = q.ZZ;
-        acc = qxyzz_select(acc_id, q, r);
-        acc_id = cancel;
+        acc = r;
+        return cancel;
     }
 
     // acc += q (both XYZZ; X < 6.5p as stored by the accumulation loop,

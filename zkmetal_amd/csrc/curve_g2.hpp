@@ -144,15 +144,12 @@ struct G2Arith {
         return r;
     }
 
-    // the value an accumulator holds at a bucket run's start: never used (the
-    // run's first addition selects the point), ZZ = ZZZ = 1
-    static __device__ __forceinline__ QXyzz2 run_start() {
-        return QXyzz2{zero2(), zero2(), one2(), one2()};
-    }
+    // (x, y) as an XYZZ point
+    static __device__ __forceinline__ QXyzz2 of(const QAff2& q) { return QXyzz2{q.x, q.y, one2(), one2()}; }
 
-    // acc += (x2, y2) in the bucket-accumulation loop (x2, y2 < 2p, never the
-    // identity); acc_id says acc is the identity (a run start, or a
-    // cancellation earlier in the run).  Doubling and cancellation have P = 0;
+    // acc += (x2, y2) in the bucket-accumulation loop (x2, y2 < 2p; neither
+    // is the identity: a run's first addition assigns).  Returns whether they
+    // cancelled.  Doubling and cancellation have P = 0;
     // the exact tests and the doubling run in a branch a wave takes only when
     // one of its lanes needs it (a ballot makes the branch wave-uniform, so
     // the compiler keeps it a branch instead of computing the doubling on
@@ -161,8 +158,7 @@ struct G2Arith {
     // per component, P, R < 3.1p, PP < 1.3p, PPP, Q < 1.1p, T = 2Q + PPP < 4p,
     // X3 < 5.3p and Y3 < 3.2p before their conditional subtractions, every
     // stored component < 2p after them.
-    static __device__ __forceinline__ void madd_run(QXyzz2& acc, bool& acc_id, const Fq2& x2,
-                                                    const Fq2& y2) {
+    static __device__ __forceinline__ bool madd_run(QXyzz2& acc, const Fq2& x2, const Fq2& y2) {
         const Fq2 P = mul2m<2>(x2, acc.ZZ, acc.X);   // U2 - X1 + 2p
         const Fq2 R = mul2m<2>(y2, acc.ZZZ, acc.Y);  // S2 - Y1 + 2p
         // PP = (P0 + P1)(P0 - P1 + 4p) + 2 P0 P1 u
@@ -190,16 +186,15 @@ struct G2Arith {
         r.ZZ = mul2m<0>(acc.ZZ, PP, P);
         r.ZZZ = mul2m<0>(acc.ZZZ, PPP, P);
         bool cancel = false;
-        const bool ex = !acc_id && is_zero2(PP);  // P = 0 iff PP = 0
+        const bool ex = is_zero2(PP);  // P = 0 iff PP = 0
         if (__builtin_expect(__ballot(ex) != 0, 0)) {
             const bool d = ex && is_zero2(Fq2{red4(R.c0), red4(R.c1)});
             cancel = ex && !d;
             const QXyzz2 dd = dbl_aff(x2, y2);
             r = select(d, dd, r);
         }
-        const QXyzz2 q{x2, y2, one2(), one2()};
-        acc = select(acc_id, q, r);
-        acc_id = cancel;
+        acc = r;
+        return cancel;
     }
 
     // acc += q (both XYZZ, components < 2p), on the merged-reduction products

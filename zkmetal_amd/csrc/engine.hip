@@ -118,10 +118,13 @@ static void plan_reset(Plan& pl) {
 // parts for a call of `entries` sorted entries: the exposed sort is the first
 // part's, and every part adds a round of launches and merge records
 uint32_t default_parts(uint64_t entries) {
-    // measured: a 2^22-point MSM (2^26 entries) runs best in 2 parts, the
-    // 64-MSM batch (2^27.7 entries) in 3; more parts add merge records and
-    // launches faster than they hide sort time
-    return entries >= (1ull << 27) ? 3u : entries >= (1ull << 24) ? 2u : 1u;
+    // measured, 1 against 2 parts: 2^20 points (2^24 entries) 1580 against
+    // 1630 us, 2^20 G2 points (2^24) 4360 against 4400; 2^22 points (2^26)
+    // 5870 against 5715 us, the 64-MSM batch (2^27.7) 15.25 against 15.0 ms (3
+    // parts: 16.0).  With three accumulation waves per SIMD a sort beside the
+    // accumulation finds little room; what two parts gain is the second sort
+    // running on while the first waves start.
+    return entries > (1ull << 24) ? 2u : 1u;
 }
 
 // Window-shifted or plain, by an estimate in mixed-addition units: every
@@ -278,7 +281,12 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
         }
         const uint64_t ns_p = pt.seg_hi - pt.seg_lo;
         const uint64_t half_bucket = ent / (2 * std::max<uint64_t>(1, bk));
-        const uint64_t cap = lane_cap > 2ull * ns_p + 64 ? lane_cap - ns_p : std::max<uint64_t>(lane_cap / 2, 64);
+        uint64_t cap = lane_cap > 2ull * ns_p + 64 ? lane_cap - ns_p : std::max<uint64_t>(lane_cap / 2, 64);
+        // lanes of fewer than 8 entries leave more partial sums to merge than
+        // a third wave per SIMD hides, so such a call fills two (2^16 points: 344
+        // against 352 us); 8 MSMs of 2^16, 28 entries a lane, take 840 us with
+        // three and 853 with two.  The G2 kernel runs one wave per SIMD anyway.
+        if (cv != CurveId::Bn254G2 && ent < 8 * cap) cap = cap * 2 / 3;
         pt.T = (uint32_t)std::max<uint64_t>(std::max<uint64_t>(4, std::min<uint64_t>(32, half_bucket)),
                                             (ent + cap - 1) / cap);
         pt.entries = ent;

@@ -88,9 +88,9 @@ struct G1Curve {
     using Af = QAff;
     static constexpr uint32_t kSlots = 1;
     static constexpr uint64_t kPtBytes = kBucketBytes;
-    static __device__ __forceinline__ Pt run_start() { return Arith<F>::qxyzz_run_start(); }
-    static __device__ __forceinline__ void madd_run(Pt& a, bool& id, const Af& q) {
-        Arith<F>::qxyzz_madd_run(a, id, q.x, q.y);
+    static __device__ __forceinline__ Pt of(const Af& q) { return Arith<F>::qxyzz_of(q); }
+    static __device__ __forceinline__ bool madd_run(Pt& a, const Af& q) {
+        return Arith<F>::qxyzz_madd_run(a, q.x, q.y);
     }
     static __device__ __forceinline__ Af load_tab(const uint4* t, uint64_t e, bool neg) { return load_qtab(t, e, neg); }
     static __device__ __forceinline__ void store(uint4* b, uint64_t i, const Pt& p) { store_qxyzz(b, i, p); }
@@ -101,10 +101,8 @@ struct G2Curve {
     using Af = QAff2;
     static constexpr uint32_t kSlots = 2;
     static constexpr uint64_t kPtBytes = 2 * kBucketBytes;
-    static __device__ __forceinline__ Pt run_start() { return G2Arith::run_start(); }
-    static __device__ __forceinline__ void madd_run(Pt& a, bool& id, const Af& q) {
-        G2Arith::madd_run(a, id, q.x, q.y);
-    }
+    static __device__ __forceinline__ Pt of(const Af& q) { return G2Arith::of(q); }
+    static __device__ __forceinline__ bool madd_run(Pt& a, const Af& q) { return G2Arith::madd_run(a, q.x, q.y); }
     static __device__ __forceinline__ Af load_tab(const uint4* t, uint64_t e, bool neg) { return load_qtab2(t, e, neg); }
     static __device__ __forceinline__ void store(uint4* b, uint64_t i, const Pt& p) { store_qxyzz2(b, i, p); }
 };
@@ -1006,8 +1004,8 @@ __global__ __launch_bounds__(256) void k_accumulate(
     uint32_t cur = keys[b];
     const bool head_open = (b > sg.ent0) && keys[b - 1] == cur;
     bool first = true;
-    typename C::Pt acc = C::run_start();
-    bool acc_id = true;
+    typename C::Pt acc;
+    bool acc_id = true;  // acc is the identity: nothing added yet, or cancelled
     // software pipeline: before entry p's mixed addition the base of entry
     // p+1 is gathered (its value was loaded one iteration earlier, so the
     // gather's address waits on nothing issued in this iteration) and the key
@@ -1031,13 +1029,17 @@ __global__ __launch_bounds__(256) void k_accumulate(
                 if (first) put_record<C>(rec_keys, rec_pts, 2 * L, gk, false, acc);
             }
             first = false;
-            acc = C::run_start();
             acc_id = true;
             cur = k;
         }
         // y is already negated for a negative digit; identity bases have no
         // digits (table bitmap), so q is never the identity
-        C::madd_run(acc, acc_id, q);
+        if (acc_id) {
+            acc = C::of(q);
+            acc_id = false;
+        } else {
+            acc_id = C::madd_run(acc, q);
+        }
         k = kn;
         kn = knn;
         vn = vnn;
@@ -1174,9 +1176,8 @@ __global__ __launch_bounds__(64) void k_test_g2(int op, const uint4* __restrict_
     else if (op == 2) G::madd(a, b.X, b.Y, b_aff_id);
     else if (op == 3) {
         bool id = G::is_id(a);
-        if (id) a = G::run_start();
-        G::madd_run(a, id, b.X, b.Y);
-        if (id) a = G::identity();
+        if (id) a = G::of(QAff2{b.X, b.Y});
+        else if (G::madd_run(a, b.X, b.Y)) a = G::identity();
     } else {
         const Fq2 r = op == 4 ? G::mul2(a.X, b.X) : op == 5 ? G::sqr2(a.X) : G::inv2(a.X);
         a = G::identity();
