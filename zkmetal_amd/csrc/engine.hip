@@ -364,11 +364,15 @@ int32_t Engine::create(Engine** out) {
         return kGpuError;
     }
     {
-        bool ok = hipEventCreate(&e->ev_dec_) == hipSuccess;
+        // Between kernels of one stream: without the system-scope fence, whose
+        // cache write-back every next kernel would wait for.  (The last event,
+        // ev_[kNumStages], keeps it.)
+        bool ok = true;
+        for (hipEvent_t* ev : {&e->ev_dec_, &e->ev_m1_, &e->ev_r1_, &e->ev_tail_})
+            ok = ok && hipEventCreateWithFlags(ev, hipEventDisableSystemFence) == hipSuccess;
         for (uint32_t p = 0; p < kMaxParts; p++)
-            for (hipEvent_t* ev : {&e->ev_s0_[p], &e->ev_s1_[p], &e->ev_a0_[p], &e->ev_a1_[p], &e->ev_m1_[p],
-                                   &e->ev_r0_[p], &e->ev_r1_[p]})
-                ok = ok && hipEventCreate(ev) == hipSuccess;
+            for (hipEvent_t* ev : {&e->ev_s1_[p], &e->ev_a0_[p], &e->ev_a1_[p]})
+                ok = ok && hipEventCreateWithFlags(ev, hipEventDisableSystemFence) == hipSuccess;
         ok = ok && hipEventCreateWithFlags(&e->dep_fork_, hipEventDisableTiming) == hipSuccess;
         for (uint32_t p = 0; p < kMaxParts; p++)
             ok = ok && hipEventCreateWithFlags(&e->dep_sort_[p], hipEventDisableTiming) == hipSuccess;
@@ -393,10 +397,6 @@ int32_t Engine::create(Engine** out) {
             return kGpuError;
         }
     }
-    if (hipEventCreate(&e->ev_tail_) != hipSuccess) {
-        delete e;
-        return kGpuError;
-    }
     for (auto& ev : e->stage_ev_) {
         if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
             delete e;
@@ -418,16 +418,15 @@ Engine::~Engine() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     if (stream_sort_) (void)hipStreamSynchronize(stream_sort_);
     for (uint32_t p = 0; p < kMaxParts; p++)
-        for (hipEvent_t ev : {ev_s0_[p], ev_s1_[p], ev_a0_[p], ev_a1_[p], ev_m1_[p], ev_r0_[p], ev_r1_[p],
+        for (hipEvent_t ev : {ev_s1_[p], ev_a0_[p], ev_a1_[p],
                               dep_sort_[p]})
             if (ev) (void)hipEventDestroy(ev);
-    for (hipEvent_t ev : {ev_dec_, dep_fork_})
+    for (hipEvent_t ev : {ev_dec_, ev_m1_, ev_r1_, ev_tail_, dep_fork_})
         if (ev) (void)hipEventDestroy(ev);
     if (stream_sort_) (void)hipStreamDestroy(stream_sort_);
     if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
     for (auto& ev : ev_)
         if (ev) (void)hipEventDestroy(ev);
-    if (ev_tail_) (void)hipEventDestroy(ev_tail_);
     for (auto& ev : stage_ev_)
         if (ev) (void)hipEventDestroy(ev);
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -741,7 +740,10 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
     // while part p accumulates (the accumulation leaves registers and LDS for
     // the sort's workgroups).
     // Timing events are recorded only outside graph capture; the dependency
-    // events are part of a captured graph.
+    // events are part of a captured graph.  One event per boundary between
+    // stages, since each holds the next kernel up by ~4 us (a call outside a
+    // graph with two at each: 256 points 216 us, 8 MSMs of 2^16 884; 184 and
+    // 851 now).
     auto enqueue = [&](bool events) -> int32_t {
         auto rec = [&](hipEvent_t e, hipStream_t s) -> hipError_t { return events ? hipEventRecord(e, s) : hipSuccess; };
         // one part: everything on stream A (no cross-stream waits)
@@ -765,7 +767,6 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         for (uint32_t p = 0; p < P; p++) {
             const PlanPart& pt = pl.parts[p];
             const uint32_t ns_p = pt.seg_hi - pt.seg_lo;
-            ZK_TRY(rec(ev_s0_[p], S));
             if (pl.small_sort) {
                 launch_sort_small(d_segs, ns_p, (const uint16_t*)ws.digits, (uint32_t*)ws.segvalid, (uint16_t*)ws.keysB,
                                   (uint32_t*)ws.valsB, S);
@@ -788,7 +789,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         for (uint32_t p = 0; p < P; p++) {
             const PlanPart& pt = pl.parts[p];
             if (P > 1) ZK_TRY(hipStreamWaitEvent(st, dep_sort_[p], 0));
-            ZK_TRY(rec(ev_a0_[p], st));
+            if (P > 1) ZK_TRY(rec(ev_a0_[p], st));
             launch_accumulate(pl.curve, d_segs, d_seg_lane0, pt.seg_lo, pt.seg_hi - pt.seg_lo, d_msms,
                               (const uint32_t*)ws.segvalid, (const uint16_t*)ws.keysB, (const uint32_t*)ws.valsB,
                               d_table, pt.seg_hi - pt.seg_lo > kPlanSegs ? d_part_T + p : nullptr, pt.nbk, pt.lane_lo,
@@ -802,22 +803,20 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
         // merge after the last part instead of one after each keeps the
         // accumulations back to back.
         launch_merge_runs(pl.curve, (const uint32_t*)ws.recAk, ws.recAp, nrec, ws.buckets, d_err + 1, ws.lists, st);
-        ZK_TRY(rec(ev_m1_[0], st));
+        ZK_TRY(rec(ev_m1_, st));
         // the bucket reduction of all parts at once, after the last merge: as
         // a kernel beside the next part's accumulation it finds no free slots
         // (its waves need as many registers as the accumulation's) and
         // measured slower
-        ZK_TRY(rec(ev_r0_[0], st));
         const bool bits_end = !dev_tail && pl.curve != CurveId::Bn254G2;  // the planes go to the host
         launch_bucket_reduce(pl.curve, d_segs, d_seg_rcb0, d_seg_grp0, nseg, pl.rc_blocks, pl.G, pl.reduce_lanes,
                              ws.buckets, ws.rc, ws.bits, bits_end, bits_end ? back : CallBack{}, st);
         if (pl.curve == CurveId::Bn254G2) launch_g2_windows(d_segs, d_msms, nseg, ws.bits, hw, back, st);
-        ZK_TRY(rec(ev_r1_[0], st));
+        if (dev_tail || !ws.mapped) ZK_TRY(rec(ev_r1_, st));
         if (dev_tail) {
             launch_tail(pl.curve, d_segs, d_msms, nseg, nmsm, ws.bits, ws.wins, ws.res, norm, back, st);
-            ZK_TRY(rec(ev_tail_, st));
+            if (!ws.mapped) ZK_TRY(rec(ev_tail_, st));
         }
-        ZK_TRY(rec(ev_[kStCopyOut], st));
         if (ws.mapped) return kOk;
         ZK_TRY(hipMemcpyAsync(hw, dev_tail ? ws.res : ws.bits, back_bytes, hipMemcpyDeviceToHost, st));
         ZK_TRY(hipMemcpyAsync(hw + back_bytes, ws.err, 4 * 5, hipMemcpyDeviceToHost, st));
@@ -910,15 +909,17 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             (void)hipEventElapsedTime(&ms, a, b);
             return ms;
         };
+        hipEvent_t end = ev_[kNumStages], tail1 = ws.mapped ? end : ev_tail_;
+        hipEvent_t r1 = dev_tail || !ws.mapped ? ev_r1_ : end;
         timing_.stage_ms[kStDecompose] = span(ev_[0], ev_dec_);
         for (uint32_t p = 0; p < P; p++) {
-            timing_.stage_ms[kStSort] += span(ev_s0_[p], ev_s1_[p]);
-            timing_.stage_ms[kStAccumulate] += span(ev_a0_[p], ev_a1_[p]);
+            timing_.stage_ms[kStSort] += span(p ? ev_s1_[p - 1] : ev_dec_, ev_s1_[p]);
+            timing_.stage_ms[kStAccumulate] += span(P > 1 ? ev_a0_[p] : ev_s1_[p], ev_a1_[p]);
         }
-        timing_.stage_ms[kStMerge] = span(ev_a1_[P - 1], ev_m1_[0]);
-        timing_.stage_ms[kStReduce] = span(ev_r0_[0], ev_r1_[0]);
-        if (dev_tail) timing_.device_tail_ms = span(ev_r1_[0], ev_tail_);
-        timing_.stage_ms[kStCopyOut] = span(ev_[kStCopyOut], ev_[kNumStages]);
+        timing_.stage_ms[kStMerge] = span(ev_a1_[P - 1], ev_m1_);
+        timing_.stage_ms[kStReduce] = span(ev_m1_, r1);
+        if (dev_tail) timing_.device_tail_ms = span(r1, tail1);
+        if (!ws.mapped) timing_.stage_ms[kStCopyOut] = span(dev_tail ? tail1 : r1, end);
     }
     (void)hipEventElapsedTime(&timing_.device_ms, ev_[0], ev_[kNumStages]);
 

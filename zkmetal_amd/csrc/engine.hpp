@@ -435,14 +435,13 @@ class Engine {
     HostBuf stage_[kStageSlots];
     hipEvent_t stage_ev_[kStageSlots] = {};
     hipEvent_t ev_[kNumStages + 1] = {};
-    hipEvent_t ev_tail_ = nullptr;  // after the device tail, before the copy-out
-    // the part pipeline: the sort stream; timing events per part (sort,
-    // accumulation and merge starts and ends; the reduction uses slot 0) and
-    // the dependency events between the two streams
+    // the part pipeline: the sort stream; timing events (after the
+    // decomposition, the merge, the reduction, the device tail; per part after
+    // its sort and around its accumulation) and the dependency events between
+    // the two streams
     hipStream_t stream_sort_ = nullptr;
-    hipEvent_t ev_dec_ = nullptr;
-    hipEvent_t ev_s0_[kMaxParts] = {}, ev_s1_[kMaxParts] = {}, ev_a0_[kMaxParts] = {},
-               ev_a1_[kMaxParts] = {}, ev_m1_[kMaxParts] = {}, ev_r0_[kMaxParts] = {}, ev_r1_[kMaxParts] = {};
+    hipEvent_t ev_dec_ = nullptr, ev_m1_ = nullptr, ev_r1_ = nullptr, ev_tail_ = nullptr;
+    hipEvent_t ev_s1_[kMaxParts] = {}, ev_a0_[kMaxParts] = {}, ev_a1_[kMaxParts] = {};
     hipEvent_t dep_fork_ = nullptr;
     hipEvent_t dep_sort_[kMaxParts] = {};
     uint32_t parts_req_ = 0;  // 0: default_parts
