@@ -957,6 +957,14 @@ __global__ __launch_bounds__(256) void k_lane_plan(const SegDesc* __restrict__ s
     }
 }
 
+// Bound by the multiply-adds of the mixed additions (G1: 1,467 of 2,032 VALU
+// instructions) at the clock the power limit leaves, 1.95 GHz: 2^25 entries
+// 2.40 ms at 81% of the issue slots (2.48 before the shorter reductions, the
+// fixed chains and the run starts by assignment).  A run's first base is
+// assigned, under the execution mask, instead of added to a placeholder and
+// selected: no registers for the base past the addition's first products, so
+// 167 registers and three waves per SIMD, which cover each other's waits on
+// the gathers (13% of a wave's cycles).
 template <class C>
 __global__ __launch_bounds__(256) void k_accumulate(
     const SegDesc* __restrict__ segs, const uint64_t* __restrict__ seg_lane0, uint32_t seg_lo, uint32_t nseg,

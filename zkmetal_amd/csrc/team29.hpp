@@ -5,8 +5,8 @@
 // chains of dependent additions with too few of them to fill the chip.  One
 // lane per addition issues its ~3,300 instructions one after another -- 7.5 us
 // per addition whether or not the wave's other lanes have work.  A team
-// computes the independent products of one level in different lanes: ~1,100
-// instructions, 2 us per addition (MI355X, one wave per SIMD).  In lanes spent
+// computes the independent products of one level in different lanes: ~1,200
+// instructions, 2.6 us per addition (MI355X, one wave per SIMD).  In lanes spent
 // it costs 16 products where one lane needs 14, so it also holds its own where
 // the chip is full.
 //
@@ -21,7 +21,8 @@
 //
 // Bounds, in multiples of p: points in and out X < 6.5p, Y < 4p (G2: 3.5p),
 // ZZ, ZZZ < 2p, limbs normalised; a product of operands a, b is below
-// ab/169 + 1 (G1), (ab + 10a)/169 + 1 (G2, b < 10): below 1.5 unless noted.
+// ab/169 + 1 (G1), (ab + 10a)/169 + 1 (G2, b < 10), and 2^-29 (Arith::q_m):
+// below 1.5 unless noted.
 #pragma once
 #include "curve29.hpp"
 #include "curve_g2.hpp"
