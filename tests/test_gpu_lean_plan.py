@@ -49,3 +49,23 @@ def test_capped_resident_call():
         assert e.msm_batch_resident(ds, [n]) == want
     finally:
         e.close()
+
+
+def test_capped_call_of_many_lanes():
+    # a cap that leaves no room for the third wave's merge records
+    n = 1 << 17
+    gen = zk.MetalMSM()
+    e = zk.MetalMSM()
+    try:
+        gen.srs_generate(SEED, n)
+        pts, sc = gen.srs_download(n), zk.gen_scalars(SEED + 3, n, 0)
+        want = e.msm(pts, sc)
+        need = e.workspace_bytes()
+        e.close()
+        e = zk.MetalMSM()
+        e.set_workspace_limit(need - (8 << 20))
+        assert e.msm(pts, sc) == want
+        assert e.workspace_bytes() <= need - (8 << 20)
+    finally:
+        e.close()
+        gen.close()

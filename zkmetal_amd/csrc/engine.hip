@@ -281,12 +281,12 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
         }
         const uint64_t ns_p = pt.seg_hi - pt.seg_lo;
         const uint64_t half_bucket = ent / (2 * std::max<uint64_t>(1, bk));
-        uint64_t cap = lane_cap > 2ull * ns_p + 64 ? lane_cap - ns_p : std::max<uint64_t>(lane_cap / 2, 64);
         // lanes of fewer than 8 entries leave more partial sums to merge than
         // a third wave per SIMD hides, so such a call fills two (2^16 points: 344
         // against 352 us); 8 MSMs of 2^16, 28 entries a lane, take 840 us with
-        // three and 853 with two.  The G2 kernel runs one wave per SIMD anyway.
-        if (cv != CurveId::Bn254G2 && ent < 8 * cap) cap = cap * 2 / 3;
+        // three and 853 with two
+        const uint64_t lc = ent < 8 * lane_cap ? std::min(lane_cap, kTwoWaveLanes) : lane_cap;
+        const uint64_t cap = lc > 2ull * ns_p + 64 ? lc - ns_p : std::max<uint64_t>(lc / 2, 64);
         pt.T = (uint32_t)std::max<uint64_t>(std::max<uint64_t>(4, std::min<uint64_t>(32, half_bucket)),
                                             (ent + cap - 1) / cap);
         pt.entries = ent;
@@ -1193,12 +1193,13 @@ uint32_t Engine::shift_floor(const std::vector<uint32_t>& ns, bool lean) const {
 
 // The call's plan: the tuned window widths and the shift rule; where a cap on
 // the engine's memory leaves no room for it, the widths and the rule that need
-// the fewest buckets (lean).  other: bytes the call will allocate besides.
+// the fewest buckets, and two accumulation waves' merge records (lean).  other: bytes the call will allocate besides.
 int32_t Engine::plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
                           CurveId cv, uint64_t shift_stride, uint64_t other) {
     const uint32_t nmsm = (uint32_t)ns.size();
     auto make = [&](bool lean) {
-        return make_plan(ns.data(), t0.data(), nmsm, window_bits_for(ns, cv, lean).data(), pl, form, lane_cap(cv), cv,
+        const uint64_t lanes = lean ? std::min(lane_cap(cv), kTwoWaveLanes) : lane_cap(cv);
+        return make_plan(ns.data(), t0.data(), nmsm, window_bits_for(ns, cv, lean).data(), pl, form, lanes, cv,
                          parts_req_, shift_stride, kShiftC, shift_floor(ns, lean), schedule(nmsm));
     };
     const int32_t rc = make(false);

@@ -105,6 +105,8 @@ constexpr int kSortItems = 8;
 constexpr int kSortTile = kSortThreads * kSortItems;
 // one-block sort of a whole segment (k_sort_small): entries and buckets at most
 constexpr uint32_t kSmallSortLen = 16384, kSmallSortBuckets = 4096;
+// accumulation lanes of two waves per SIMD (256 CUs x 4 SIMDs x 2 x 64)
+constexpr uint64_t kTwoWaveLanes = 1u << 17;
 // segments of a part up to which k_accumulate plans its lanes itself (one per
 // thread of a block)
 constexpr uint32_t kPlanSegs = 256;
