@@ -4,9 +4,12 @@
 // The formulas are those of the G1 kernels (madd-2008-s, add-2008-s,
 // dbl-2008-s-1) with Fp2 coefficients; b' enters none of them.
 //
-// Bounds: every Fp2 value held between operations has both components below
-// 2p with normalised limbs (so fq_is_zero2 decides == 0, and sums of two stay
-// below 4p as multiplicands).  Each operation restores that with conditional
+// Bounds, per component and with normalised limbs.  A stored point (bucket,
+// merge record, row or column sum) has X < 6.5p, Y < 3.5p, ZZ, ZZZ < 2p: what
+// the lane teams leave (team29.hpp) and what every operation on stored points
+// here takes.  The accumulator of madd_run, and every other Fp2 value held
+// between operations, is below 2p (so fq_is_zero2 decides == 0, and sums of
+// two stay below 4p as multiplicands).  Each operation restores that with conditional
 // subtractions: a product of components < 4p is < 1.1p; mul2's c0 = t0 - t1
 // + 2p < 3.1p and c1 = t2 - (t0 + t1) + 3p < 4.1p, sub2 = a - b + 2p < 4p,
 // 2a < 4p, 3a < 6p are brought under 2p by one subtraction of 2p (below 4p)
@@ -134,11 +137,13 @@ struct G2Arith {
         return r;
     }
 
-    // 2 P; the identity stays the identity (ZZ3 = V ZZ = 0)
+    // 2 P for a stored point (dbl_core's products want X and Y below 2p); the
+    // identity stays the identity (ZZ3 = V ZZ = 0)
     static __device__ __forceinline__ QXyzz2 dbl(const QXyzz2& p) {
         QXyzz2 r;
         Fq2 V, W;
-        dbl_core(p.X, p.Y, r.X, r.Y, V, W);
+        const Fq2 X{red8(p.X.c0), red8(p.X.c1)}, Y{red4(p.Y.c0), red4(p.Y.c1)};
+        dbl_core(X, Y, r.X, r.Y, V, W);
         r.ZZ = mul2(V, p.ZZ);
         r.ZZZ = mul2(W, p.ZZZ);
         return r;
@@ -197,8 +202,9 @@ struct G2Arith {
         return cancel;
     }
 
-    // acc += q (both XYZZ, components < 2p), on the merged-reduction products
-    // of madd_run with the same bounds (U1, S1 < 1.1p)
+    // acc += q (both stored points), on the merged-reduction products of
+    // madd_run: U1, S1 < 1.2p, P, R < 3.2p, the rest as there.  Out: components
+    // < 2p, or q as it was where acc is the identity.
     static __device__ __forceinline__ void add(QXyzz2& acc, const QXyzz2& q) {
         const bool p_id = is_id(acc);
         const bool q_id = is_id(q);
