@@ -348,8 +348,8 @@ __device__ __forceinline__ uint32_t window_bits256(const uint32_t k[8], uint32_t
 // over 255 bits, the scalar reduced mod r (kModR, BN254 G2) or mod p
 // (Grumpkin).  Window w's entries: segment seg0 + w / wps, at local window
 // v = w % wps, i.e. tiles v * ntw + tin and positions v * ntw * kSortTile +
-// (entry) of the segment, ntw = the window's tiles; a window-shifted MSM
-// (wps > 1) pads each window to whole tiles with "no bucket" digits.
+// (entry) of the segment, ntw = the window's tiles; a window-shifted MSM pads
+// each window to whole tiles with "no bucket" digits.
 // A block has kThreads threads.  Each walks its scalars one after another, a
 // chain of ~700 instructions each, so a call too small to fill the chip takes
 // 1024 threads, 2 scalars deep (2^16 points: 43 us with 256 threads, 27 with
@@ -420,8 +420,8 @@ __global__ __launch_bounds__(kDecThreads) void k_decompose(const MsmDesc* __rest
         const uint64_t i = (uint64_t)tin * (kSortTile / EPS) + (uint64_t)r * kDecThreads + threadIdx.x;
         const bool live = i < m.n;
         // past the MSM's scalars: done, unless its windows are padded to whole
-        // tiles (window-shifted), whose tails take "no bucket" digits
-        if (!live && m.wps == 1) break;
+        // tiles, whose tails take "no bucket" digits
+        if (!live && !padded(m)) break;
         uint32_t k[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         if (live) {
             const uint64_t g = m.scalar0 + i;

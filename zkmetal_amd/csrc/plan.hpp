@@ -61,6 +61,9 @@ struct MsmDesc {
     uint32_t wps;      // windows per segment (1 plain)
     uint32_t cstep;    // doublings between consecutive segments' sums (c plain, 0 shifted)
 };
+// The MSM's windows are padded to whole sort tiles: window-shifted, whatever
+// the windows per segment (one, where eight parts share one MSM).
+constexpr bool padded(const MsmDesc& m) { return m.cstep == 0; }
 
 struct SegDesc {
     uint64_t ent0;    // first entry in the digit / sorted arrays
