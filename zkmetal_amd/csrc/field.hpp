@@ -65,14 +65,38 @@ __device__ __forceinline__ Fp fp_zero() {
     return r;
 }
 
-// acc(96 bit: lo64, hi32) += x * y
-__device__ __forceinline__ void mac(uint64_t& lo, uint32_t& hi, uint32_t x, uint32_t y) {
-    uint64_t c;
-    asm("v_mad_u64_u32 %0, %1, %3, %4, %0\n\t"
-        "v_addc_co_u32_e64 %2, %1, 0, %2, %1"
-        : "+v"(lo), "=&s"(c), "+v"(hi)
-        : "v"(x), "v"(y));
-}
+// acc(96 bit: lo64, hi32) += one, two or three products x y, the multiply-adds'
+// carries straight into the third word: two instructions a product.  Between
+// the instruction that writes a carry and the one that reads it gfx950 wants
+// two others; the compiler does not look inside, so the blocks keep them apart
+// (three products need no wait).  ZK_MACS(NAME, Y): the y in registers of
+// constraint Y, "v" or (uniform) "s".
+#define ZK_MAD(c, x, y) "v_mad_u64_u32 %0, %" #c ", %" #x ", %" #y ", %0\n\t"
+#define ZK_ADC(c) "v_addc_co_u32_e64 %1, %" #c ", 0, %1, %" #c "\n\t"
+#define ZK_MACS(NAME, Y)                                                                                          \
+    __device__ __forceinline__ void NAME(uint64_t& lo, uint32_t& hi, uint32_t x, uint32_t y) {                    \
+        uint64_t c;                                                                                               \
+        asm(ZK_MAD(2, 3, 4) "s_nop 1\n\t" ZK_ADC(2) : "+&v"(lo), "+v"(hi), "=&s"(c) : "v"(x), Y(y));              \
+    }                                                                                                             \
+    __device__ __forceinline__ void NAME(uint64_t& lo, uint32_t& hi, uint32_t x0, uint32_t y0, uint32_t x1,       \
+                                         uint32_t y1) {                                                           \
+        uint64_t c0, c1;                                                                                          \
+        asm(ZK_MAD(2, 4, 5) ZK_MAD(3, 6, 7) "s_nop 0\n\t" ZK_ADC(2) ZK_ADC(3)                                     \
+            : "+&v"(lo), "+v"(hi), "=&s"(c0), "=&s"(c1)                                                           \
+            : "v"(x0), Y(y0), "v"(x1), Y(y1));                                                                    \
+    }                                                                                                             \
+    __device__ __forceinline__ void NAME(uint64_t& lo, uint32_t& hi, uint32_t x0, uint32_t y0, uint32_t x1,       \
+                                         uint32_t y1, uint32_t x2, uint32_t y2) {                                 \
+        uint64_t c0, c1, c2;                                                                                      \
+        asm(ZK_MAD(2, 5, 6) ZK_MAD(3, 7, 8) ZK_MAD(4, 9, 10) ZK_ADC(2) ZK_ADC(3) ZK_ADC(4)                        \
+            : "+&v"(lo), "+v"(hi), "=&s"(c0), "=&s"(c1), "=&s"(c2)                                                \
+            : "v"(x0), Y(y0), "v"(x1), Y(y1), "v"(x2), Y(y2));                                                    \
+    }
+ZK_MACS(mac, "v")
+ZK_MACS(mac_uniform, "s")
+#undef ZK_MACS
+#undef ZK_MAD
+#undef ZK_ADC
 
 __device__ __forceinline__ void shift32(uint64_t& lo, uint32_t& hi) {
     lo = (lo >> 32) | ((uint64_t)hi << 32);
@@ -100,8 +124,7 @@ __device__ __forceinline__ Fp fp_mul(const Fp& a, const Fp& b) {
     for (int i = 0; i < 8; i++) {
 #pragma unroll
         for (int j = 0; j < i; j++) {
-            mac(lo, hi, a.v[j], b.v[i - j]);
-            mac(lo, hi, m[j], p_limb(i - j));
+            mac(lo, hi, a.v[j], b.v[i - j], m[j], p_limb(i - j));
         }
         mac(lo, hi, a.v[i], b.v[0]);
         m[i] = (uint32_t)lo * ZK_PINV32;
@@ -112,8 +135,7 @@ __device__ __forceinline__ Fp fp_mul(const Fp& a, const Fp& b) {
     for (int i = 8; i < 15; i++) {
 #pragma unroll
         for (int j = i - 7; j < 8; j++) {
-            mac(lo, hi, a.v[j], b.v[i - j]);
-            mac(lo, hi, m[j], p_limb(i - j));
+            mac(lo, hi, a.v[j], b.v[i - j], m[j], p_limb(i - j));
         }
         t.v[i - 8] = (uint32_t)lo;
         shift32(lo, hi);

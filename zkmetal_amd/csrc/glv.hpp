@@ -105,15 +105,6 @@ struct GlvSplit {
     bool neg1, neg2;
 };
 
-// hi:lo += a * b (b uniform): the multiply-add's carry goes straight into the
-// third word, two instructions a product where the compiler's rows take four
-__device__ __forceinline__ void mac_uniform(uint64_t& lo, uint32_t& hi, uint32_t a, uint32_t b) {
-    asm("v_mad_u64_u32 %0, vcc, %2, %3, %0\n\tv_addc_co_u32 %1, vcc, 0, %1, vcc"
-        : "+v"(lo), "+v"(hi)
-        : "v"(a), "s"(b)
-        : "vcc");
-}
-
 // Words FROM.. of a * b (NA and NB words, b uniform), column by column; the
 // products of lower columns are left out, so out[FROM] is low by less than
 // min(NA, NB) carries into the column above, which is why the caller starts
@@ -124,12 +115,18 @@ __device__ __forceinline__ void mul_columns(const uint32_t* a, const uint32_t* b
 #pragma unroll
     for (int q = FROM; q <= LAST; q++) {
         uint32_t hi = 0;
+        const int end = q < NA ? q + 1 : NA;  // i < end, q - i < NB
+        int i = q < NB ? 0 : q - NB + 1;
+        if (q < LAST) {
 #pragma unroll
-        for (int i = 0; i < NA; i++)
-            if (q - i >= 0 && q - i < NB) {
-                if (q < LAST) mac_uniform(lo, hi, a[i], b[q - i]);
-                else lo = (uint32_t)lo + a[i] * b[q - i];
-            }
+            for (; i + 3 <= end; i += 3)
+                mac_uniform(lo, hi, a[i], b[q - i], a[i + 1], b[q - i - 1], a[i + 2], b[q - i - 2]);
+            if (i + 2 == end) mac_uniform(lo, hi, a[i], b[q - i], a[i + 1], b[q - i - 1]);
+            else if (i + 1 == end) mac_uniform(lo, hi, a[i], b[q - i]);
+        } else {
+#pragma unroll
+            for (; i < end; i++) lo = (uint32_t)lo + a[i] * b[q - i];
+        }
         out[q] = (uint32_t)lo;
         lo = (lo >> 32) | ((uint64_t)hi << 32);
     }
