@@ -1,7 +1,8 @@
-"""The inline assembly's carries: an instruction that reads a carry has at
-least two others, or as many wait states, after the vector instruction that
-wrote it (the distance the compiler keeps on gfx950 between its own), within
-the same block."""
+"""The inline assembly's operands.  Carries: an instruction that reads a carry
+has at least two others, or as many wait states, after the vector instruction
+that wrote it (the distance the compiler keeps on gfx950 between its own),
+within the same block.  Registers: an operand that a block writes before it
+has read all the others is early clobber, so that no other shares its place."""
 import glob
 import os
 import re
@@ -32,7 +33,8 @@ def blocks(text):
             part = re.sub(r"\b(%s)\(([^)]*)\)" % name, expand, part[:4000])
         head = re.match(r"(?:\s*\"(?:[^\"\\]|\\.)*\")*", part).group(0)
         code = "".join(re.findall(r"\"((?:[^\"\\]|\\.)*)\"", head))
-        yield [i.strip() for i in re.split(r"\\n|\\t", code) if i.strip()]
+        outs = re.findall(r"(?:\"([^\"]*)\"|\bY)\s*\(", part[len(head):].split(";")[0])
+        yield [i.strip() for i in re.split(r"\\n|\\t", code) if i.strip()], outs
 
 
 def short_waits(block):
@@ -54,12 +56,30 @@ def short_waits(block):
 
 @pytest.mark.parametrize("name", sorted(os.path.basename(p) for p in glob.glob(os.path.join(CSRC, "*.h*"))))
 def test_carries_are_read_in_time(name):
-    for block in blocks(open(os.path.join(CSRC, name)).read()):
+    for block, _ in blocks(open(os.path.join(CSRC, name)).read()):
         assert not short_waits(block), block
 
 
+def shared(block, constraints):
+    """operands written while others are still to be read, not early clobber"""
+    out = []
+    for k, ins in enumerate(block):
+        for d in re.findall(r"^v_\S+ %(\d+),", ins):
+            later = {int(x) for i in block[k + 1:] for x in re.findall(r"%(\d+)", i.partition(",")[2])}
+            inputs = {x for x in later if x < len(constraints) and not constraints[x].startswith(("+", "="))}
+            if inputs and "&" not in constraints[int(d)]:
+                out.append(ins)
+    return out
+
+
+@pytest.mark.parametrize("name", sorted(os.path.basename(p) for p in glob.glob(os.path.join(CSRC, "*.h*"))))
+def test_written_operands_share_no_register(name):
+    for block, constraints in blocks(open(os.path.join(CSRC, name)).read()):
+        assert not shared(block, constraints), (block, constraints)
+
+
 def test_the_check_sees_the_products():
-    found = [b for b in blocks(open(os.path.join(CSRC, "field.hpp")).read()) if any("addc" in i for i in b)]
+    found = [b for b, _ in blocks(open(os.path.join(CSRC, "field.hpp")).read()) if any("addc" in i for i in b)]
     assert sorted(sum("v_mad_u64_u32" in i for i in b) for b in found) == [1, 2, 3]
     assert short_waits(["v_mad_u64_u32 %0, vcc, %2, %3, %0", "v_addc_co_u32 %1, vcc, 0, %1, vcc"])
     assert short_waits(["v_mad_u64_u32 %0, %2, %3, %4, %0", "s_nop 0", "v_addc_co_u32_e64 %1, %2, 0, %1, %2"])

@@ -178,11 +178,12 @@ __device__ __forceinline__ void qmac(uint64_t& acc, uint32_t x, uint32_t y) {
 // s_setpc through registers whose scalar load may still be in flight.
 // 2^22 points: 5.94 -> 5.84 ms per call with the shorter reductions (q_m),
 // 2,080 -> 1,930 instructions and 186 -> 178 registers per mixed addition.
+// (Early clobber: s1 is written before the block's last operands are read.)
 #define ZQ_MAD(d, x, y) "v_mad_u64_u32 %" #d ", vcc, %" #x ", %" #y ", %" #d "\n\t"
 template <bool kFixed>
 __device__ __forceinline__ void qmac2(uint64_t& s1, uint64_t& s2, uint32_t x1, uint32_t y1, uint32_t x2, uint32_t y2) {
     if constexpr (kFixed) {
-        asm(ZQ_MAD(0, 2, 3) ZQ_MAD(1, 4, 5) : "+v"(s1), "+v"(s2) : "v"(x1), "v"(y1), "v"(x2), "v"(y2) : "vcc");
+        asm(ZQ_MAD(0, 2, 3) ZQ_MAD(1, 4, 5) : "+&v"(s1), "+&v"(s2) : "v"(x1), "v"(y1), "v"(x2), "v"(y2) : "vcc");
     } else {
         qmac(s1, x1, y1);
         qmac(s2, x2, y2);
@@ -192,7 +193,7 @@ __device__ __forceinline__ void qmac2(uint64_t& s1, uint64_t& s2, uint32_t x1, u
 template <bool kFixed>
 __device__ __forceinline__ void qred2(uint64_t& s1, uint64_t& s2, uint32_t m1, uint32_t m2, uint32_t n) {
     if constexpr (kFixed) {
-        asm(ZQ_MAD(0, 2, 4) ZQ_MAD(1, 3, 4) : "+v"(s1), "+v"(s2) : "v"(m1), "v"(m2), "s"(n) : "vcc");
+        asm(ZQ_MAD(0, 2, 4) ZQ_MAD(1, 3, 4) : "+&v"(s1), "+&v"(s2) : "v"(m1), "v"(m2), "s"(n) : "vcc");
     } else {
         qmac(s1, m1, n);
         qmac(s2, m2, n);
@@ -204,7 +205,7 @@ __device__ __forceinline__ void qmac4(uint64_t& s1, uint64_t& s2, uint32_t x1, u
                                       uint32_t m1, uint32_t m2, uint32_t n) {
     if constexpr (kFixed) {
         asm(ZQ_MAD(0, 2, 3) ZQ_MAD(1, 4, 5) ZQ_MAD(0, 6, 8) ZQ_MAD(1, 7, 8)
-            : "+v"(s1), "+v"(s2)
+            : "+&v"(s1), "+&v"(s2)
             : "v"(x1), "v"(y1), "v"(x2), "v"(y2), "v"(m1), "v"(m2), "s"(n)
             : "vcc");
     } else {

@@ -1377,8 +1377,8 @@ __global__ __launch_bounds__(256) void k_probe(int mode, uint32_t iters, uint64_
                 "v_mad_u64_u32 %5, s[0:1], %13, %16, %5\n"
                 "v_mad_u64_u32 %6, s[0:1], %14, %16, %6\n"
                 "v_mad_u64_u32 %7, s[0:1], %15, %16, %7\n"
-                : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]),
-                  "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7])
+                : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]),
+                  "+&v"(acc[5]), "+&v"(acc[6]), "+&v"(acc[7])
                 : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]),
                   "v"(x[7]), "v"(y)
                 : "s0", "s1");
