@@ -2,12 +2,7 @@
 its blocks and scalars over the planner's own plans (a small C++ program on the
 library's make_plan), plain and window-shifted, whole and split into up to
 eight parts, at sizes that do and do not fill their last sort tile."""
-import os
-import subprocess
-
-import zkmetal_amd as zk
-
-CSRC = os.path.join(os.path.dirname(zk.LIB_PATH), "csrc")
+from plan_program import run_cpp
 
 SOURCE = r"""
 #include <stdio.h>
@@ -55,12 +50,4 @@ int main() {
 
 
 def test_every_sorted_position_is_written(tmp_path):
-    src, exe = tmp_path / "walk.cpp", tmp_path / "walk"
-    src.write_text(SOURCE)
-    libdir = os.path.dirname(zk.LIB_PATH)
-    r = subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I", CSRC,
-                        str(src), "-o", str(exe), zk.LIB_PATH, f"-Wl,-rpath,{libdir}", "-L/opt/rocm/lib",
-                        "-Wl,-rpath,/opt/rocm/lib"], capture_output=True, text=True)
-    assert r.returncode == 0, r.stderr
-    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
-    assert r.returncode == 0, r.stdout + r.stderr
+    run_cpp(tmp_path, SOURCE)

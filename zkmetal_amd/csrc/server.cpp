@@ -7,15 +7,33 @@
 #include <algorithm>
 #include <cmath>
 
+#include "tuned_gfx950.hpp"
+
 namespace zk {
 
-// Device bytes a request may occupy while it runs: scalars, digit words,
-// two sorted key/value copies and merge records (~300 B per point at the
-// default window widths) plus its buckets.
+// Device bytes a request may occupy while it runs, alone or in a batch, at the
+// built-in window widths: the larger of its plans (plain at either width,
+// window-shifted into one set of 2^(kShiftC - 1) buckets).  Per entry: a digit
+// word, two sorted key/value copies, the tile histograms; per accumulation
+// lane two merge records and their share of the merge's lists.  A lane takes
+// at least four entries, and each part of a call at most a resident round of
+// lanes (a request of more than half a part's entries may share its call with
+// as much again).
 uint64_t Server::footprint(uint32_t n) {
-    const uint32_t c = default_window_bits(n);
-    const uint64_t w = (128 + c - 1) / c;
-    return (uint64_t)n * 32 + 2ull * n * w * 16 + w * (1ull << (c - 1)) * kBucketBytes + (1u << 20);
+    uint32_t cls = 0;
+    while ((1ull << cls) < n) cls++;
+    const uint64_t tiles = (2ull * n + kSortTile - 1) / kSortTile;  // of one window
+    uint64_t entries = 0, buckets = 0;
+    auto plan = [&](uint64_t c, bool shifted) {
+        const uint64_t w = (128 + c - 1) / c;
+        entries = std::max<uint64_t>(entries, shifted ? w * tiles * kSortTile : w * 2 * n);
+        buckets = std::max<uint64_t>(buckets, (shifted ? 1 : w) << (c - 1));
+    };
+    for (uint32_t c : {kTunedPlain[cls], kTunedBatch[cls]}) plan(c ? c : default_window_bits(n), false);
+    plan(Engine::kShiftC, true);
+    constexpr uint64_t kRound = 3 * kTwoWaveLanes / 2;  // three waves per SIMD
+    const uint64_t lanes = std::min(entries / 4, default_parts(2 * entries) * kRound) + kMaxWindows;
+    return (uint64_t)n * 32 + entries * 15 + buckets * kBucketBytes + lanes * 2 * (kBucketBytes + 6) + (1u << 20);
 }
 
 int32_t Server::create(Engine* owner, const ServerConfig& cfg, Server** out) {
