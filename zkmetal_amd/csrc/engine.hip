@@ -640,30 +640,23 @@ WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
     return z;
 }
 
+// the device buffers of a call and the bytes it needs of each (0: not used)
+std::array<Engine::BufSize, 17> Engine::call_buffers(const WsSizes& z, bool dev_tail, CurveId cv) {
+    const bool dev_bits = dev_tail || cv == CurveId::Bn254G2;  // else the planes go to host memory
+    return {{{&desc_, z.desc}, {&digits_, z.digits}, {&keysA_, z.keys}, {&valsA_, z.vals}, {&keysB_, z.keys},
+             {&valsB_, z.vals}, {&hist_, z.hist}, {&part_, z.part}, {&segvalid_, z.segvalid},
+             {&buckets_, z.buckets}, {&recAk_, z.rec_keys}, {&recAp_, z.rec_pts}, {&lists_, z.lists}, {&rc_, z.rc},
+             {&winsum_, dev_bits ? z.bits : 0}, {&wins_, z.wins}, {&err_, z.err}}};
+}
+
 int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, uint64_t table_n,
                     uint8_t* out96) {
     // window combine on the device (graph mode, large batches) or the host
     const bool dev_tail = device_tail(pl);
     const WsSizes z = ws_sizes(pl, dev_tail);
-    ZK_ALLOC(desc_, z.desc);
-    ZK_ALLOC(hdesc_, z.desc);
-    ZK_ALLOC(digits_, z.digits);
-    ZK_ALLOC(keysA_, z.keys);
-    ZK_ALLOC(valsA_, z.vals);
-    ZK_ALLOC(keysB_, z.keys);
-    ZK_ALLOC(valsB_, z.vals);
-    ZK_ALLOC(hist_, z.hist);
-    ZK_ALLOC(part_, z.part);
-    ZK_ALLOC(segvalid_, z.segvalid);
-    ZK_ALLOC(buckets_, z.buckets);
-    ZK_ALLOC(recAk_, z.rec_keys);
-    ZK_ALLOC(recAp_, z.rec_pts);
-    ZK_ALLOC(lists_, z.lists);
-    ZK_ALLOC(rc_, z.rc);
     const bool dev_bits = dev_tail || pl.curve == CurveId::Bn254G2;
-    if (dev_bits) ZK_ALLOC(winsum_, z.bits);
-    if (dev_tail) ZK_ALLOC(wins_, z.wins);
-    ZK_ALLOC(err_, z.err);
+    for (const BufSize& b : call_buffers(z, dev_tail, pl.curve)) ZK_ALLOC(*b.buf, b.bytes);
+    ZK_ALLOC(hdesc_, z.desc);
     ZK_ALLOC(hwin_, z.host);
     Workspace ws;
     ws.desc = (uint8_t*)desc_.p;
@@ -1204,13 +1197,9 @@ int32_t Engine::plan_call(const std::vector<uint32_t>& ns, const std::vector<uin
     };
     const int32_t rc = make(false);
     if (rc != kOk || !ws_.limit) return rc;
-    const WsSizes z = ws_sizes(pl, device_tail(pl));
-    const uint64_t need = other + desc_.growth(z.desc) + digits_.growth(z.digits) + keysA_.growth(z.keys) +
-                          valsA_.growth(z.vals) + keysB_.growth(z.keys) + valsB_.growth(z.vals) +
-                          hist_.growth(z.hist) + part_.growth(z.part) + segvalid_.growth(z.segvalid) +
-                          buckets_.growth(z.buckets) + recAk_.growth(z.rec_keys) + recAp_.growth(z.rec_pts) +
-                          lists_.growth(z.lists) + rc_.growth(z.rc) + winsum_.growth(z.bits) +
-                          wins_.growth(z.wins) + err_.growth(z.err);
+    const bool dev_tail = device_tail(pl);
+    uint64_t need = other;
+    for (const BufSize& b : call_buffers(ws_sizes(pl, dev_tail), dev_tail, cv)) need += b.buf->growth(b.bytes);
     return ws_.used + need > ws_.limit ? make(true) : rc;
 }
 

@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <mutex>
 #include <string>
@@ -399,6 +400,11 @@ class Engine {
     // after the table's bases are written: the shifted copies, then wait
     int32_t srs_finish(uint64_t n, uint64_t stride);
     uint64_t plan_shift(const void* table, uint64_t shift_stride) const;
+    struct BufSize {
+        DevBuf* buf;
+        uint64_t bytes;
+    };
+    std::array<BufSize, 17> call_buffers(const WsSizes& z, bool dev_tail, CurveId cv);
     int32_t plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
                       CurveId cv, uint64_t shift_stride, uint64_t other);
     // make_plan's shift_floor for a call: in calls of up to kShiftAlwaysMsms
