@@ -370,6 +370,9 @@ ZkMetalStatus zkmsm_test_xyzz(ZkMetalMSMEngine engine, int32_t op, const uint8_t
  * 4: p.X * q.X, 5: p.X^2, 6: 1 / p.X; 7: p + q, 8: 2p by lane teams. */
 ZkMetalStatus zkmsm_test_g2(ZkMetalMSMEngine engine, int32_t op, const uint8_t* p,
                             const uint8_t* q, uint8_t* out, uint32_t n);
+/* device allocations of this engine that would take its workspace past bytes
+ * fail as if the device were full (0: none do) */
+ZkMetalStatus zkmsm_test_device_memory(ZkMetalMSMEngine engine, uint64_t bytes);
 /* GLV split of n scalars: out n x 48 B = k1 (16 B), k2 (16 B), neg1, neg2 (u32). */
 ZkMetalStatus zkmsm_test_glv(ZkMetalMSMEngine engine, const uint8_t* scalars, uint8_t* out,
                              uint32_t n);

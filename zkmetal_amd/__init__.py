@@ -128,6 +128,7 @@ def lib():
         "zkmsm_bn254_g2_msm_batch": (i32, [vp, vp, vp, vp, u32, vp]),
         "zkmsm_bn254_g2_msm_batch_device": (i32, [vp, vp, vp, vp, u32, vp]),
         "zkmsm_bn254_g2_points_generate": (i32, [vp, u64, u32, vp]),
+        "zkmsm_test_device_memory": (i32, [vp, u64]),
         "zkmsm_test_g2": (i32, [vp, i32, vp, vp, vp, u32]),
         "zkmsm_srs_detect_hits": (u64, [vp]),
         "zkmsm_inner_product_msm": (i32, [vp, vp, vp, u32, vp, u32, vp]),

@@ -559,6 +559,14 @@ ZkMetalStatus zkmsm_set_workspace_limit(ZkMetalMSMEngine engine, uint64_t bytes)
     return ZKMETAL_SUCCESS;
 }
 
+ZkMetalStatus zkmsm_test_device_memory(ZkMetalMSMEngine engine, uint64_t bytes) {
+    Engine* e = as_engine(engine);
+    if (!e) return ZKMETAL_ERR_INVALID_INPUT;
+    std::lock_guard<std::mutex> lk(e->mutex());
+    e->test_device_memory(bytes);
+    return ZKMETAL_SUCCESS;
+}
+
 uint64_t zkmsm_workspace_bytes(ZkMetalMSMEngine engine) {
     Engine* e = as_engine(engine);
     if (!e) return 0;

@@ -38,6 +38,7 @@ hipError_t DevBuf::ensure(size_t bytes) {
     size_t want = std::max<size_t>(bytes, 256);
     if (acct && acct->limit && acct->used - cap + want > acct->limit) return hipErrorOutOfMemory;
     release();
+    if (acct && acct->device && acct->used + want > acct->device) return hipErrorOutOfMemory;
     hipError_t e = hipMalloc(&p, want);
     if (e != hipSuccess) {
         p = nullptr;
@@ -1084,10 +1085,8 @@ int32_t Engine::msm_batch_host(const uint8_t* points, const uint8_t* scalars,
     }
     Plan pl;
     rc = plan_call(ns, t0, pl, 0, cv, 0,
-                   pts_in_.growth(total * input_point_bytes(cv)) + ptable_.growth(table_bytes(total, cv)));
+                   {{&pts_in_, total * input_point_bytes(cv)}, {&ptable_, table_bytes(total, cv)}});
     if (rc != kOk) return rc;
-    ZK_ALLOC(pts_in_, total * input_point_bytes(cv));
-    ZK_ALLOC(ptable_, table_bytes(total, cv));
     rc = stage_upload(pts_in_.p, points, total * input_point_bytes(cv));
     if (rc != kOk) return rc;
     launch_build_table(cv, pts_in_.p, ptable_.p, total, stream_);
@@ -1138,7 +1137,7 @@ int32_t Engine::msm_device(const void* d_points, const void* d_scalars, const ui
     ZK_ALLOC(ptable_, table_bytes(total, cv));
     launch_build_table(cv, d_points, ptable_.p, total, stream_);
     Plan& pl = plan_;
-    int rc = plan_call(ns, t0, pl, 0, cv, 0, 0);
+    int rc = plan_call(ns, t0, pl, 0, cv, 0, {});
     if (rc != kOk) return rc;
     std::vector<uint8_t> res(ns.size() * result_bytes(cv));
     rc = run(pl, d_scalars, ptable_.p, total, res.data());
@@ -1184,11 +1183,13 @@ uint32_t Engine::shift_floor(const std::vector<uint32_t>& ns, bool lean) const {
     return kShiftFloor;
 }
 
-// The call's plan: the tuned window widths and the shift rule; where a cap on
-// the engine's memory leaves no room for it, the widths and the rule that need
-// the fewest buckets, and two accumulation waves' merge records (lean).  other: bytes the call will allocate besides.
+// The call's plan and its device memory: the tuned window widths and the shift
+// rule; where a cap on the engine's memory leaves no room for that plan, or the
+// device itself has none left, the widths and the rule that need the fewest
+// buckets, and two accumulation waves' merge records (lean).  other: the call's
+// buffers besides, allocated here too.
 int32_t Engine::plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
-                          CurveId cv, uint64_t shift_stride, uint64_t other) {
+                          CurveId cv, uint64_t shift_stride, std::initializer_list<BufSize> other) {
     const uint32_t nmsm = (uint32_t)ns.size();
     auto make = [&](bool lean) {
         const uint64_t lanes = lean ? std::min(lane_cap(cv), kTwoWaveLanes) : lane_cap(cv);
@@ -1196,11 +1197,21 @@ int32_t Engine::plan_call(const std::vector<uint32_t>& ns, const std::vector<uin
                          parts_req_, shift_stride, kShiftC, shift_floor(ns, lean), schedule(nmsm));
     };
     const int32_t rc = make(false);
-    if (rc != kOk || !ws_.limit) return rc;
+    if (rc != kOk) return rc;
     const bool dev_tail = device_tail(pl);
-    uint64_t need = other;
-    for (const BufSize& b : call_buffers(ws_sizes(pl, dev_tail), dev_tail, cv)) need += b.buf->growth(b.bytes);
-    return ws_.used + need > ws_.limit ? make(true) : rc;
+    const auto bufs = call_buffers(ws_sizes(pl, dev_tail), dev_tail, cv);
+    uint64_t need = 0;
+    for (const BufSize& b : other) need += b.buf->growth(b.bytes);
+    for (const BufSize& b : bufs) need += b.buf->growth(b.bytes);
+    const bool fits = !ws_.limit || ws_.used + need <= ws_.limit;
+    for (const BufSize& b : other) ZK_ALLOC(*b.buf, b.bytes);
+    if (!fits) return make(true);
+    for (const BufSize& b : bufs)
+        if (b.buf->ensure(b.bytes) != hipSuccess) {
+            for (const BufSize& r : bufs) r.buf->release();  // the lean plan's turn, from nothing
+            return make(true);
+        }
+    return kOk;
 }
 
 uint64_t Engine::plan_shift(const void* table, uint64_t shift_stride) const {
@@ -1514,11 +1525,10 @@ int32_t Engine::msm_table_parts(const void* table, uint32_t table_n,
     if (total >= (1ull << 30)) return kInvalidInput;
     Plan& pl = plan_;
     int rc = plan_call(ns, t0, pl, form, CurveId::Bn254, plan_shift(table, shift_stride),
-                       host_parts ? scalars_.growth(total * 32) : 0);
+                       {{&scalars_, host_parts ? total * 32 : 0}});
     if (rc != kOk) return rc;
     const void* d_sc = d_scalars;
     if (host_parts) {
-        ZK_ALLOC(scalars_, total * 32);
         uint64_t off = 0;
         for (uint32_t k = 0; k < idx.size(); k++) {
             const uint64_t bytes = (uint64_t)ns[k] * 32;

@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -31,6 +32,7 @@ enum Status : int32_t {
 struct WsAccount {
     uint64_t limit = 0;  // 0: no cap
     uint64_t used = 0;
+    uint64_t device = 0;   // tests: where the device itself runs out (0: nowhere)
 };
 
 // grow-only device buffer; with an account, a growth that would take the
@@ -283,6 +285,7 @@ class Engine {
     // and leaves the engine usable
     void set_workspace_limit(uint64_t bytes) { ws_.limit = bytes; }
     uint64_t workspace_bytes() const { return ws_.used; }
+    void test_device_memory(uint64_t bytes) { ws_.device = bytes; }
     // graph mode: the device launch sequence of a call is captured into a
     // hipGraph and replayed while calls keep the same shape and buffers
     // kGraphAuto (default): a call whose shape and buffers repeat the
@@ -406,7 +409,7 @@ class Engine {
     };
     std::array<BufSize, 17> call_buffers(const WsSizes& z, bool dev_tail, CurveId cv);
     int32_t plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
-                      CurveId cv, uint64_t shift_stride, uint64_t other);
+                      CurveId cv, uint64_t shift_stride, std::initializer_list<BufSize> other);
     // make_plan's shift_floor for a call: in calls of up to kShiftAlwaysMsms
     // MSMs every MSM of at least kShiftFloor points (a single one up to
     // kShiftSingleMax): below that a plain reduction of narrow windows is as
