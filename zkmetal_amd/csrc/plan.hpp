@@ -91,6 +91,10 @@ struct SegDesc {
 constexpr uint32_t reduce_teams(uint32_t len, uint32_t per, uint32_t block_teams) {
     return len <= per ? 1 : len / per < block_teams ? len / per : block_teams;
 }
+// Whole waves without elements may leave before a tree over P teams only if it
+// stays within one wave: a wider one has barriers, where every wave is waited
+// for.
+constexpr bool tree_idle(uint32_t P, uint32_t team, uint32_t per_wave) { return P <= per_wave && team >= per_wave; }
 // lanes that share one point in the merge and reduction kernels (team29.hpp):
 // a block of 256 holds 256 / this many teams
 constexpr uint32_t team_lanes(CurveId cv) { return cv == CurveId::Bn254G2 ? 8u : 4u; }

@@ -36,7 +36,8 @@ __device__ __forceinline__ void wave_tree(typename T::Pt& acc, uint32_t P) {
 }
 
 // the same over groups of up to a block's teams: the waves of a group meet in
-// LDS (lds: four points).  P uniform over the block; every thread calls it.
+// LDS (lds: four points).  P uniform over the block; every thread calls it,
+// but those that tree_idle excuses.
 template <class T>
 __device__ __forceinline__ void block_tree(typename T::Pt& acc, uint32_t P, uint4* lds) {
     wave_tree<T>(acc, min(P, T::kPerWave));
@@ -447,9 +448,10 @@ __global__ __launch_bounds__(256) void k_br_bits(const SegDesc* __restrict__ seg
     } else {
         base = R0; b = j - 1 - g; count = 1u << (h - 1); masked = true;
     }
-    // count is a power of 2: teams take elements team, team + P, ...
+    // count is a power of 2: teams take elements team, team + P, ...; teams past
+    // P repeat the first ones'
     const uint32_t P = min(count, blockDim.x / T::kLanes), team = threadIdx.x / T::kLanes;
-    if (team >= max(P, T::kPerWave)) return;  // whole waves without elements (then no LDS tree)
+    if (tree_idle(P, team, T::kPerWave)) return;
     auto element = [&](uint32_t i) { return T::load(rc, base + (masked ? with_bit(i, b) : i)); };
     typename T::Pt acc = element(team & (P - 1));
 #pragma unroll 1
