@@ -118,14 +118,17 @@ static void plan_reset(Plan& pl) {
 
 // parts for a call of `entries` sorted entries: the exposed sort is the first
 // part's, and every part adds a round of launches and merge records
-uint32_t default_parts(uint64_t entries) {
-    // measured, 1 against 2 parts: 2^20 points (2^24 entries) 1580 against
-    // 1630 us, 2^20 G2 points (2^24) 4360 against 4400; 2^22 points (2^26)
-    // 5870 against 5715 us, the 64-MSM batch (2^27.7) 15.25 against 15.0 ms (3
-    // parts: 16.0).  With three accumulation waves per SIMD a sort beside the
-    // accumulation finds little room; what two parts gain is the second sort
-    // running on while the first waves start.
-    return entries > (1ull << 24) ? 2u : 1u;
+uint32_t default_parts(uint64_t entries, CurveId cv) {
+    // The line is where one part and two take the same time on MI355X.  With
+    // three accumulation waves per SIMD a sort beside the accumulation finds
+    // little room; what two parts gain is the second sort running on while the
+    // first waves start.  Two parts against one, million entries: G1 16.8 1.07,
+    // 19 1.03, 29 1.02, 40 1.007, 48 0.993, 67 0.986; batches 17 1.05, 34
+    // 1.03, 50 0.997, 64 0.994; Grumpkin 17 1.04, 29 1.003, 34 0.988, 67 0.986;
+    // G2 17 1.004, 29 1.004, 34 0.996.  Three parts took longer than two at
+    // each of the batches (64 MSMs of 2^12 to 2^20 points: 16.0 ms against 15.0).
+    const uint64_t line = cv == CurveId::Bn254 ? 44000000 : 31000000;
+    return entries > line ? 2u : 1u;
 }
 
 // Window-shifted or plain, by an estimate in mixed-addition units: every
@@ -173,7 +176,7 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm, const u
     auto parts_for = [&](uint64_t entries) -> uint32_t {
         if (nparts) return nparts;
         if (sched && sched->parts[size_class(entries)]) return sched->parts[size_class(entries)];
-        return default_parts(entries);
+        return default_parts(entries, cv);
     };
     plan_reset(pl);
     pl.curve = cv;

@@ -160,7 +160,7 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm,
               uint64_t lane_cap = 1u << 17, CurveId cv = CurveId::Bn254, uint32_t nparts = 0,
               uint64_t shift_stride = 0, uint32_t shift_c = 0, uint32_t shift_floor = 0,
               const Schedule* sched = nullptr);
-uint32_t default_parts(uint64_t entries);
+uint32_t default_parts(uint64_t entries, CurveId cv = CurveId::Bn254);
 bool shifted_pays(uint64_t n, uint32_t c, uint32_t c_s);
 
 class Engine {
