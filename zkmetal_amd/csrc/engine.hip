@@ -122,11 +122,11 @@ uint32_t default_parts(uint64_t entries, CurveId cv) {
     // The line is where one part and two take the same time on MI355X.  With
     // three accumulation waves per SIMD a sort beside the accumulation finds
     // little room; what two parts gain is the second sort running on while the
-    // first waves start.  Two parts against one, million entries: G1 16.8 1.07,
-    // 19 1.03, 29 1.02, 40 1.007, 48 0.993, 67 0.986; batches 17 1.05, 34
-    // 1.03, 50 0.997, 64 0.994; Grumpkin 17 1.04, 29 1.003, 34 0.988, 67 0.986;
-    // G2 17 1.004, 29 1.004, 34 0.996.  Three parts took longer than two at
-    // each of the batches (64 MSMs of 2^12 to 2^20 points: 16.0 ms against 15.0).
+    // first waves start.  Two parts against one, million entries: G1 17 1.07,
+    // 19 1.04, 29 1.02, 34 1.02, 40 1.00, 48 0.99, 67 0.99; batches 17 1.04, 34
+    // 1.01, 50 0.99, 67 0.98; Grumpkin 17 1.04, 29 1.01, 34 1.00, 48 0.99; G2 17
+    // 1.01, 22 to 29 1.00, 34 0.99 (1.00: within 0.5%).  Three parts were
+    // nowhere ahead of both (64 MSMs of 2^12 to 2^20 points: 16.0 ms, two 15.0).
     const uint64_t line = cv == CurveId::Bn254 ? 44000000 : 31000000;
     return entries > line ? 2u : 1u;
 }
