@@ -636,9 +636,8 @@ struct Arith {
 
     static __device__ __forceinline__ bool qxyzz_is_id(const QXyzz& p) { return fq_is_zero2(p.ZZ); }
 
-    // doubling core: X, Y < 4p.  Returns X3 < 2.5p, Y3 < 3.5p; V, W < 1.5p.
-    // (independent products in pairs: the doubling also runs alone in one
-    // lane, in the device tail, where a second chain hides the latency)
+    // doubling core: X < 6.5p, Y < 4p (a stored point).  Returns X3 < 2.5p,
+    // Y3 < 3.5p; V, W < 1.5p.
     static __device__ __forceinline__ void qdbl_core(const Fq& X, const Fq& Y, Fq& X3, Fq& Y3, Fq& V, Fq& W) {
         const Fq U = fq_add(Y, Y);  // < 8p
         Fq xx, S;
@@ -668,11 +667,9 @@ struct Arith {
         return r;
     }
 
-    // ---- repeated doubling (the device tail's window combine).  A chain of
-    // doublings runs in Jacobian coordinates (x = X/Z^2, y = Y/Z^3;
-    // dbl-2009-l for a = 0: 2M + 5S against XYZZ's 6M + 3S), with the
-    // independent products in pairs (one lane runs the chain alone, so a
-    // second multiply-add chain fills the dependent-issue latency).
+    // ---- repeated doubling (the window copies of a resident table): in
+    // Jacobian coordinates (x = X/Z^2, y = Y/Z^3; dbl-2009-l for a = 0: 2M + 5S
+    // against XYZZ's 6M + 3S), with the independent products in pairs.
     // Bounds: X, Y, Z < 2p in and out; Z = 0 mod p is the identity.
     static __device__ __forceinline__ void qjac_dbl(Fq& X, Fq& Y, Fq& Z) {
         Fq A, B, C, T;
@@ -696,24 +693,6 @@ struct Arith {
         X = X3;
         Y = Y3;
         Z = Z3;
-    }
-
-    // 2^k P for an XYZZ point (X < 6.5p, Y < 4p, ZZ, ZZZ < 2p): to Jacobian
-    // (X ZZ^2, Y ZZZ^2, ZZZ), k doublings, back (ZZ = Z^2, ZZZ = Z^3).  The
-    // identity (ZZ = ZZZ = 0) stays the identity.  Out: X, Y < 2p, ZZ, ZZZ < 1.5p.
-    static __device__ __forceinline__ QXyzz qxyzz_dbl_k(const QXyzz& p, uint32_t k) {
-        Fq ZZ2, ZZZ2, X, Y;
-        fq_sqr_x2(p.ZZ, ZZ2, p.ZZZ, ZZZ2);
-        fq_mul_sub_x2<0, 1, 0, 1>(p.X, ZZ2, p.X, X, p.Y, ZZZ2, p.Y, Y);  // < 1.5p each
-        Fq Z = p.ZZZ;                                                     // < 2p
-#pragma unroll 1
-        for (uint32_t i = 0; i < k; i++) qjac_dbl(X, Y, Z);
-        QXyzz r;
-        r.X = X;
-        r.Y = Y;
-        r.ZZ = fq_sqr(Z);
-        r.ZZZ = fq_mul(r.ZZ, Z);
-        return r;
     }
 
     // acc += (x2, y2); x2, y2 < p.  q_id: the affine point is (0,0).
