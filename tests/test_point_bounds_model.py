@@ -1,7 +1,8 @@
 """CPU model of the point additions that hand stored points to one another
-between the kernels: the lane teams (zkmetal_amd/csrc/team29.hpp) and the
-one-lane G2 addition and doubling (curve_g2.hpp), limb for limb, on the
-products with the reduction digits of curve29.hpp (q_m, q_red).
+between the kernels: the bucket loop's (curve29.hpp, curve_g2.hpp), the lane
+teams' (zkmetal_amd/csrc/team29.hpp) and the one-lane G2 addition and doubling
+(curve_g2.hpp), limb for limb, on single and merged products with the reduction
+digits of curve29.hpp (q_m, q_red).
 
 What it pins: the one bound of a stored point (X < 6.5p, Y < 3.5p, ZZ, ZZZ <
 2p per component, limbs normalised) holds for what either form stores and is
@@ -211,6 +212,51 @@ def lane_add(a, q):
     return a if qid else r
 
 
+# ---- the bucket loop's additions of an affine table point
+
+def run_g1(a, q):
+    """Arith::qxyzz_madd_run (its columns in fixed order; the sums are these):
+    the new accumulator and whether the two cancelled"""
+    X, Y, ZZ, ZZZ = (c[0] for c in stored(a))
+    x2, y2 = q[0][0], q[1][0]
+    Pp, Rr = prod([(x2, ZZ)], 7, X), prod([(y2, ZZZ)], 5, Y)
+    lt(Pp, 8.5), lt(Rr, 6.5)
+    PP, RR = prod([(Pp, Pp)]), prod([(Rr, Rr)])
+    lt(PP, 1.6), lt(RR, 1.6)
+    PPP, Q = prod([(Pp, PP)]), prod([(X, PP)])
+    X3 = fq_sub(5, RR, [2 * x + y for x, y in zip(Q, PPP)])
+    Y3 = prod([(Rr, sub_lazy(7, Q, X3)), (Y, sub_lazy(2, ZERO, PPP))])
+    r = stored(((X3,), (Y3,), (prod([(ZZ, PP)]),), (prod([(ZZZ, PPP)]),)))
+    assert iz2(PP) == (PP[0] in (0, PL[0]) and iz2(PP))  # the one-limb screen misses none
+    cancel = False
+    if iz2(PP):
+        cancel = not iz2(RR)
+        if not cancel:
+            r = team_dbl((q[0], q[1], (limbs(R % P),), (limbs(R % P),)))
+    return r, cancel
+
+
+def run_g2(a, q):
+    """G2Arith::madd_run"""
+    for c in a:
+        below(c, 2)
+    Pp, Rr = below(m2(q[0], a[2], 2, a[0]), 3.1), below(m2(q[1], a[3], 2, a[1]), 3.1)
+    PP = (prod([(fq_add(*Pp), sub_lazy(4, *Pp))]), prod([([2 * v for v in Pp[0]], Pp[1])]))
+    PPP, Q = below(m2(Pp, PP), 1.1), below(m2(a[0], PP), 1.1)
+    T = below(each(lambda u, v: [2 * x + y for x, y in zip(u, v)], Q, PPP), 4)
+    X3 = each(red8, (prod([(fq_add(*Rr), sub_lazy(4, *Rr))], 4, T[0], 3),
+                     prod([([2 * v for v in Rr[0]], Rr[1])], 4, T[1], 3)))
+    Y3 = each(red4, m2(Rr, esub(2, Q, X3), 2, m2(a[1], PPP), kb=4))
+    r = tuple(below(c, 2) for c in (X3, Y3, m2(a[2], PP), m2(a[3], PPP)))
+    cancel = False
+    if zero(PP):
+        cancel = not zero(each(red4, Rr))
+        if not cancel:
+            one = (limbs(R % P), ZERO)
+            r = lane_dbl((q[0], q[1], one, one))
+    return r, cancel
+
+
 # ---- points
 
 def xyzz(pt, rnd, g2):
@@ -290,3 +336,41 @@ def test_lane_additions_of_merged_points():
             u = team_add(xyzz(G2.neg(a), rnd, True), xyzz(G2.neg(b), rnd, True))
             assert affine(lane_add(s, u)) is None
             assert affine(lane_add(lane_add(s, xyzz(a, rnd, True)), t)) == G2.add(G2.add(want, want), a)
+
+
+@pytest.mark.parametrize("C", [B, G2], ids=["g1", "g2"])
+def test_bucket_runs_and_their_merge(C):
+    """runs of table points (a repeat, a cancellation), then the merge of two
+    runs by a team, and in G2 the lane addition of two such buckets"""
+    rnd = random.Random(44)
+    g2, step = C is G2, run_g2 if C is G2 else run_g1
+    one = (limbs(R % P), ZERO) if g2 else (limbs(R % P),)
+
+    def table(pt):
+        return tuple(tuple(limbs(v * R % P) for v in (c if g2 else (c,))) for c in pt)
+
+    def run(pts):
+        acc, want = None, None
+        for pt in pts:
+            q = table(pt)
+            if acc is None:
+                acc, cancel = (q[0], q[1], one, one), False
+            else:
+                acc, cancel = step(acc, q)
+            want = C.add(want, pt)
+            if cancel:
+                assert want is None and affine(acc) is None
+                acc = None
+            else:
+                assert affine(acc) == want
+        return acc, want
+
+    for _ in range(4):
+        pts = [C.mul(C.G2 if g2 else C.G, rnd.randrange(1, B.R_ORDER)) for _ in range(6)]
+        a, wa = run([pts[0], pts[0], pts[1], C.neg(C.add(C.add(pts[0], pts[0]), pts[1])), pts[2], pts[3]])
+        b, wb = run([pts[4], pts[5], pts[4]])
+        s = team_add(a, b)
+        assert affine(s) == C.add(wa, wb)
+        assert affine(team_add(s, a)) == C.add(C.add(wa, wb), wa)
+        if g2:
+            assert affine(lane_add(s, team_add(b, a))) == C.mul(C.add(wa, wb), 2)
