@@ -1087,12 +1087,16 @@ int32_t Engine::msm_batch_host(const uint8_t* points, const uint8_t* scalars,
         }
     }
     Plan pl;
-    rc = plan_call(ns, t0, pl, 0, cv, 0,
-                   {{&pts_in_, total * input_point_bytes(cv)}, {&ptable_, table_bytes(total, cv)}});
+    const Call call{ns, t0, 0, cv, 0};
+    rc = plan_call(call, pl, pts_in_.growth(total * input_point_bytes(cv)) + ptable_.growth(table_bytes(total, cv)));
     if (rc != kOk) return rc;
+    ZK_ALLOC(pts_in_, total * input_point_bytes(cv));
+    ZK_ALLOC(ptable_, table_bytes(total, cv));
     rc = stage_upload(pts_in_.p, points, total * input_point_bytes(cv));
     if (rc != kOk) return rc;
     launch_build_table(cv, pts_in_.p, ptable_.p, total, stream_);
+    rc = take_buffers(call, pl);
+    if (rc != kOk) return rc;
     std::vector<uint8_t> res(ns.size() * result_bytes(cv));
     rc = run(pl, scalars_.p, ptable_.p, total, res.data());
     if (rc != kOk) return rc;
@@ -1140,7 +1144,9 @@ int32_t Engine::msm_device(const void* d_points, const void* d_scalars, const ui
     ZK_ALLOC(ptable_, table_bytes(total, cv));
     launch_build_table(cv, d_points, ptable_.p, total, stream_);
     Plan& pl = plan_;
-    int rc = plan_call(ns, t0, pl, 0, cv, 0, {});
+    const Call call{ns, t0, 0, cv, 0};
+    int rc = plan_call(call, pl, 0);
+    if (rc == kOk) rc = take_buffers(call, pl);
     if (rc != kOk) return rc;
     std::vector<uint8_t> res(ns.size() * result_bytes(cv));
     rc = run(pl, d_scalars, ptable_.p, total, res.data());
@@ -1186,33 +1192,36 @@ uint32_t Engine::shift_floor(const std::vector<uint32_t>& ns, bool lean) const {
     return kShiftFloor;
 }
 
-// The call's plan and its device memory: the tuned window widths and the shift
-// rule; where a cap on the engine's memory leaves no room for that plan, or the
-// device itself has none left, the widths and the rule that need the fewest
-// buckets, and two accumulation waves' merge records (lean).  other: the call's
-// buffers besides, allocated here too.
-int32_t Engine::plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
-                          CurveId cv, uint64_t shift_stride, std::initializer_list<BufSize> other) {
-    const uint32_t nmsm = (uint32_t)ns.size();
-    auto make = [&](bool lean) {
-        const uint64_t lanes = lean ? std::min(lane_cap(cv), kTwoWaveLanes) : lane_cap(cv);
-        return make_plan(ns.data(), t0.data(), nmsm, window_bits_for(ns, cv, lean).data(), pl, form, lanes, cv,
-                         parts_req_, shift_stride, kShiftC, shift_floor(ns, lean), schedule(nmsm));
-    };
-    const int32_t rc = make(false);
-    if (rc != kOk) return rc;
+// make_plan for a call: the tuned window widths and the shift rule, or (lean)
+// the widths and the rule that need the fewest buckets, and two accumulation
+// waves' merge records.
+int32_t Engine::call_plan(const Call& c, Plan& pl, bool lean) {
+    const uint32_t nmsm = (uint32_t)c.ns.size();
+    const uint64_t lanes = lean ? std::min(lane_cap(c.cv), kTwoWaveLanes) : lane_cap(c.cv);
+    return make_plan(c.ns.data(), c.t0.data(), nmsm, window_bits_for(c.ns, c.cv, lean).data(), pl, c.form, lanes, c.cv,
+                     parts_req_, c.shift_stride, kShiftC, shift_floor(c.ns, lean), schedule(nmsm));
+}
+
+// The call's plan, lean where a cap on the engine's memory leaves no room for
+// the other.  other: bytes the call will allocate besides.
+int32_t Engine::plan_call(const Call& c, Plan& pl, uint64_t other) {
+    const int32_t rc = call_plan(c, pl, false);
+    if (rc != kOk || !ws_.limit) return rc;
     const bool dev_tail = device_tail(pl);
-    const auto bufs = call_buffers(ws_sizes(pl, dev_tail), dev_tail, cv);
-    uint64_t need = 0;
-    for (const BufSize& b : other) need += b.buf->growth(b.bytes);
-    for (const BufSize& b : bufs) need += b.buf->growth(b.bytes);
-    const bool fits = !ws_.limit || ws_.used + need <= ws_.limit;
-    for (const BufSize& b : other) ZK_ALLOC(*b.buf, b.bytes);
-    if (!fits) return make(true);
+    uint64_t need = other;
+    for (const BufSize& b : call_buffers(ws_sizes(pl, dev_tail), dev_tail, c.cv)) need += b.buf->growth(b.bytes);
+    return ws_.used + need > ws_.limit ? call_plan(c, pl, true) : rc;
+}
+
+// Before run: the call's device buffers, or, where the device has no room for
+// them, the lean plan and none of them (run allocates its own).
+int32_t Engine::take_buffers(const Call& c, Plan& pl) {
+    const bool dev_tail = device_tail(pl);
+    const auto bufs = call_buffers(ws_sizes(pl, dev_tail), dev_tail, c.cv);
     for (const BufSize& b : bufs)
         if (b.buf->ensure(b.bytes) != hipSuccess) {
-            for (const BufSize& r : bufs) r.buf->release();  // the lean plan's turn, from nothing
-            return make(true);
+            for (const BufSize& r : bufs) r.buf->release();
+            return call_plan(c, pl, true);
         }
     return kOk;
 }
@@ -1527,11 +1536,12 @@ int32_t Engine::msm_table_parts(const void* table, uint32_t table_n,
     if (ns.empty()) return kOk;
     if (total >= (1ull << 30)) return kInvalidInput;
     Plan& pl = plan_;
-    int rc = plan_call(ns, t0, pl, form, CurveId::Bn254, plan_shift(table, shift_stride),
-                       {{&scalars_, host_parts ? total * 32 : 0}});
+    const Call call{ns, t0, form, CurveId::Bn254, plan_shift(table, shift_stride)};
+    int rc = plan_call(call, pl, host_parts ? scalars_.growth(total * 32) : 0);
     if (rc != kOk) return rc;
     const void* d_sc = d_scalars;
     if (host_parts) {
+        ZK_ALLOC(scalars_, total * 32);
         uint64_t off = 0;
         for (uint32_t k = 0; k < idx.size(); k++) {
             const uint64_t bytes = (uint64_t)ns[k] * 32;
@@ -1541,6 +1551,8 @@ int32_t Engine::msm_table_parts(const void* table, uint32_t table_n,
         }
         d_sc = scalars_.p;
     }
+    rc = take_buffers(call, pl);
+    if (rc != kOk) return rc;
     std::vector<uint8_t> res(ns.size() * 96);
     rc = run(pl, d_sc, table, table_n, res.data());
     if (rc != kOk) return rc;

@@ -10,7 +10,6 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
-#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -408,8 +407,17 @@ class Engine {
         uint64_t bytes;
     };
     std::array<BufSize, 17> call_buffers(const WsSizes& z, bool dev_tail, CurveId cv);
-    int32_t plan_call(const std::vector<uint32_t>& ns, const std::vector<uint64_t>& t0, Plan& pl, uint32_t form,
-                      CurveId cv, uint64_t shift_stride, std::initializer_list<BufSize> other);
+    // what a call's plan is made from
+    struct Call {
+        const std::vector<uint32_t>& ns;  // points of each MSM
+        const std::vector<uint64_t>& t0;  // first table entries
+        uint32_t form;
+        CurveId cv;
+        uint64_t shift_stride;
+    };
+    int32_t call_plan(const Call& c, Plan& pl, bool lean);
+    int32_t plan_call(const Call& c, Plan& pl, uint64_t other);
+    int32_t take_buffers(const Call& c, Plan& pl);
     // make_plan's shift_floor for a call: in calls of up to kShiftAlwaysMsms
     // MSMs every MSM of at least kShiftFloor points (a single one up to
     // kShiftSingleMax): below that a plain reduction of narrow windows is as
