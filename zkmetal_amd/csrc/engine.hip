@@ -413,7 +413,7 @@ int32_t Engine::create(Engine** out) {
 
 void Engine::account_buffers() {
     for (DevBuf* b : {&desc_, &digits_, &keysA_, &valsA_, &keysB_, &valsB_, &hist_, &part_, &segvalid_,
-                      &buckets_, &recAk_, &recAp_, &lists_, &rc_, &winsum_, &err_, &wins_,
+                      &buckets_, &recAk_, &recAp_, &lists_, &rc_, &err_, &wins_,
                       &pts_in_, &ptable_, &scalars_, &srs_, &gtab_, &gtab_gk_, &gtab_g2_, &tmp_})
         b->acct = &ws_;
 }
@@ -625,32 +625,27 @@ WsSizes ws_sizes(const Plan& pl, bool dev_tail) {
     z.rec_pts = rec_cap * ptb;
     z.lists = merge_lists_bytes(rec_cap, pl.curve);
     z.rc = pl.groups * ptb;
-    // bit-plane points: host form for the host tail, stored form for the device's
-    // and for BN254 G2, whose window sums (host form) the device makes of them
-    const bool g2 = pl.curve == CurveId::Bn254G2;
-    z.bits = nseg * 16 * (dev_tail || g2 ? ptb : hpb);
     z.err = 32;  // the decomposition flag, the merge's list counters
     z.wins = dev_tail ? nseg * ptb : 0;
     // device tail: the sums, normalised on the host, or (many) the results
     z.res = dev_tail ? nmsm * (nmsm <= kHostNormMsms ? hpb : result_bytes(pl.curve)) : 0;
-    // copied back: those (device tail) or the bit planes, then err, then
-    // the per-segment valid-entry counts
-    z.back = dev_tail ? z.res : g2 ? nseg * hpb : z.bits;
+    // copied back: those (device tail), the window sums (BN254 G2) or the bit
+    // planes, then err, then the per-segment valid-entry counts.  (Planes that
+    // the device combines lie over the buckets.)
+    z.back = dev_tail ? z.res : pl.curve == CurveId::Bn254G2 ? nseg * hpb : nseg * 16 * hpb;
     z.host = z.back + z.err + nseg * 4;
     const uint64_t parts[] = {z.desc, z.digits, z.keys, z.vals, z.keys, z.vals, z.hist, z.part,
-                              z.segvalid, z.buckets, z.rec_keys, z.rec_pts, z.lists, z.rc, z.bits,
-                              z.err, z.wins, z.res};
+                              z.segvalid, z.buckets, z.rec_keys, z.rec_pts, z.lists, z.rc, z.err, z.wins, z.res};
     for (uint64_t b : parts) z.device += (b + 255) & ~uint64_t(255);
     return z;
 }
 
 // the device buffers of a call and the bytes it needs of each (0: not used)
-std::array<Engine::BufSize, 17> Engine::call_buffers(const WsSizes& z, bool dev_tail, CurveId cv) {
-    const bool dev_bits = dev_tail || cv == CurveId::Bn254G2;  // else the planes go to host memory
+std::array<Engine::BufSize, 16> Engine::call_buffers(const WsSizes& z) {
     return {{{&desc_, z.desc}, {&digits_, z.digits}, {&keysA_, z.keys}, {&valsA_, z.vals}, {&keysB_, z.keys},
              {&valsB_, z.vals}, {&hist_, z.hist}, {&part_, z.part}, {&segvalid_, z.segvalid},
              {&buckets_, z.buckets}, {&recAk_, z.rec_keys}, {&recAp_, z.rec_pts}, {&lists_, z.lists}, {&rc_, z.rc},
-             {&winsum_, dev_bits ? z.bits : 0}, {&wins_, z.wins}, {&err_, z.err}}};
+             {&wins_, z.wins}, {&err_, z.err}}};
 }
 
 int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, uint64_t table_n,
@@ -658,8 +653,7 @@ int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, 
     // window combine on the device (graph mode, large batches) or the host
     const bool dev_tail = device_tail(pl);
     const WsSizes z = ws_sizes(pl, dev_tail);
-    const bool dev_bits = dev_tail || pl.curve == CurveId::Bn254G2;
-    for (const BufSize& b : call_buffers(z, dev_tail, pl.curve)) ZK_ALLOC(*b.buf, b.bytes);
+    for (const BufSize& b : call_buffers(z)) ZK_ALLOC(*b.buf, b.bytes);
     ZK_ALLOC(hdesc_, z.desc);
     ZK_ALLOC(hwin_, z.host);
     Workspace ws;
@@ -682,7 +676,7 @@ int32_t Engine::run(const Plan& pl, const void* d_scalars, const void* d_table, 
     ws.hdesc = (uint8_t*)hdesc_.p;
     ws.hw = (uint8_t*)hwin_.p;
     ws.mapped = true;
-    ws.bits = dev_bits ? winsum_.p : hwin_.p;
+    ws.bits = dev_tail || pl.curve == CurveId::Bn254G2 ? buckets_.p : hwin_.p;
     ws.res = hwin_.p;
     return run_ws(pl, ws, z, dev_tail, graph_mode_, d_scalars, d_table, table_n, out96);
 }
@@ -815,7 +809,7 @@ int32_t Engine::run_ws(const Plan& pl, const Workspace& ws, const WsSizes& z, bo
             if (!ws.mapped) ZK_TRY(rec(ev_tail_, st));
         }
         if (ws.mapped) return kOk;
-        ZK_TRY(hipMemcpyAsync(hw, dev_tail ? ws.res : ws.bits, back_bytes, hipMemcpyDeviceToHost, st));
+        ZK_TRY(hipMemcpyAsync(hw, ws.res, back_bytes, hipMemcpyDeviceToHost, st));
         ZK_TRY(hipMemcpyAsync(hw + back_bytes, ws.err, 4 * 5, hipMemcpyDeviceToHost, st));
         ZK_TRY(hipMemcpyAsync(hw + back_bytes + z.err, ws.segvalid, (uint64_t)nseg * 4,
                               hipMemcpyDeviceToHost, st));
@@ -1207,17 +1201,15 @@ int32_t Engine::call_plan(const Call& c, Plan& pl, bool lean) {
 int32_t Engine::plan_call(const Call& c, Plan& pl, uint64_t other) {
     const int32_t rc = call_plan(c, pl, false);
     if (rc != kOk || !ws_.limit) return rc;
-    const bool dev_tail = device_tail(pl);
     uint64_t need = other;
-    for (const BufSize& b : call_buffers(ws_sizes(pl, dev_tail), dev_tail, c.cv)) need += b.buf->growth(b.bytes);
+    for (const BufSize& b : call_buffers(ws_sizes(pl, device_tail(pl)))) need += b.buf->growth(b.bytes);
     return ws_.used + need > ws_.limit ? call_plan(c, pl, true) : rc;
 }
 
 // Before run: the call's device buffers, or, where the device has no room for
 // them, the lean plan and none of them (run allocates its own).
 int32_t Engine::take_buffers(const Call& c, Plan& pl) {
-    const bool dev_tail = device_tail(pl);
-    const auto bufs = call_buffers(ws_sizes(pl, dev_tail), dev_tail, c.cv);
+    const auto bufs = call_buffers(ws_sizes(pl, device_tail(pl)));
     for (const BufSize& b : bufs)
         if (b.buf->ensure(b.bytes) != hipSuccess) {
             for (const BufSize& r : bufs) r.buf->release();
@@ -1738,7 +1730,7 @@ int32_t Engine::msm_resident_noalloc(const void* d_scalars, const uint32_t* coun
     ws.recAp = take(z.rec_pts);
     ws.lists = take(z.lists);
     ws.rc = take(z.rc);
-    ws.bits = take(z.bits);
+    ws.bits = ws.buckets;
     ws.err = take(z.err);
     ws.wins = take(z.wins);
     ws.res = take(z.res);

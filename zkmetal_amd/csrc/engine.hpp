@@ -121,14 +121,14 @@ struct Workspace {
     uint8_t* hdesc = nullptr;  // host: descriptors before upload
     uint8_t* hw = nullptr;     // host: copy-back area
     // hdesc and hw are pinned, and bits (host tail) or res point into hw: the
-    // kernels read and write them, no copies
+    // kernels read and write them, no copies.  Not mapped: device tail only.
     bool mapped = false;
 };
 
 // bytes of each buffer of a planned call; device = all device buffers, each
 // rounded up to 256 bytes; host = the copy-back area
 struct WsSizes {
-    uint64_t desc, digits, keys, vals, hist, part, segvalid, buckets, rec_keys, rec_pts, lists, rc, bits, err,
+    uint64_t desc, digits, keys, vals, hist, part, segvalid, buckets, rec_keys, rec_pts, lists, rc, err,
         wins, res, back, host, device;
 };
 WsSizes ws_sizes(const Plan& pl, bool dev_tail);
@@ -388,7 +388,7 @@ class Engine {
     Timing timing_{};
 
     DevBuf desc_, digits_, keysA_, valsA_, keysB_, valsB_, hist_, part_, segvalid_, buckets_;
-    DevBuf recAk_, recAp_, lists_, rc_, winsum_, err_;  // lists_: the merge's run lists
+    DevBuf recAk_, recAp_, lists_, rc_, err_;  // lists_: the merge's run lists
     DevBuf wins_;  // device tail: window sums
     DevBuf pts_in_, ptable_, scalars_, srs_, gtab_, gtab_gk_, gtab_g2_, tmp_;
     HostBuf hdesc_, hwin_;
@@ -406,7 +406,7 @@ class Engine {
         DevBuf* buf;
         uint64_t bytes;
     };
-    std::array<BufSize, 17> call_buffers(const WsSizes& z, bool dev_tail, CurveId cv);
+    std::array<BufSize, 16> call_buffers(const WsSizes& z);
     // what a call's plan is made from
     struct Call {
         const std::vector<uint32_t>& ns;  // points of each MSM

@@ -83,16 +83,17 @@ struct CallBack {
     uint32_t nseg;
     uint32_t* out;
 };
-// bits: 16 points per segment (U and the bit-plane sums), in the host form
-// (Xyzz, 2^256 Montgomery, 128 B) for the host tail or in the stored form
-// (144 B) for launch_tail; seg_blk0: first row/column block of each segment,
+// bits: U and the bit-plane sums, 16 points per segment in the host form
+// (Xyzz, 2^256 Montgomery, 128 B) for the host tail, or in the stored form over
+// each segment's first buckets (bits is buckets) for launch_tail and
+// launch_g2_windows; seg_blk0: first row/column block of each segment,
 // blocks: their number; by_lanes: the plan's reduce_lanes; bits may be pinned
 // host memory, and back as above, when this ends the call
 void launch_bucket_reduce(CurveId cv, const SegDesc* segs, const uint64_t* seg_blk0, const uint64_t* seg_rc0,
                           uint32_t nseg, uint64_t blocks, uint32_t per, bool by_lanes, const void* buckets, void* rc,
                           void* bits, bool host_form, const CallBack& back, hipStream_t st);
-// window combine on the device (BN254 G1 and Grumpkin): bits in the stored
-// form, wins: nseg stored points (scratch), out: nmsm sums in the host form
+// window combine on the device (BN254 G1 and Grumpkin): bits as above, wins:
+// nseg stored points (scratch), out: nmsm sums in the host form
 // (Xyzz, 128 B), or with norm nmsm results of 96 B (normalised Jacobian
 // X | Y | Z, 2^256 Montgomery form)
 void launch_tail(CurveId cv, const SegDesc* segs, const MsmDesc* msms, uint32_t nseg, uint32_t nmsm,

@@ -281,9 +281,10 @@ __global__ __launch_bounds__(256) void k_merge_spans(uint4* __restrict__ dest, M
 // summed by reduce_teams(2^g, per) teams (about `per` buckets each, then a
 // tree), a column of 2^h buckets likewise; the rows and the columns of a
 // segment start on block boundaries, so the tree's width is block-uniform.
-// k_br_bits: one block per output point, bits[s*16 + j]: j = 0 -> U,
-// 1..g -> Pl_{j-1}, g+1..c-1 -> Ph_{j-1-g}.  The host (or k_tail_windows)
-// applies the powers of 2.  Small calls are bound by the depth of the two
+// k_br_bits: one block per output point j of segment s: j = 0 -> U, 1..g ->
+// Pl_{j-1}, g+1..c-1 -> Ph_{j-1-g}.  The host (bits[s*16 + j]) or
+// k_tail_windows (plane j over the segment's bucket j, whose sums are taken by
+// then: c planes, 2^(c-1) buckets) applies the powers of 2.  Small calls are bound by the depth of the two
 // kernels' chains: 256 points (16 windows of 128 buckets) 79 us with one lane
 // per addition, 26 us with teams.
 
@@ -459,15 +460,15 @@ __global__ __launch_bounds__(256) void k_br_bits(const SegDesc* __restrict__ seg
     block_tree<T>(acc, P, lds);
     if (threadIdx.x < T::kLanes) {
         if (host_form) T::store_host(bits, blockIdx.x, acc);  // for the host tail
-        else T::store(bits, blockIdx.x, acc);                 // for k_tail_windows
+        else T::store(bits, sg.bkt0 + j, acc);                // for k_tail_windows
     }
 }
 
 // ------------------------------------------------ window combine on the device
 // The device form of the call's tail (the host form is Engine::run's
 // host_tail): result_j = sum_w 2^(cstep w) S_w over the MSM's segments w,
-// S_w = U_w + sum_{t < c-1} 2^t Q_{w,t}, the planes k_br_bits stored
-// (bits[s*16] = U, bits[s*16 + 1 + t] = Q_t), then the affine normalisation;
+// S_w = U_w + sum_{t < c-1} 2^t Q_{w,t}, the planes k_br_bits stored over the
+// segment's first buckets (U, then Q_t), then the affine normalisation;
 // cstep = c for plain windows, 0 for window-shifted segments (a plain sum).
 // The reference does its window combine on the host
 // (Sources/zkMetal/MSM/MSMEngine.swift:899-904); on the device it lets a
@@ -489,7 +490,7 @@ __global__ __launch_bounds__(16 * T::kLanes) void k_tail_windows(const SegDesc* 
     write_back(back);
     const uint32_t s = blockIdx.x, t = threadIdx.x / T::kLanes;
     const uint32_t c = msms[segs[s].msm].c;
-    const uint64_t b0 = (uint64_t)s * 16;
+    const uint64_t b0 = segs[s].bkt0;
     // plane t (c - 1 <= 15 of them) or U; the identity in between
     const bool plane = t + 1 < c, has = plane || t == 15;
     typename T::Pt v = T::load(bits, has ? b0 + (plane ? 1 + t : 0) : b0);
