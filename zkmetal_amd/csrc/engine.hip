@@ -146,13 +146,6 @@ bool shifted_pays(uint64_t n, uint32_t c, uint32_t c_s) {
     return shifted < plain;
 }
 
-// A single MSM's shifted buckets are deep enough to span several accumulation
-// lanes, which costs merge work where the reduction it saves no longer counts.
-// Measured on MI355X, one MSM shifted against plain: 2^16 points 290 / 425 us
-// (witness-like scalars 277 / 393), 2^18 586 / 594 (410 / 444), 2^19 883 / 894
-// (576 / 525), 2^20 1594 / 1671 (912 / 808).
-constexpr uint64_t kShiftSingleMax = 1u << 18;
-
 // Row and column sums by lanes from this many additions on (two per bucket),
 // by lane teams below: 2^16 of them make a wave of one-lane chains for every
 // SIMD, but a lane's chain is 7 us per addition against a team's 2.6.  Whole
@@ -1593,8 +1586,8 @@ int32_t Engine::set_schedule_table(const uint32_t* parts, const uint32_t* per, u
     for (uint32_t i = 0; i <= 32; i++) {
         const uint32_t p = (parts && i < len) ? parts[i] : 0;
         const uint32_t g = (per && i < len) ? per[i] : 0;
-        // per: a power of two from 4 (a column of up to 256 buckets then has
-        // at most 64 lanes, one wave's shuffle tree) to 64
+        // per: a power of two (a row or column is split evenly) from 4 to 64
+        // (the longest chain the built-in rule takes)
         if (p > kMaxParts || (g != 0 && (g < 4 || g > 64 || (g & (g - 1)) != 0))) return kInvalidInput;
         t.parts[i] = (uint8_t)p;
         t.per[i] = (uint8_t)g;

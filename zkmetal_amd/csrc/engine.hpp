@@ -160,6 +160,12 @@ int make_plan(const uint32_t* ns, const uint64_t* table0, uint32_t nmsm,
               uint64_t shift_stride = 0, uint32_t shift_c = 0, uint32_t shift_floor = 0,
               const Schedule* sched = nullptr);
 uint32_t default_parts(uint64_t entries, CurveId cv = CurveId::Bn254);
+// A single MSM's shifted buckets are deep enough to span several accumulation
+// lanes, which costs merge work where the reduction it saves no longer counts.
+// Measured on MI355X, one MSM shifted against plain: 2^16 points 292 / 336 us
+// (witness-like scalars 261 / 327), 2^18 552 / 561 (391 / 417), 2^19 942 / 830,
+// 2^20 1494 / 1447 (783 / 684).
+constexpr uint64_t kShiftSingleMax = 1u << 18;
 bool shifted_pays(uint64_t n, uint32_t c, uint32_t c_s);
 
 class Engine {
@@ -217,11 +223,11 @@ class Engine {
     // window-shifted resident tables: with mode kShiftAuto (default) or
     // kShiftAll an SRS set afterwards also gets the copies 2^(kShiftC w) P_i
     // of every window w (memory: the table times ceil(128 / kShiftC)); MSMs
-    // on it share one bucket set across windows when shifted_pays (auto) or
-    // always (all).  kShiftOff: plain plans, and the next SRS is plain.
+    // on it share one bucket set across windows by size and number of MSMs
+    // (auto: shift_floor, shifted_pays) or always (all).  kShiftOff: plain plans, and the next SRS is plain.
     // Falls back to the plain table when the copies do not fit.  Results are
     // the same bytes in every mode.
-    static constexpr uint32_t kShiftC = 16;
+    static constexpr uint32_t kShiftC = 16, kShiftFloor = 512;  // (the floor: shift_floor)
     enum ShiftMode { kShiftOff = 0, kShiftAuto = 1, kShiftAll = 2 };
     int32_t set_window_shift(int32_t mode) {
         if (mode < kShiftOff || mode > kShiftAll) return kInvalidInput;
@@ -421,14 +427,14 @@ class Engine {
     // make_plan's shift_floor for a call: in calls of up to kShiftAlwaysMsms
     // MSMs every MSM of at least kShiftFloor points (a single one up to
     // kShiftSingleMax): below that a plain reduction of narrow windows is as
-    // quick (one MSM of 256 / 512 / 2048 points 187 / 184 / 175 us shifted,
-    // 172 / 195 / 246 plain; 64 of 512 752 / 916), and beyond so many MSMs
+    // quick (one MSM of 256 / 512 / 2048 points 174 / 164 / 158 us shifted,
+    // 159 / 179 / 199 plain; 64 of 512 737 / 742), and beyond so many MSMs
     // their 2^15 buckets each no longer fill idle lanes but cost time, and the
     // estimate (shifted_pays) decides.  Otherwise: every MSM in kShiftAll
     // mode; in a call whose window combine runs on the device, every MSM of
     // at least kShiftDeviceTailFloor points (a plain MSM's serial doubling
     // chain would set the combine's latency)
-    static constexpr uint32_t kShiftDeviceTailFloor = 4096, kShiftFloor = 512, kShiftAlwaysMsms = 64;
+    static constexpr uint32_t kShiftDeviceTailFloor = 4096, kShiftAlwaysMsms = 64;
     uint32_t shift_floor(const std::vector<uint32_t>& ns, bool lean) const;
     // host image of the resident bases (64 B each) for the prefix check:
     // srs_first_ is filled whenever an SRS is set, srs_host_ on the first

@@ -11,30 +11,40 @@
 
 namespace zk {
 
-// Device bytes a request may occupy while it runs, alone or in a batch, at the
-// built-in window widths: the larger of its plans (plain at either width,
-// window-shifted into one set of 2^(kShiftC - 1) buckets).  Per entry: a digit
-// word, two sorted key/value copies, the tile histograms; per accumulation
-// lane two merge records and their share of the merge's lists.  A lane takes
-// at least four entries, and each part of a call at most a resident round of
-// lanes (a request of more than half a part's entries may share its call with
-// as much again).
-uint64_t Server::footprint(uint32_t n) {
+// What a request adds to its call, at the built-in window widths: its sorted
+// entries, and the bytes of its own beside the merge records.  The larger of
+// the plans that its table allows: plain at the batch's width, or at the width
+// of an MSM alone where that runs plain; window-shifted into one set of
+// 2^(kShiftC - 1) buckets.  Per entry: a digit word, two sorted key/value
+// copies, the tile histograms.
+Server::Load Server::load(uint32_t n, bool shifted) {
     uint32_t cls = 0;
     while ((1ull << cls) < n) cls++;
     const uint64_t tiles = (2ull * n + kSortTile - 1) / kSortTile;  // of one window
     uint64_t entries = 0, buckets = 0;
-    auto plan = [&](uint64_t c, bool shifted) {
+    auto plan = [&](uint64_t c, bool sh) {
         const uint64_t w = (128 + c - 1) / c;
-        entries = std::max<uint64_t>(entries, shifted ? w * tiles * kSortTile : w * 2 * n);
-        buckets = std::max<uint64_t>(buckets, (shifted ? 1 : w) << (c - 1));
+        entries = std::max<uint64_t>(entries, sh ? w * tiles * kSortTile : w * 2 * n);
+        buckets = std::max<uint64_t>(buckets, (sh ? 1 : w) << (c - 1));
     };
-    for (uint32_t c : {kTunedPlain[cls], kTunedBatch[cls]}) plan(c ? c : default_window_bits(n), false);
-    plan(Engine::kShiftC, true);
-    constexpr uint64_t kRound = 3 * kTwoWaveLanes / 2;  // three waves per SIMD
-    const uint64_t lanes = std::min(entries / 4, default_parts(2 * entries) * kRound) + kMaxWindows;
-    return (uint64_t)n * 32 + entries * 15 + buckets * kBucketBytes + lanes * 2 * (kBucketBytes + 6) + (1u << 20);
+    auto plain = [&](uint32_t c) { plan(c ? c : default_window_bits(n), false); };
+    plain(kTunedBatch[cls] ? kTunedBatch[cls] : kTunedPlain[cls]);
+    if (!shifted || n < Engine::kShiftFloor || n > kShiftSingleMax) plain(kTunedPlain[cls]);
+    if (shifted) plan(Engine::kShiftC, true);
+    return Load{entries, (uint64_t)n * 32 + entries * 15 + buckets * kBucketBytes + (1u << 20)};
 }
+
+// Bytes of a call of these requests: their own, and two merge records with
+// their share of the merge's lists per accumulation lane.  A lane takes at
+// least four entries (but a segment's last), and each part of a call at most a
+// resident round of lanes.
+uint64_t Server::charge(const Load& sum) {
+    constexpr uint64_t kRound = 3 * kTwoWaveLanes / 2;  // three waves per SIMD
+    const uint64_t lanes = std::min(sum.entries / 4, default_parts(sum.entries) * kRound);
+    return sum.bytes + lanes * 2 * (kBucketBytes + 6);
+}
+
+uint64_t Server::footprint(uint32_t n) { return std::max(charge(load(n, false)), charge(load(n, true))); }
 
 int32_t Server::create(Engine* owner, const ServerConfig& cfg, Server** out) {
     if (!out || !owner || cfg.slots == 0 || cfg.max_batch == 0) return kInvalidInput;
@@ -94,7 +104,7 @@ int32_t Server::submit(const uint8_t* scalars, uint32_t n, uint64_t* ticket, boo
         r->scalars = scalars;
     }
     r->n = n;
-    r->bytes = footprint(n);
+    r->load = load(n, table_shift_ != 0);
     r->t_submit = std::chrono::steady_clock::now();
     {
         std::lock_guard<std::mutex> lk(mu_);
@@ -123,7 +133,8 @@ void Server::worker(size_t slot) {
     std::vector<const uint8_t*> parts;
     for (;;) {
         std::vector<Request*> batch;
-        uint64_t bytes = 0;
+        Load sum{0, 0};
+        uint64_t bytes = 0;  // charge(sum)
         {
             std::unique_lock<std::mutex> lk(mu_);
             for (;;) {
@@ -132,10 +143,12 @@ void Server::worker(size_t slot) {
                 while (!queue_.empty() && batch.size() < cfg_.max_batch) {
                     Request* r = queue_.front();
                     const bool alone_ok = batch.empty() && in_use_ == 0;
-                    if (in_use_ + bytes + r->bytes > cfg_.hbm_budget && !alone_ok) break;
+                    const Load with{sum.entries + r->load.entries, sum.bytes + r->load.bytes};
+                    if (in_use_ + charge(with) > cfg_.hbm_budget && !alone_ok) break;
                     queue_.pop_front();
                     batch.push_back(r);
-                    bytes += r->bytes;
+                    sum = with;
+                    bytes = charge(sum);
                 }
                 if (!batch.empty()) break;
                 cv_work_.wait(lk);

@@ -3,7 +3,7 @@
 //
 // Each slot is an Engine with its own HIP stream and workspace.  A slot's
 // worker takes the queued requests in arrival order (up to max_batch) whose
-// estimated device footprint fits the free part of the HBM budget, runs them
+// device memory, as one call, fits the free part of the HBM budget, runs them
 // as one batched launch sequence, and returns the budget when they finish.
 // Requests arriving while slots are busy join the next batch; batches on
 // different slots overlap on the device.  A request larger than the whole
@@ -54,7 +54,13 @@ class Server {
     int32_t wait(uint64_t ticket, uint8_t* out96, double* latency_ms);
     int32_t poll(uint64_t ticket, uint8_t* out96, int32_t* done);
     void stats(ServerStats* s);
+    // what a request is charged alone, at most
     static uint64_t footprint(uint32_t n);
+    struct Load {
+        uint64_t entries, bytes;
+    };
+    static Load load(uint32_t n, bool shifted);
+    static uint64_t charge(const Load& sum);
 
   private:
     struct Request {
@@ -62,7 +68,7 @@ class Server {
         std::vector<uint8_t> owned;
         const uint8_t* scalars;
         uint32_t n;
-        uint64_t bytes;
+        Load load;
         std::chrono::steady_clock::time_point t_submit, t_done;
         uint8_t out[96];
         int32_t status = 0;
