@@ -190,14 +190,15 @@ ZkMetalStatus zkmsm_set_window_bits(ZkMetalMSMEngine engine, uint32_t c);
 uint32_t zkmsm_default_window_bits(uint64_t n);
 
 /* Timing of the engine's last call.  out[0..5]: device ms of the stages
- * decompose, sort, accumulate, merge, bucket-reduce, copy-out; out[6]:
+ * decompose, sort, accumulate, merge, bucket-reduce, copy-out (0 where the
+ * last kernel leaves the results in host memory: every call but the
+ * allocation-free ones); out[6]:
  * device total; out[7]: host tail ms; out[8]: wall ms of the call;
  * out[9]: window bits of the first MSM; out[10]: entries per accumulation
  * lane; out[11]: buckets per reduction group; out[12]: sorted entries;
  * out[13]: accumulation lanes; out[14]: entries with a nonzero digit (the
- * mixed additions performed); out[15]: device time of the window combine and
- * normalisation when the device ran them (0 when the host did, see
- * zkmsm_set_tail_mode); out[16]: pipeline parts of the call.  Returns the
+ * mixed additions performed); out[15]: device time of the window combine when
+ * the device ran it (0 when the host did, see zkmsm_set_tail_mode); out[16]: pipeline parts of the call.  Returns the
  * number of values written (at most 17). */
 int32_t zkmsm_last_timing(ZkMetalMSMEngine engine, double* out, int32_t max_values);
 
@@ -206,8 +207,9 @@ int32_t zkmsm_last_timing(ZkMetalMSMEngine engine, double* out, int32_t max_valu
  * starts from the tables measured on MI355X (zkmetal_amd/csrc/tuned_gfx950.hpp);
  * these calls replace them.  The plain
  * table applies to calls with one MSM, the batch table to each MSM of a call
- * with several (falling back to the plain table where it holds 0).  Tables
- * come from the autotuning sweep in zkmetal_amd/tune.py; a request server
+ * with several (falling back to the plain table where it holds 0); both are
+ * BN254 G1's (Grumpkin and G2 calls have their own, which nothing replaces).
+ * zkmetal_amd/tune.py sweeps them for a device; a request server
  * copies both tables from the engine it is created on. */
 ZkMetalStatus zkmsm_set_window_table(ZkMetalMSMEngine engine, const uint32_t* c_by_log2n,
                                      uint32_t len);
@@ -220,14 +222,13 @@ ZkMetalStatus zkmsm_set_batch_window_table(ZkMetalMSMEngine engine, const uint32
  *   parts_by_log2e[k]: pipeline parts the call's segments are split into
  *     (the sort of part p + 1 runs on a second stream beside the bucket
  *     accumulation of part p), 1..8;
- *   reduce_per_by_log2e[k]: buckets each bucket-reduction lane sums before
- *     the lanes of a row or column meet in a shuffle tree, a power of two
- *     in 4..64.
+ *   reduce_per_by_log2e[k]: buckets each bucket-reduction team or lane sums
+ *     before those of a row or column meet in a tree, a power of two in 4..64.
  * 0 keeps the built-in rule for that class; either array may be NULL (all
  * 0).  batch != 0 sets the table for calls of several MSMs, 0 for calls of
  * one.  An engine starts from the tables measured on MI355X
- * (zkmetal_amd/csrc/tuned_gfx950.hpp); they come from the autotuning sweep in
- * zkmetal_amd/tune.py, and a request server copies them from the engine it
+ * (zkmetal_amd/csrc/tuned_gfx950.hpp); zkmetal_amd/tune.py sweeps them for a
+ * device, and a request server copies them from the engine it
  * is created on.  zkmsm_set_pipeline_parts, when nonzero, overrides the
  * parts.  Results do not depend on the schedule.  An out-of-range value
  * returns ZKMETAL_ERR_INVALID_INPUT and leaves the table unchanged.  (No
@@ -252,8 +253,8 @@ ZkMetalStatus zkmsm_set_graph_mode(ZkMetalMSMEngine engine, int32_t mode);
 
 /* A large call runs as a pipeline over parts of its bucket segments: the
  * bucket sort of part p + 1 on a second stream while part p accumulates,
- * then one bucket reduction over all parts.  parts = 0 (default) picks 1, 2
- * or 3 parts by size; 1..8 forces that many (at most one per segment).
+ * then one bucket reduction over all parts.  parts = 0 (default) picks 1 or 2
+ * parts by size; 1..8 forces that many (at most one per segment).
  * Results are the same bytes for any value. */
 ZkMetalStatus zkmsm_set_pipeline_parts(ZkMetalMSMEngine engine, uint32_t parts);
 
@@ -265,13 +266,14 @@ ZkMetalStatus zkmsm_set_pipeline_parts(ZkMetalMSMEngine engine, uint32_t parts);
  * resident table can then accumulate all its windows into one set of 2^15
  * buckets: the bucket reduction shrinks eightfold and the window combine
  * needs no doublings, at the price of gathers spread over the larger table.
- * Auto takes it, in calls of several MSMs, for those whose cost estimate
- * favours it (the reduction saved against the padding added), for a single
- * MSM of at most 2^17 points, and for MSMs of >= 4096 points in calls whose
- * window combine runs on the device; all takes it for every MSM (measured
- * on MI355X: the 64-MSM batch 20.8 -> 18.0 ms, 32 witness-like MSMs of 2^18
- * points 13.1 -> 8.0 ms, one 2^16 MSM 0.61 -> 0.42 ms, one 2^22 MSM 6.05 ->
- * 6.23 ms, which auto runs plain).  mode 0 (off):
+ * Auto takes it in calls of up to 64 MSMs for those of at least 512 points (a
+ * single one up to 2^18), in larger calls for those whose cost estimate favours
+ * it (the reduction saved against the padding added) and, where the window
+ * combine runs on the device, for those of at least 4096 points; all takes it
+ * for every MSM (measured on MI355X, plain -> shifted: 48 MSMs of 2^12 to 2^20
+ * points 13.1 -> 11.6 ms, 32 witness-like MSMs of 2^18 points 5.8 -> 3.9 ms, one
+ * 2^16 MSM 0.34 -> 0.29 ms, one 2^22 MSM 5.58 -> 5.76 ms, which auto runs
+ * plain).  mode 0 (off):
  * plain plans, and the next SRS is plain.  When the copies do not fit
  * (device memory, zkmsm_set_workspace_limit) the plain table is kept.
  * Results are the same bytes in every mode.  No counterpart in the
@@ -281,13 +283,15 @@ ZkMetalStatus zkmsm_set_window_shift(ZkMetalMSMEngine engine, int32_t mode);
 /* 16 when the resident table holds window-shifted copies, else 0 */
 uint32_t zkmsm_srs_window_shift(ZkMetalMSMEngine engine);
 
-/* Where a call's window combine (Horner over the windows) and affine
- * normalisation run: 0 auto (the device in graph mode and for calls of 16 or
- * more MSMs, the host otherwise), 1 the host, 2 the device.  Results are the
- * same bytes either way.  BN254 G2 calls always use the host.  The device
- * form lets a graph replay end with final results; the host is faster for a
- * single MSM (the combine is a serial chain of ~127 doublings, which one
- * host core runs faster than one GPU lane). */
+/* Where a call's window combine (Horner over the windows) runs: 0 auto (the
+ * device in graph mode, for calls of 16 or more MSMs and for calls of 8 or more
+ * that are not window-shifted, the host otherwise), 1 the host, 2 the device.
+ * The affine normalisation of up to 1024 sums is the host's either way, that
+ * of more the device's with its combine.  Results are the same bytes either
+ * way.  BN254 G2 calls always use the host (the device sums each window's bit
+ * planes).  The device form lets a graph replay end with one sum per MSM; the
+ * host is faster for a single MSM (the combine is a serial chain of ~127
+ * doublings, which one host core runs faster than the device). */
 ZkMetalStatus zkmsm_set_tail_mode(ZkMetalMSMEngine engine, int32_t mode);
 
 /* Cap on the device memory an engine's buffers may grow to (its resident SRS
@@ -307,7 +311,7 @@ uint64_t zkmsm_graph_captures(ZkMetalMSMEngine engine);
  * server sees it), and zkmetal_msm_engine_destroy on it defers the release
  * until the last server is destroyed.  `slots` engines, each
  * with its own stream and workspace, take queued requests in arrival order
- * (at most max_batch per launch) while their estimated device footprint fits
+ * (at most max_batch per launch) while the device memory of their call fits
  * the free HBM budget; batches on different slots overlap on the device.
  * Submission copies the scalars; all calls are thread-safe. */
 typedef void* ZkmsmServer;
@@ -340,7 +344,8 @@ ZkMetalStatus zkmsm_server_poll(ZkmsmServer server, uint64_t ticket, uint8_t* re
                                 int32_t* done);
 ZkMetalStatus zkmsm_server_stats(ZkmsmServer server, ZkmsmServerStats* out);
 void zkmsm_server_destroy(ZkmsmServer server);
-/* bytes of the HBM budget a request of n points is charged */
+/* bytes of the HBM budget a request of n points is charged alone, at most
+ * (those of one launch share its merge records) */
 uint64_t zkmsm_server_footprint(uint32_t n);
 
 /* ---- seeded synthetic scalars (host) ------------------------------------ */

@@ -562,8 +562,9 @@ class MetalMSM:
     TAIL_AUTO, TAIL_HOST, TAIL_DEVICE = 0, 1, 2
 
     def set_tail_mode(self, mode):
-        """Where the window combine and normalisation run: TAIL_AUTO (device in
-        graph mode and for calls of >= 16 MSMs), TAIL_HOST or TAIL_DEVICE."""
+        """Where the window combine runs: TAIL_AUTO (device in graph mode, for
+        calls of >= 16 MSMs and of >= 8 that are not window-shifted), TAIL_HOST
+        or TAIL_DEVICE."""
         _check(lib().zkmsm_set_tail_mode(self.handle, mode), "set_tail_mode")
 
     SHIFT_OFF, SHIFT_AUTO, SHIFT_ALL = 0, 1, 2
@@ -571,8 +572,8 @@ class MetalMSM:
     def set_window_shift(self, mode):
         """Window-shifted resident tables: SHIFT_AUTO (default) or SHIFT_ALL
         make an SRS set afterwards also hold 2^(16 w) P_i for every window w,
-        and MSMs on it share one bucket set across windows (auto: when the
-        cost estimate favours it; all: always); SHIFT_OFF runs plain and
+        and MSMs on it share one bucket set across windows (auto: by size
+        and number of MSMs, where it is quicker; all: always); SHIFT_OFF runs plain and
         makes the next SRS plain.  True / False mean auto / off.  Results do
         not change."""
         _check(lib().zkmsm_set_window_shift(self.handle, int(mode)), "set_window_shift")

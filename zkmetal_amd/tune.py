@@ -13,8 +13,8 @@ engine's own size measure for a call; one table for calls of one MSM, one
 for calls of several): the pipeline parts (how the call's (MSM, window)
 segments are split so that the sort of one part runs on a second stream
 beside the accumulation of the previous one) and the bucket reduction's
-buckets per lane (the tile of buckets a lane sums before the lanes of a row
-or column meet in a shuffle tree).  Each is swept on single MSMs of every
+buckets per lane or team (the tile of buckets each sums before those of a row
+or column meet in a tree).  Each is swept on single MSMs of every
 size and on batches of log-uniform sizes from 2^19 to 2^24 points, parts
 first (at the built-in reduction tile), then the tile.
 
